@@ -60,7 +60,29 @@ struct SoundArgs {
   // copies them into u3d, v3d, w3d on the halo ring only; skip_winds marks it
   int skip_winds;
   const float* u_in; const float* v_in; const float* w_in;
+  // resident pass: which words this small step adds into the time averages
+  // (AVG_*), and whether the pressure gradient takes ppd's halo words from the
+  // cells the fill would copy (from the second small step on)
+  int avg_on, avg;
+  int map_ppd;
 };
+
+// The time averages are sums over the small steps in step order.  Both winds of
+// a pair of steps are at hand in the second one (the pass that steps a word
+// reads the step before's), so a resident stage adds two steps' words at every
+// second small step and touches rru, rrv, rrw half as often; an odd last step
+// adds its own.  (The values are the number of steps added: a sum starts from
+// +0, or from beta*wa, when that many steps are all there have been.)
+enum { AVG_NONE = 0, AVG_SINGLE = 1, AVG_PAIR = 2 };
+
+// the pressure-family index (1-based cells, halos 0 and n+1) whose word the
+// family fill copies to index i: the far cell on a periodic side, the edge cell
+// otherwise
+GM1_DEV int filled_index(int i, int n, bool periodic_lo, bool periodic_hi) {
+  if (i < 1) return periodic_lo ? n : 1;
+  if (i > n) return periodic_hi ? 1 : n;
+  return i;
+}
 
 GM1_DEV const float* P_sigma(const SoundArgs& a) { return a.prof; }
 GM1_DEV const float* P_sigmaf(const SoundArgs& a) { return a.prof + (a.nk + 2); }
@@ -494,9 +516,9 @@ __global__ __launch_bounds__(256) void k_snd_ssopen_flat(SoundArgs a) {
 // boundary face and on the row outside the grid (param.F:9182-9219).
 // Each thread steps its face pair at PG_KB consecutive levels, every level's
 // words requested before any level is formed.
-constexpr int PG_KB = 2;  // (measured at 640x768x80: 242 us against 253 at four levels, 240 at one)
+constexpr int PG_KB = 2;  // (without averages, at 640x768x80: 242 us against 253 at four levels, 240 at one)
 
-__global__ __launch_bounds__(PG_TX * PG_TY) void k_snd_pgrad_flat(SoundArgs a) {
+__global__ __launch_bounds__(PG_TX * PG_TY) void k_snd_pgrad_flat(SoundArgs a, int n) {
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const int gx = (ni + 1 + PG_TX - 1) / PG_TX, gy = (nj + 1 + PG_TY - 1) / PG_TY;
   const int nkb = (nk + PG_KB - 1) / PG_KB;
@@ -514,6 +536,17 @@ __global__ __launch_bounds__(PG_TX * PG_TY) void k_snd_pgrad_flat(SoundArgs a) {
   const float wv = (i <= ni && (j > 1 || ps) && (j < nj + 1 || pn)) ? 1.0f : 0.0f;
   // a level's words at 32-bit byte offsets from the level's base
   const uint32_t op = (uint32_t)((j * (ni + 2) + i) * 4), onp = (uint32_t)(ni + 2) * 4u;
+  // ppd's own, west and south words: where the fill would have copied them from
+  // (each side's copy is of an interior word, so no pass has to fill the ring
+  // between small steps)
+  uint32_t opc = op, opw = op - 4u, ops = op - onp;
+  if (a.map_ppd) {
+    const int ic = filled_index(i, ni, pw, pe), iw = filled_index(i - 1, ni, pw, pe);
+    const int jc = filled_index(j, nj, ps, pn), js = filled_index(j - 1, nj, ps, pn);
+    opc = (uint32_t)((jc * (ni + 2) + ic) * 4);
+    opw = (uint32_t)((jc * (ni + 2) + iw) * 4);
+    ops = (uint32_t)((js * (ni + 2) + ic) * 4);
+  }
   const uint32_t ou = (uint32_t)(((y + NG) * ux(ni) + x + NG) * 4), ov = (uint32_t)(((y + NG) * sx(ni) + x + NG) * 4);
   const int64_t pst = (int64_t)(nj + 2) * (ni + 2), ust = (int64_t)sy(nj) * ux(ni), vst = (int64_t)vy(nj) * sx(ni);
   // the words before this small step: u_in / v_in when set, except on the open
@@ -533,13 +566,27 @@ __global__ __launch_bounds__(PG_TX * PG_TY) void k_snd_pgrad_flat(SoundArgs a) {
       ut[q] = ldo(a.uten + (int64_t)k * ust, ou);
       v[q] = ldo(vsrc + (int64_t)k * vst, ov);
       vt[q] = ldo(a.vten + (int64_t)k * vst, ov);
-      dc[q] = ldo(P, op);
-      dw[q] = ldo(P, op - 4u);
-      ds[q] = ldo(P, op - onp);
+      dc[q] = ldo(P, opc);
+      dw[q] = ldo(P, opw);
+      ds[q] = ldo(P, ops);
       tc[q] = ldo(T, op);
       tw[q] = ldo(T, op - 4u);
       ts[q] = ldo(T, op - onp);
     }
+  }
+  // the time averages of this face pair (resident stage).  An open boundary
+  // face has been stepped since the last small step, so its word of that step is
+  // gone: it adds every step's own word.
+  const bool last = n == a.nloop;
+  const int au = (ow_face && y < nj) ? (a.avg_on ? AVG_SINGLE : AVG_NONE) : a.avg;
+  const int av = (os_face && x < ni) ? (a.avg_on ? AVG_SINGLE : AVG_NONE) : a.avg;
+  const float tavg = 1.0f / (float)a.nloop;
+  float ru[PG_KB], rv[PG_KB];
+#pragma unroll
+  for (int q = 0; q < PG_KB; ++q) {
+    const int k = kb + q;
+    ru[q] = (au && n > au && k <= nk) ? ldo(a.rru + (int64_t)k * ust, ou) : 0.0f;
+    rv[q] = (av && n > av && k <= nk) ? ldo(a.rrv + (int64_t)k * vst, ov) : 0.0f;
   }
 #pragma unroll
   for (int q = 0; q < PG_KB; ++q) {
@@ -547,10 +594,20 @@ __global__ __launch_bounds__(PG_TX * PG_TY) void k_snd_pgrad_flat(SoundArgs a) {
     if (k <= nk) {
       float pu = tem1 * (dc[q] - dw[q]);
       pu = pu * (tc[q] + tw[q]);
-      sto(a.u3d + (int64_t)k * ust, ou, u[q] + (a.dts * wu) * (ut[q] - pu));
+      const float un = u[q] + (a.dts * wu) * (ut[q] - pu);
+      sto(a.u3d + (int64_t)k * ust, ou, un);
       float pv = tem2 * (dc[q] - ds[q]);
       pv = pv * (tc[q] + ts[q]);
-      sto(a.v3d + (int64_t)k * vst, ov, v[q] + (a.dts * wv) * (vt[q] - pv));
+      const float vn = v[q] + (a.dts * wv) * (vt[q] - pv);
+      sto(a.v3d + (int64_t)k * vst, ov, vn);
+      if (au) {
+        const float t = (au == AVG_PAIR ? ru[q] + u[q] : ru[q]) + un;
+        sto(a.rru + (int64_t)k * ust, ou, last ? t * tavg : t);
+      }
+      if (av) {
+        const float t = (av == AVG_PAIR ? rv[q] + v[q] : rv[q]) + vn;
+        sto(a.rrv + (int64_t)k * vst, ov, last ? t * tavg : t);
+      }
     }
   }
 }
@@ -762,10 +819,8 @@ int column2_lds_bytes(int nk, int cw, bool pipe = false, bool flat_pipe = false)
 // rru(k) += u(k) and rrv(k) += v(k) on one column's west u face and south v
 // face for levels kb..ke (divided by nloop on the last small step); the words
 // of four levels are requested before any is written.
-// (fresh: the averages start here, from 0 rather than the words in rru, rrv)
 GM1_DEV void average_uv_faces(const SoundArgs& a, const float* __restrict__ u3, const float* __restrict__ v3, int kb,
-                              int ke, int64_t ust, int64_t uc, int64_t vst, int64_t vc, bool last, float tavg,
-                              bool fresh = false) {
+                              int ke, int64_t ust, int64_t uc, int64_t vst, int64_t vc, bool last, float tavg) {
   float* __restrict__ rru = a.rru;
   float* __restrict__ rrv = a.rrv;
   constexpr int B = 4;
@@ -775,9 +830,9 @@ GM1_DEV void average_uv_faces(const SoundArgs& a, const float* __restrict__ u3, 
     for (int u = 0; u < B; ++u)
       if (k0 + u <= ke) {
         const int64_t pu = (int64_t)(k0 + u) * ust + uc, pv = (int64_t)(k0 + u) * vst + vc;
-        ru[u] = fresh ? 0.0f : rru[pu];
+        ru[u] = rru[pu];
         uu[u] = u3[pu];
-        rv[u] = fresh ? 0.0f : rrv[pv];
+        rv[u] = rrv[pv];
         vv[u] = v3[pv];
       }
 #pragma unroll
@@ -1485,6 +1540,13 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(4))) void k
 // recurrence reads (s1, s2, mm -> ec, dd -> ed -> w), the level factors and
 // the slots' last-level words: about 48 KiB at 32 columns x 81 levels, three
 // workgroups a CU where the seven-plane pass fits two.
+// Bound by HBM: 13 words a cell and step are algorithmic (u, v, w, wten, pp3d,
+// ppten, ppterm, piadv, thv read; w, pp3d, ppd written; rrw read and written at
+// every second step).  The u and v averages are the pressure gradient's (one
+// read and one write of rru, rrv per two steps, where this pass moved them every
+// step), and this pass makes the open sides' next step: at 640x768x80 this pass
+// 816 -> 645 us and the pressure gradient 244 -> 302 us a small step, with no
+// open-side and ring-fill launches between small steps (9 + 6 us).
 constexpr int C3PLANES = 4;
 
 int column3_lds_bytes(int nk, int cw, int slots) {
@@ -1505,7 +1567,7 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
   const bool inside = (i <= ni);
   const bool phys = (i < ni) && (j < nj);
   const bool last = (n == a.nloop);
-  const bool fresh = a.fresh_averages && n == 1;  // the first small step starts the time averages
+  const bool first = n == 1;
   const float tavg = 1.0f / (float)a.nloop;
   const int nxs = sx(ni), nys = sy(nj), nxu = ux(ni), nyv = vy(nj);
   const int64_t wst = (int64_t)nys * nxs;
@@ -1543,7 +1605,7 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
   const float asq = a.alph * a.alph;
   const float smeps = 1.0e-30f;
   const int pj = j + 1, pi = i + 1;
-  float rpp[CH], rfpk[CH];
+  float rpp[CH], rfpk[CH], rwo[CH];
   float wt0 = 0.0f, wo0 = 0.0f;  // level kb's wten and w, for its right-hand side after the barrier
 
   // ---------------- phase A (sound.F:491-509 and the right-hand sides)
@@ -1554,10 +1616,10 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
     const float* wi = a.w_in ? a.w_in : w;
     if (kb == 1) lw1[c] = wi[wst + wc];
     struct In {
-      float uw, ue, vs, vn, pc, pe, pw, pn, ps, wup, wt, ppten, ppterm, pp, th, ru, rv;
+      float uw, ue, vs, vn, pc, pe, pw, pn, ps, wup, wt, ppten, ppterm, pp, th;
     };
     const uint32_t onp = (uint32_t)(ni + 2) * 4u, onx = (uint32_t)nxs * 4u, ows = (uint32_t)wst * 4u;
-    const float* pp_in = (fresh && a.nrk != 1) ? a.ppi : a.pp3d;  // the first small step reads ppi
+    const float* pp_in = (first && a.nrk != 1) ? a.ppi : a.pp3d;  // the first small step reads ppi
     auto load = [&](int k) {
       const uint32_t op = (uint32_t)pix(k, pj, pi, ni, nj) * 4u;
       const uint32_t ou = (uint32_t)((int64_t)k * ust + uc) * 4u;
@@ -1579,8 +1641,6 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
       v.ppterm = ldo(a.ppterm, op);
       v.pp = ldo(pp_in, op);
       v.th = ldo(a.thv, op);
-      v.ru = fresh ? 0.0f : ldo(a.rru, ou);  // the own faces' time averages so far
-      v.rv = fresh ? 0.0f : ldo(a.rrv, ov);
       return v;
     };
     float wraw = wi[(int64_t)kb * wst + wc];
@@ -1606,11 +1666,7 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
         const float s1 = t.pk1 + t.qk, s2 = t.pk2 - t.qk;
         const float vert = wraw * s1 + cu.wup * s2;
         const float fpk = (a.dts * (cu.ppten - cu.ppterm * div) + hp) + a.beta * vert;
-        {  // the own u and v faces into their time averages, from the words read above
-          const float au = cu.ru + cu.uw, av = cu.rv + cu.vs;
-          a.rru[(int64_t)k * ust + uc] = last ? au * tavg : au;
-          a.rrv[(int64_t)k * vst + vc] = last ? av * tavg : av;
-        }
+        rwo[kk] = wraw;
         Ls1[at(k)] = s1;
         Ls2[at(k)] = s2;
         Lmm[at(k)] = t.mm;
@@ -1646,15 +1702,33 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
   }
   __syncthreads();
   // ---------------- phase B: Thomas recurrence, one lane per column, while
-  // the slots outside wavefront 0 add the u and v faces into their averages
+  // the slots outside wavefront 0 make the next small step's open-side step of
+  // the tile's boundary faces (k_snd_ssopen_flat's statements): the column
+  // beside a face is the only reader of it in this pass, and has read it
   if (phys && slot == 0) thomas_column<C2W>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
   {
     constexpr int S0 = 64 / C2W;
-    static_assert(C2S > S0, "the averages need slots outside wavefront 0");
-    if (inside && !phys && slot >= S0) {  // the east column's and north row's faces
-      const int ch2 = (nk + (C2S - S0) - 1) / (C2S - S0);
-      const int kb2 = 1 + (slot - S0) * ch2, ke2 = min(nk, kb2 + ch2 - 1);
-      average_uv_faces(a, a.u3d, a.v3d, kb2, ke2, ust, uc, vst, vc, last, tavg, fresh);
+    static_assert(C2S > S0, "the open sides need slots outside wavefront 0");
+    const bool ow = i == 0 && side_of(a.sides, 0) == 2u, oe = i == ni - 1 && side_of(a.sides, 1) == 2u;
+    const bool os = j == 0 && side_of(a.sides, 2) == 2u, on = j == nj - 1 && side_of(a.sides, 3) == 2u;
+    if (!last && phys && slot >= S0 && (ow || oe || os || on)) {
+      for (int k = 1 + slot - S0; k <= nk; k += C2S - S0) {
+        if (ow || oe) {
+          const int64_t pu = (int64_t)k * ust + uc, rx = (int64_t)k * (nj + 2 * NG) + j + NG;
+          const float uw = a.u3d[pu], ue = a.u3d[pu + 1], d = ue - uw;
+          if (ow) a.u3d[pu] = uw + a.dts * (((((-a.radbcw[rx]) * d) * a.rdx) * a.uh[NG]) + a.uten[pu]);
+          if (oe)
+            a.u3d[pu + 1] = ue + a.dts * (((((-a.radbce[rx]) * d) * a.rdx) * a.uh[ni + NG - 1]) + a.uten[pu + 1]);
+        }
+        if (os || on) {
+          const int64_t pv = (int64_t)k * vst + vc, ry = (int64_t)k * (ni + 2 * NG) + i + NG;
+          const float vs = a.v3d[pv], vn = a.v3d[pv + nxs], d = vn - vs;
+          if (os) a.v3d[pv] = vs + a.dts * (((((-a.radbcs[ry]) * d) * a.rdy) * a.vh[NG]) + a.vten[pv]);
+          if (on)
+            a.v3d[pv + nxs] =
+                vn + a.dts * (((((-a.radbcn[ry]) * d) * a.rdy) * a.vh[nj + NG - 1]) + a.vten[pv + nxs]);
+        }
+      }
     }
   }
   __syncthreads();
@@ -1664,8 +1738,8 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
     float rw[CH];
 #pragma unroll
     for (int kk = 0; kk < CH; ++kk)
-      if (kb + kk <= ke)
-        rw[kk] = fresh ? a.wa[(int64_t)(kb + kk) * wst + wc] * a.beta : a.rrw[(int64_t)(kb + kk) * wst + wc];
+      if (a.avg && kb + kk <= ke)
+        rw[kk] = n <= a.avg ? a.wa[(int64_t)(kb + kk) * wst + wc] * a.beta : a.rrw[(int64_t)(kb + kk) * wst + wc];
 #pragma unroll
     for (int kk = 0; kk < CH; ++kk) {
       const int k = kb + kk;
@@ -1682,8 +1756,10 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
         const float tend = a.kdiv * (up - old);
         a.ppd[p] = up + tend;
         if (a.nrk == 3 && last) a.ppx[p] = tend;
-        const float vw = rw[kk] + (last ? wk * a.alph : wk);
-        a.rrw[(int64_t)k * wst + wc] = last ? vw * tavg : vw;
+        if (a.avg) {
+          const float vw = (a.avg == AVG_PAIR ? rw[kk] + rwo[kk] : rw[kk]) + (last ? wk * a.alph : wk);
+          a.rrw[(int64_t)k * wst + wc] = last ? vw * tavg : vw;
+        }
       }
     }
   } else if (inside) {
@@ -1691,8 +1767,11 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
       const int64_t pw = (int64_t)k * wst + wc;
       const float wk = a.w_in ? a.w_in[pw] : w[pw];
       if (a.w_in) w[pw] = wk;  // the east column's and north row's w, copied on the first step
-      const float vw = (fresh ? a.wa[pw] * a.beta : a.rrw[pw]) + (last ? wk * a.alph : wk);
-      a.rrw[pw] = last ? vw * tavg : vw;
+      if (a.avg) {  // (this w is the same in every small step)
+        const float r0 = n <= a.avg ? a.wa[pw] * a.beta : a.rrw[pw];
+        const float vw = (a.avg == AVG_PAIR ? r0 + wk : r0) + (last ? wk * a.alph : wk);
+        a.rrw[pw] = last ? vw * tavg : vw;
+      }
     }
   }
 }
@@ -1881,6 +1960,7 @@ static int psolver3_stage(
                    span >= ((int64_t)1 << 32)))
     return (int)hipErrorInvalidValue;
   a.fresh_averages = resident ? 1 : 0;
+  a.avg_on = resident ? 1 : 0;
   // (the fills after small steps 1..nloop-1 rewrite ppd's whole halo ring when every side is a family)
   const bool all_sides = side_of(sides, 0) && side_of(sides, 1) && side_of(sides, 2) && side_of(sides, 3);
   a.skip_ppd = (resident && nloop >= 2 && all_sides) ? 1 : 0;
@@ -1928,7 +2008,12 @@ static int psolver3_stage(
     for (int n = 1; n <= nloop; ++n) {
       SoundArgs b = a;
       first_step(b, n);
-      if (any_open)
+      if (resident) {
+        b.avg = (n % 2 == 0) ? AVG_PAIR : (n == nloop) ? AVG_SINGLE : AVG_NONE;
+        b.map_ppd = (n > 1 && all_sides) ? 1 : 0;
+      }
+      // (the resident pass steps the open faces for the next small step itself)
+      if (any_open && (n == 1 || !resident))
         hipLaunchKernelGGL(k_snd_ssopen_flat, dim3(gm1_blocks((int64_t)nk * (ni + nj), 256)), dim3(256), 0, s, b);
       SoundArgs pg = b;
       if (a.skip_ppd && n == 1) pg.ppd = ppx;  // ppd = ppx until the first small step writes it
@@ -1937,14 +2022,15 @@ static int psolver3_stage(
                   hipLaunchKernelGGL(k_snd_pgrad_flat,
                                      dim3(((ni + 1 + PG_TX - 1) / PG_TX) * ((nj + 1 + PG_TY - 1) / PG_TY) *
                                           ((nk + PG_KB - 1) / PG_KB)),
-                                     dim3(PG_TX * PG_TY), 0, s, pg));
+                                     dim3(PG_TX * PG_TY), 0, s, pg, n));
         if (resident)
           GM1_TIMED(TK_ACOUSTIC_COLUMN, s, launch_column3(narrow, b, n, s));
         else
           GM1_TIMED(TK_ACOUSTIC_COLUMN, s, launch_column2<true>(narrow, pipe, a, n, s));
       });
       GM1_LAUNCH_CHECK();
-      if (n < nloop) {
+      // (mapped reads need the ring itself only as the stage leaves it)
+      if (n < nloop && (!(resident && all_sides) || n == nloop - 1)) {
         int rc = fill_pressure(ppd, sides, ni, nj, nk, s);
         if (rc) return rc;
       }

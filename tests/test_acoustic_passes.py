@@ -1,0 +1,54 @@
+"""The acoustic stage's column passes against its general one, word for word, where their rules branch."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+from helpers import assert_bits_equal, to_host
+
+OUT = ("u3d", "v3d", "w3d", "pp3d", "ppd", "ppx", "rru", "rrv", "rrw", "radbcw", "radbce", "radbcs", "radbcn")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nloop", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("sides,ni,nj,nk", [((2, 2, 2, 2), 33, 9, 18), ((1, 1, 2, 2), 32, 11, 16), ((2, 4, 1, 1), 31, 8, 33),
+                                            ((4, 2, 2, 4), 64, 9, 66), ((1, 1, 1, 1), 9, 33, 17)])
+def test_gpu_flat_resident_stage_equals_the_staged_one(device, monkeypatch, nloop, sides, ni, nj, nk):
+    """Odd and even counts of small steps (time averages are added two steps at a time), mixed lateral families
+    (ppd's halo words are taken from the cells the fill copies), tiles with and without a ragged edge."""
+    from dataclasses import replace
+
+    import torch
+
+    from gm1_amd import stretched
+    from gm1_amd.fields import large_stretched_c3
+    from gm1_amd.large_step import create_gm1_large_step_state, host_initial_state, launch_cuda_gm1_large_step
+
+    cfg = replace(large_stretched_c3(ni, nj, nk), lateral_sides=sides,
+                  stretched=(nk * 100.0, 0.0, nk * 100.0, 60.0, 140.0))
+    print(f"resident stage {ni}x{nj}x{nk} sides {sides} nloop {nloop}", flush=True)
+    st = create_gm1_large_step_state(host_initial_state(cfg), device)
+    launch_cuda_gm1_large_step(st)
+    torch.cuda.synchronize()
+    g = torch.Generator(device=device).manual_seed(nloop)
+    for n in ("ppi", "ppx", "uten", "vten", "wten", "ua", "va", "wa", "u3d", "v3d", "w3d"):
+        scale = 1e-4 if n in ("ppi", "ppx") else 1e-3 if n.endswith("ten") else 1.0
+        st.a[n] += scale * torch.randn(st.a[n].shape, device=device, generator=g)
+    schedule = stretched.sound3_stage_schedule_f32
+    monkeypatch.setattr(stretched, "sound3_stage_schedule_f32", lambda dt, ns, nrk: (nloop, schedule(dt, ns, nrk)[1]))
+    runs = {}
+    for column_pass in ("staged", "resident", "resident16"):
+        a = {k: v.clone() for k, v in st.a.items()}
+        out = []
+        for nrk in (1, 3):
+            stretched.launch_cuda_gm1_flat_acoustic_stage(a, st.metrics, ni=ni, nj=nj, nk=nk, nrk=nrk, dt=cfg.dt,
+                                                          nsound=cfg.nsound, dx=cfg.dx, dy=cfg.dy, vertical=st.flat,
+                                                          lateral_sides=sides, column_pass=column_pass)
+            torch.cuda.synchronize()
+            out.append({n: to_host(a[n]) for n in OUT})
+        runs[column_pass] = out
+    for column_pass in ("resident", "resident16"):
+        for got, want, nrk in zip(runs[column_pass], runs["staged"], (1, 3)):
+            for n in OUT:
+                assert_bits_equal(got[n], want[n], f"{column_pass} stage {nrk} {n}")
+    assert np.isfinite(runs["staged"][1]["w3d"]).all() and np.abs(runs["staged"][1]["w3d"]).max() > 0.0
