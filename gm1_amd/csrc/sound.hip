@@ -337,9 +337,10 @@ __global__ __launch_bounds__(SS_T) void k_snd_ssopen2(SoundArgs a) {
   else if (side == 1) { j0 = idx; cb = (int64_t)(idx + NG) * nx + NG + ni; cc = cb - 1; }
   else if (side == 2) { i0 = idx; cb = (int64_t)NG * nx + idx + NG; cc = cb + nx; }
   else { i0 = idx; cb = (int64_t)(NG + nj) * nx + idx + NG; cc = cb - nx; }
+  const float* qi = xdir ? (a.u_in ? a.u_in : a.u3d) : (a.v_in ? a.v_in : a.v3d);  // before this small step
   for (int k = 1 + (int)threadIdx.x; k <= nk; k += SS_T) {
-    sb[k] = q[(int64_t)k * st + cb];
-    sc[k] = q[(int64_t)k * st + cc];
+    sb[k] = qi[(int64_t)k * st + cb];
+    sc[k] = qi[(int64_t)k * st + cc];
   }
   __syncthreads();
   const float* cgs = P_cgs(a);
@@ -393,71 +394,158 @@ __global__ __launch_bounds__(SS_T) void k_snd_ssopen2(SoundArgs a) {
 // ------------------------------------------------------------------ pgrad
 constexpr int PG_TX = 64, PG_TY = 4;
 
+// The u/v forward step over sloping terrain, on every face the family advances.
+// Each thread steps its face pair at KB consecutive levels, every level's words
+// requested before any is formed and the vertical ppd differences shared between
+// them (ppd is read at KB+2 levels).  HBM-bound: 8 words a cell (10 with the
+// slopes), plus one for rru and rrv each, at every second step two.
+//
 // SLOPES0: the caller states gxu = gyv = +0 everywhere, so the terrain term tr = (vs/8)*(gxu+gxu) is a
 // signed zero and h + tr = h whenever h != 0; tr (and the vertical differences it needs) is then formed
 // only where h == 0, which keeps every word of the general text.
+//
+// With u_in, v_in (a resident stage's first small step) the faces that no one
+// steps are copied from there, as the prepare pass does otherwise.
 template <bool SLOPES0>
-__global__ __launch_bounds__(PG_TX * PG_TY) void k_snd_pgrad(SoundArgs a) {
+__global__ __launch_bounds__(PG_TX * PG_TY) void k_snd_pgrad(SoundArgs a, int n) {
+  constexpr int KB = SLOPES0 ? 2 : 4;
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const int gx = (ni + 1 + PG_TX - 1) / PG_TX, gy = (nj + 1 + PG_TY - 1) / PG_TY;
-  const int tile = xcd_tile((int)blockIdx.x, gx * gy * nk);
-  const int k = tile / (gx * gy) + 1;
+  const int nkb = (nk + KB - 1) / KB;
+  const int tile = xcd_tile((int)blockIdx.x, gx * gy * nkb);
+  const int kb = (tile / (gx * gy)) * KB + 1;
   const int rem = tile % (gx * gy);
-  const int x = (rem % gx) * PG_TX + (int)threadIdx.x % PG_TX;  // 0..ni
-  const int y = (rem / gx) * PG_TY + (int)threadIdx.x / PG_TX;  // 0..nj
+  const int x = (rem % gx) * PG_TX + (int)threadIdx.x % PG_TX;  // i - 1, 0..ni
+  const int y = (rem / gx) * PG_TY + (int)threadIdx.x / PG_TX;  // j - 1, 0..nj
   if (x > ni || y > nj) return;
   const float halfcp = a.cp * 0.5f, eighth = 0.125f;
   const float* rds = P_rds(a);
-  const float* ppd = a.ppd;
-  // the terrain term of a face whose cells are (pj, pi) and (pjm, pim), slope pair gsum
-  auto terrain = [&](int pj, int pi, int pjm, int pim, float gsum) {
-    // vertical differences, same statement order for face and its west (south) cell
-    float dph = 0.0f, dphl = 0.0f, dpl = 0.0f, dpll = 0.0f;
-    if (k < nk) {
-      dph = (ppd[pix(k + 1, pj, pi, ni, nj)] - ppd[pix(k, pj, pi, ni, nj)]) * rds[k + 1];
-      dphl = (ppd[pix(k + 1, pjm, pim, ni, nj)] - ppd[pix(k, pjm, pim, ni, nj)]) * rds[k + 1];
-    }
-    if (k > 1) {
-      dpl = (ppd[pix(k, pj, pi, ni, nj)] - ppd[pix(k - 1, pj, pi, ni, nj)]) * rds[k];
-      dpll = (ppd[pix(k, pjm, pim, ni, nj)] - ppd[pix(k - 1, pjm, pim, ni, nj)]) * rds[k];
-    }
-    const float vs = (dph + dphl) + (dpl + dpll);
-    return (eighth * vs) * gsum;
-  };
-  // u face ff = x+1 (1-based) on row j = y
-  if (y < nj) {
-    const int ff = x + 1;
-    const bool on = (ff >= 2 && ff <= ni) || (ff == 1 && side_of(a.sides, 0) == 1u) ||
-                    (ff == ni + 1 && side_of(a.sides, 1) == 1u);
-    if (on) {
-      const int pj = y + 1;
-      const float h = (ppd[pix(k, pj, ff, ni, nj)] - ppd[pix(k, pj, ff - 1, ni, nj)]) * a.rdx;
-      float hs = h;
-      if (!SLOPES0 || h == 0.0f) {
-        const int64_t g = ((int64_t)(k - 1) * nj + y) * (ni + 1) + x;
-        hs = h + terrain(pj, ff, pj, ff - 1, a.gxu[g] + a.gxu[g + (int64_t)nj * (ni + 1)]);
-      }
-      const float pg = (halfcp * (a.thv[pix(k, pj, ff, ni, nj)] + a.thv[pix(k, pj, ff - 1, ni, nj)])) * hs;
-      const int64_t pu = ix3(k, y + NG, x + NG, sy(nj), ux(ni));
-      a.u3d[pu] = a.u3d[pu] + a.dts * (a.uten[pu] - pg);
+  const bool pw = side_of(a.sides, 0) == 1u, pe = side_of(a.sides, 1) == 1u;
+  const bool ps = side_of(a.sides, 2) == 1u, pn = side_of(a.sides, 3) == 1u;
+  const bool on_u = y < nj && (x > 0 || pw) && (x < ni || pe);
+  const bool on_v = x < ni && (y > 0 || ps) && (y < nj || pn);
+  const bool open_u =
+      y < nj && ((x == 0 && side_of(a.sides, 0) == 2u) || (x == ni && side_of(a.sides, 1) == 2u));
+  const bool open_v =
+      x < ni && ((y == 0 && side_of(a.sides, 2) == 2u) || (y == nj && side_of(a.sides, 3) == 2u));
+  const int i = x + 1, j = y + 1;
+  // ppd's own, west and south words (from the cells the fill copies, k_snd_pgrad_flat)
+  const int ic = a.map_ppd ? filled_index(i, ni, pw, pe) : i, iw = a.map_ppd ? filled_index(i - 1, ni, pw, pe) : i - 1;
+  const int jc = a.map_ppd ? filled_index(j, nj, ps, pn) : j, js = a.map_ppd ? filled_index(j - 1, nj, ps, pn) : j - 1;
+  const uint32_t opc = (uint32_t)((jc * (ni + 2) + ic) * 4), opw = (uint32_t)((jc * (ni + 2) + iw) * 4),
+                 ops = (uint32_t)((js * (ni + 2) + ic) * 4);
+  const uint32_t op = (uint32_t)((j * (ni + 2) + i) * 4), onp = (uint32_t)(ni + 2) * 4u;
+  const uint32_t ou = (uint32_t)(((y + NG) * ux(ni) + x + NG) * 4), ov = (uint32_t)(((y + NG) * sx(ni) + x + NG) * 4);
+  const int64_t pst = (int64_t)(nj + 2) * (ni + 2), ust = (int64_t)sy(nj) * ux(ni), vst = (int64_t)vy(nj) * sx(ni);
+  const uint32_t ogu = (uint32_t)((y * (ni + 1) + x) * 4), ogv = (uint32_t)((y * ni + x) * 4);
+  const int64_t gust = (int64_t)nj * (ni + 1), gvst = (int64_t)(nj + 1) * ni;
+  const float* usrc = (a.u_in && !open_u) ? a.u_in : a.u3d;
+  const float* vsrc = (a.v_in && !open_v) ? a.v_in : a.v3d;
+  const bool wr_u = on_u || (a.u_in && !open_u), wr_v = on_v || (a.v_in && !open_v);
+  const bool last = n == a.nloop;
+  const int au = open_u ? (a.avg_on ? AVG_SINGLE : AVG_NONE) : a.avg;
+  const int av = open_v ? (a.avg_on ? AVG_SINGLE : AVG_NONE) : a.avg;
+  const float tavg = 1.0f / (float)a.nloop;
+  float u[KB], ut[KB], v[KB], vt[KB], tc[KB], tw[KB], ts[KB], ru[KB], rv[KB];
+  // ppd at levels kb-1..kb+KB (the outer two only for the terrain term)
+  float dc[KB + 2], dw[KB + 2], ds[KB + 2], su[KB + 1], sv[KB + 1];
+#pragma unroll
+  for (int q = 0; q < KB + 2; ++q) {
+    const int k = kb - 1 + q;
+    dc[q] = dw[q] = ds[q] = 0.0f;
+    const bool own = q >= 1 && q <= KB;
+    if ((own || !SLOPES0) && k >= 1 && k <= nk) {
+      const float* P = a.ppd + (int64_t)k * pst;
+      dc[q] = ldo(P, opc);
+      dw[q] = ldo(P, opw);
+      ds[q] = ldo(P, ops);
     }
   }
-  // v face ff = y+1 on column i = x
-  if (x < ni) {
-    const int ff = y + 1;
-    const bool on = (ff >= 2 && ff <= nj) || (ff == 1 && side_of(a.sides, 2) == 1u) ||
-                    (ff == nj + 1 && side_of(a.sides, 3) == 1u);
-    if (on) {
-      const int pi = x + 1;
-      const float h = (ppd[pix(k, ff, pi, ni, nj)] - ppd[pix(k, ff - 1, pi, ni, nj)]) * a.rdy;
-      float hs = h;
-      if (!SLOPES0 || h == 0.0f) {
-        const int64_t g = ((int64_t)(k - 1) * (nj + 1) + y) * ni + x;
-        hs = h + terrain(ff, pi, ff - 1, pi, a.gyv[g] + a.gyv[g + (int64_t)(nj + 1) * ni]);
+#pragma unroll
+  for (int q = 0; q < KB; ++q) {
+    const int k = kb + q;
+    if (k <= nk) {
+      const float* T = a.thv + (int64_t)k * pst;
+      u[q] = ldo(usrc + (int64_t)k * ust, ou);
+      ut[q] = ldo(a.uten + (int64_t)k * ust, ou);
+      v[q] = ldo(vsrc + (int64_t)k * vst, ov);
+      vt[q] = ldo(a.vten + (int64_t)k * vst, ov);
+      tc[q] = ldo(T, op);
+      tw[q] = ldo(T, op - 4u);
+      ts[q] = ldo(T, op - onp);
+      ru[q] = (au && n > au) ? ldo(a.rru + (int64_t)k * ust, ou) : 0.0f;
+      rv[q] = (av && n > av) ? ldo(a.rrv + (int64_t)k * vst, ov) : 0.0f;
+    }
+  }
+  if constexpr (!SLOPES0) {
+#pragma unroll
+    for (int q = 0; q <= KB; ++q) {
+      const int k = kb - 1 + q;  // slopes of w levels kb..kb+KB (planes kb-1..)
+      su[q] = (on_u && k <= nk) ? ldo(a.gxu + (int64_t)k * gust, ogu) : 0.0f;
+      sv[q] = (on_v && k <= nk) ? ldo(a.gyv + (int64_t)k * gvst, ogv) : 0.0f;
+    }
+  }
+  // the vertical differences below and above each level
+  float lc = 0.0f, lw = 0.0f, ls = 0.0f;
+  if (!SLOPES0 && kb > 1) {
+    lc = (dc[1] - dc[0]) * rds[kb];
+    lw = (dw[1] - dw[0]) * rds[kb];
+    ls = (ds[1] - ds[0]) * rds[kb];
+  }
+#pragma unroll
+  for (int q = 0; q < KB; ++q) {
+    const int k = kb + q;
+    if (k > nk) break;
+    float hu = (dc[q + 1] - dw[q + 1]) * a.rdx, hv = (dc[q + 1] - ds[q + 1]) * a.rdy;
+    if constexpr (SLOPES0) {
+      auto terrain = [&](uint32_t ob, float d0, float b0, float gsum) {  // ob: the west (south) cell
+        float dph = 0.0f, dphl = 0.0f, dpl = 0.0f, dpll = 0.0f;
+        if (k < nk) {
+          const float* P = a.ppd + (int64_t)(k + 1) * pst;
+          dph = (ldo(P, opc) - d0) * rds[k + 1];
+          dphl = (ldo(P, ob) - b0) * rds[k + 1];
+        }
+        if (k > 1) {
+          const float* P = a.ppd + (int64_t)(k - 1) * pst;
+          dpl = (d0 - ldo(P, opc)) * rds[k];
+          dpll = (b0 - ldo(P, ob)) * rds[k];
+        }
+        const float vs = (dph + dphl) + (dpl + dpll);
+        return (eighth * vs) * gsum;
+      };
+      if (on_u && hu == 0.0f) {
+        const float* G = a.gxu + (int64_t)(k - 1) * gust;
+        hu = hu + terrain(opw, dc[q + 1], dw[q + 1], ldo(G, ogu) + ldo(G + gust, ogu));
       }
-      const float pg = (halfcp * (a.thv[pix(k, ff, pi, ni, nj)] + a.thv[pix(k, ff - 1, pi, ni, nj)])) * hs;
-      const int64_t pv = ix3(k, y + NG, x + NG, vy(nj), sx(ni));
-      a.v3d[pv] = a.v3d[pv] + a.dts * (a.vten[pv] - pg);
+      if (on_v && hv == 0.0f) {
+        const float* G = a.gyv + (int64_t)(k - 1) * gvst;
+        hv = hv + terrain(ops, dc[q + 1], ds[q + 1], ldo(G, ogv) + ldo(G + gvst, ogv));
+      }
+    } else {
+      float hc = 0.0f, hw = 0.0f, hs = 0.0f;
+      if (k < nk) {
+        hc = (dc[q + 2] - dc[q + 1]) * rds[k + 1];
+        hw = (dw[q + 2] - dw[q + 1]) * rds[k + 1];
+        hs = (ds[q + 2] - ds[q + 1]) * rds[k + 1];
+      }
+      hu = hu + (eighth * ((hc + hw) + (lc + lw))) * (su[q] + su[q + 1]);
+      hv = hv + (eighth * ((hc + hs) + (lc + ls))) * (sv[q] + sv[q + 1]);
+      lc = hc;
+      lw = hw;
+      ls = hs;
+    }
+    const float pgu = (halfcp * (tc[q] + tw[q])) * hu, pgv = (halfcp * (tc[q] + ts[q])) * hv;
+    const float un = on_u ? u[q] + a.dts * (ut[q] - pgu) : u[q];
+    const float vn = on_v ? v[q] + a.dts * (vt[q] - pgv) : v[q];
+    if (wr_u) sto(a.u3d + (int64_t)k * ust, ou, un);
+    if (wr_v) sto(a.v3d + (int64_t)k * vst, ov, vn);
+    if (au) {
+      const float t = (au == AVG_PAIR ? ru[q] + u[q] : ru[q]) + un;
+      sto(a.rru + (int64_t)k * ust, ou, last ? t * tavg : t);
+    }
+    if (av) {
+      const float t = (av == AVG_PAIR ? rv[q] + v[q] : rv[q]) + vn;
+      sto(a.rrv + (int64_t)k * vst, ov, last ? t * tavg : t);
     }
   }
 }
@@ -1776,6 +1864,275 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
   }
 }
 
+// ------------------------------------------------------------------ resident terrain pass
+// The terrain-coordinate column pass with pp, fpk and the old w of a thread's
+// own levels (at most CH) in registers, as the flat resident pass: four LDS
+// planes, the level table {rho0(k+1), r2 and height of w level k+1, rdsf(k)} and
+// the slots' last-level words.  qk is formed from ppterm (((dts*rdsf)*ppterm)*gz,
+// the prepare pass's own statement) and the u and v averages are the pressure
+// gradient's: 17 words a cell and step (u, v, w, wten, pp3d, ppten, ppterm,
+// piadv, rr0, rrf0, pk1, pk2, mm read; w, pp3d, ppd written; rrw at every second
+// step), against 23 of the seven-plane pass.  Its 92 registers allow two
+// workgroups a CU; it is bound by the latency of the levels' words and of the
+// recurrence, not by HBM (2.7 TB/s algorithmic).  Measured a small step at
+// 320x320x80: 251 -> 208 us (and 155 -> 123 at 192x256x80).  Slower: held to 80
+// registers for three workgroups (20 spilled, 272 us), the column's metrics kept
+// in LDS (15 spilled), ten waves a workgroup (one workgroup a CU); words requested
+// two levels ahead measured the same.
+int column4_lds_bytes(int nk, int cw, int slots) {
+  return (C3PLANES * (nk + 1) * cw + (nk + 1) * 4 + 2 * slots * cw) * (int)sizeof(float);
+}
+
+template <int C2W, int C2T, int CH>
+__global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(4))) void k_snd_column4(SoundArgs a, int n) {
+  constexpr int C2S = C2T / C2W;
+  extern __shared__ float lds[];
+  __shared__ float lw1[C2W];
+  const int ni = a.ni, nj = a.nj, nk = a.nk;
+  const int gx = (ni + 1 + C2W - 1) / C2W;
+  const int tile = xcd_tile((int)blockIdx.x, gx * (nj + 1));
+  const int j = tile / gx;
+  const int c = threadIdx.x % C2W, slot = threadIdx.x / C2W;
+  const int i = (tile % gx) * C2W + c;
+  const bool inside = (i <= ni);
+  const bool phys = (i < ni) && (j < nj);
+  const bool last = (n == a.nloop);
+  const float tavg = 1.0f / (float)a.nloop;
+  const int nxs = sx(ni), nys = sy(nj), nxu = ux(ni), nyv = vy(nj);
+  const int64_t wst = (int64_t)nys * nxs;
+  const int64_t wc = (int64_t)(j + NG) * nxs + (i + NG);
+  const int64_t uc = (int64_t)(j + NG) * nxu + (i + NG);
+  const int64_t ust = (int64_t)nys * nxu;
+  const int64_t vc = (int64_t)(j + NG) * nxs + (i + NG);
+  const int64_t vst = (int64_t)nyv * nxs;
+  float* w = a.w3d;
+  const int L = (nk + 1) * C2W;
+  float* Ls1 = lds;
+  float* Ls2 = lds + L;
+  float* Lmm = lds + 2 * L;
+  float* Ldd = lds + 3 * L;
+  float4* Ltab = reinterpret_cast<float4*>(lds + 4 * L);
+  float* Lbp = lds + 4 * L + (nk + 1) * 4;  // pp of each slot's last level
+  float* Lbf = Lbp + C2S * C2W;             // fpk of each slot's last level
+  auto at = [&](int k) { return k * C2W + c; };
+  for (int k = (int)threadIdx.x; k <= nk; k += C2T) {
+    const float sgf1 = P_sigmaf(a)[k + 1];
+    Ltab[k] = make_float4(a.rho0[(int64_t)min(k, nk - 1) * ((int64_t)nj * ni)],
+                          (sgf1 - P_sigma(a)[k]) * P_rds(a)[k + 1], (sgf1 - a.zt) * a.rzt, P_rdsf(a)[k]);
+  }
+  __syncthreads();
+  const int chunk = (nk + C2S - 1) / C2S;  // at most CH (checked by the launcher)
+  const int kb = 1 + slot * chunk, ke = min(nk, kb + chunk - 1);
+  const float asq = a.alph * a.alph;
+  const float smeps = 1.0e-20f;
+  const int pj = j + 1, pi = i + 1;
+  float rpp[CH], rfpk[CH], rwo[CH];
+  float wt0 = 0.0f, wo0 = 0.0f;  // level kb's wten and w, for its right-hand side after the barrier
+
+  // ---------------- phase A: fpk, the per-level terms and the right-hand sides
+  if (phys && kb <= ke) {
+    const uint32_t h = (uint32_t)(j * ni + i) * 4u, opl = (uint32_t)(nj * ni) * 4u;
+    const float g = ldo(a.gz, h), ddx = ldo(a.dzdx, h), ddy = ldo(a.dzdy, h);
+    const float* ru = a.rgzu + (int64_t)j * (ni + 1) + i;
+    const float* rv = a.rgzv + (int64_t)j * ni + i;
+    const float rgw = ru[0], rge = ru[1], rgs = rv[0], rgn = rv[ni];
+    const float temx = (a.dts * 0.5f) * a.rdx, temy = (a.dts * 0.5f) * a.rdy;
+    // the small step's w before it (w_in, set on the first small step: levels
+    // 1..nk, the lid stays in w3d)
+    const float* wi = a.w_in ? a.w_in : w;
+    const float* pp_in = (n == 1 && a.nrk != 1) ? a.ppi : a.pp3d;  // the first small step reads ppi
+    struct In {
+      float uw, ue, vs, vn, rrf1, wup, wt, ppten, ppterm, pc, pe, pw, pn, ps, rr0, pk1, pk2, pp, mm;
+    };
+    const uint32_t onp = (uint32_t)(ni + 2) * 4u, onx = (uint32_t)nxs * 4u, ows = (uint32_t)wst * 4u,
+                   ous = (uint32_t)ust * 4u, ovs = (uint32_t)vst * 4u;
+    auto load = [&](int k) {  // level k, and the faces of level k+1 (which exist at k = nk; unused there)
+      const uint32_t op = (uint32_t)pix(k, pj, pi, ni, nj) * 4u;
+      const uint32_t ou = (uint32_t)((int64_t)k * ust + uc) * 4u + ous;
+      const uint32_t ov = (uint32_t)((int64_t)k * vst + vc) * 4u + ovs;
+      const uint32_t ow = (uint32_t)((int64_t)k * wst + wc) * 4u;
+      const uint32_t om = (uint32_t)k * opl + h;
+      In v;
+      v.uw = ldo(a.u3d, ou);
+      v.ue = ldo(a.u3d, ou + 4u);
+      v.vs = ldo(a.v3d, ov);
+      v.vn = ldo(a.v3d, ov + onx);
+      v.rrf1 = ldo(a.rrf0, om);
+      v.wup = ldo(k + 1 <= nk ? wi : w, ow + ows);
+      v.wt = ldo(a.wten, ow);
+      v.ppten = ldo(a.ppten, op);
+      v.ppterm = ldo(a.ppterm, op);
+      v.pc = ldo(a.piadv, op);
+      v.pe = ldo(a.piadv, op + 4u);
+      v.pw = ldo(a.piadv, op - 4u);
+      v.pn = ldo(a.piadv, op + onp);
+      v.ps = ldo(a.piadv, op - onp);
+      v.rr0 = ldo(a.rr0, om - opl);
+      v.pk1 = ldo(a.pk1, op);
+      v.pk2 = ldo(a.pk2, op);
+      v.pp = ldo(pp_in, op);
+      v.mm = ldo(a.mm, op);
+      return v;
+    };
+    auto faces = [&](int k) {
+      const uint32_t ou = (uint32_t)((int64_t)k * ust + uc) * 4u, ov = (uint32_t)((int64_t)k * vst + vc) * 4u;
+      ColumnFaces f;
+      f.xw = ldo(a.u3d, ou) * rgw;
+      f.xe = ldo(a.u3d, ou + 4u) * rge;
+      f.ys = ldo(a.v3d, ov) * rgs;
+      f.yn = ldo(a.v3d, ov + onx) * rgn;
+      return f;
+    };
+    // the terrain terms of the w level between two levels' faces (lev: that w level's row of the table)
+    auto wterms = [&](const float4& lev, const ColumnFaces& hi, const ColumnFaces& lo, float rho_hi, float rho_lo,
+                      float rrf, float& dum3, float& hadvp) {
+      const float r2 = lev.y, height = lev.z;
+      const float r1 = 1.0f - r2;
+      {
+        const float xt = (r2 * (hi.xw + hi.xe) + r1 * (lo.xw + lo.xe)) * ddx;
+        const float yt = (r2 * (hi.ys + hi.yn) + r1 * (lo.ys + lo.yn)) * ddy;
+        dum3 = ((0.5f * (xt + yt)) * height) * g;
+      }
+      {
+        const float xt = (r2 * (rho_hi * hi.xw + rho_hi * hi.xe) + r1 * (rho_lo * lo.xw + rho_lo * lo.xe)) * ddx;
+        const float yt = (r2 * (rho_hi * hi.ys + rho_hi * hi.yn) + r1 * (rho_lo * lo.ys + rho_lo * lo.yn)) * ddy;
+        hadvp = (((0.5f * (xt + yt)) * height) * g) * rrf;
+      }
+    };
+    In nx = load(kb);
+    ColumnFaces flo = faces(kb);
+    float rho_lo = Ltab[kb - 1].x;
+    float dum3_lo = 0.0f, hadvp_lo = 0.0f, wraw, wold;
+    if (kb == 1) {
+      wold = wi[wst + wc];
+      wraw = bcwsfc_value(a.u3d, a.v3d, a.dzdx, a.dzdy, a.gz, j, i, ni, nj);
+      w[wst + wc] = wraw;
+      lw1[c] = wraw;
+    } else {
+      wold = wraw = wi[(int64_t)kb * wst + wc];
+      wterms(Ltab[kb - 1], flo, faces(kb - 1), rho_lo, Ltab[kb - 2].x, ldo(a.rrf0, (uint32_t)(kb - 1) * opl + h),
+             dum3_lo, hadvp_lo);
+    }
+#pragma unroll
+    for (int kk = 0; kk < CH; ++kk) {
+      const int k = kb + kk;
+      if (k <= ke) {
+        const In cu = nx;
+        if (k < ke) nx = load(k + 1);
+        const float4 lev = Ltab[k];
+        ColumnFaces fhi = flo;
+        float rho_hi = 0.0f, dum3_hi = 0.0f, hadvp_hi = 0.0f;
+        if (k < nk) {  // w level k+1 is interior
+          fhi.xw = cu.uw * rgw;
+          fhi.xe = cu.ue * rge;
+          fhi.ys = cu.vs * rgs;
+          fhi.yn = cu.vn * rgn;
+          rho_hi = lev.x;
+          wterms(lev, fhi, flo, rho_hi, rho_lo, cu.rrf1, dum3_hi, hadvp_hi);
+        }
+        const float hz = (flo.xe - flo.xw) * a.rdx + (flo.yn - flo.ys) * a.rdy;
+        const float vt = (dum3_hi - dum3_lo) * lev.w;
+        float div = g * (hz + vt);
+        if (fabsf(div) < smeps) div = 0.0f;
+        const float wk = (k == 1) ? 0.0f : wraw;
+        const float wk1 = (k == nk) ? 0.0f : cu.wup;
+        const float qk = ((a.dts * lev.w) * cu.ppterm) * g;
+        float fpk = a.dts * (cu.ppten - cu.ppterm * div) + a.beta * ((-qk) * (wk1 - wk));
+        const float u2 = temx * (rho_lo * flo.xe), u1 = temx * (rho_lo * flo.xw);
+        const float v2 = temy * (rho_lo * flo.yn), v1 = temy * (rho_lo * flo.ys);
+        const float ww2 = hadvp_hi + a.beta * cu.wup;
+        const float ww1 = hadvp_lo + a.beta * wraw;
+        const float xa = u2 * (cu.pe - cu.pc) + u1 * (cu.pc - cu.pw);
+        const float ya = v2 * (cu.pn - cu.pc) + v1 * (cu.pc - cu.ps);
+        float hza = (-(xa + ya)) * cu.rr0;
+        hza = hza * g;
+        const float vta = ww1 * cu.pk1 + ww2 * cu.pk2;
+        fpk = fpk + (hza + vta);
+        Ls1[at(k)] = cu.pk1 + qk;
+        Ls2[at(k)] = cu.pk2 - qk;
+        Lmm[at(k)] = cu.mm;
+        rpp[kk] = cu.pp;
+        rfpk[kk] = fpk;
+        rwo[kk] = kk == 0 ? wold : wraw;
+        if (kk == 0) {
+          wt0 = cu.wt;
+          wo0 = wraw;
+        } else {  // the right-hand side of level k from level k-1's words
+          const float pdelta = rpp[kk] - rpp[kk - 1];
+          const float fwk = a.dts * cu.wt + a.beta * ((-cu.mm) * pdelta);
+          const float udelta = (rpp[kk] + rfpk[kk]) - (rpp[kk - 1] + rfpk[kk - 1]);
+          Ldd[at(k)] = (wraw + fwk) + a.alph * ((-cu.mm) * udelta);
+        }
+        if (k == ke) {
+          Lbp[slot * C2W + c] = cu.pp;
+          Lbf[slot * C2W + c] = fpk;
+        }
+        flo = fhi;
+        rho_lo = rho_hi;
+        dum3_lo = dum3_hi;
+        hadvp_lo = hadvp_hi;
+        wraw = cu.wup;
+      }
+    }
+  }
+  __syncthreads();
+  // ---------------- a slot's first level: its right-hand side from the previous slot's last level
+  if (phys && kb <= ke && kb >= 2) {
+    const float ppm = Lbp[(slot - 1) * C2W + c], fm = Lbf[(slot - 1) * C2W + c];
+    const float mmk = Lmm[at(kb)];
+    const float pdelta = rpp[0] - ppm;
+    const float fwk = a.dts * wt0 + a.beta * ((-mmk) * pdelta);
+    const float udelta = (rpp[0] + rfpk[0]) - (ppm + fm);
+    Ldd[at(kb)] = (wo0 + fwk) + a.alph * ((-mmk) * udelta);
+  }
+  __syncthreads();
+  // ---------------- phase B: Thomas recurrence, one lane per column
+  if (phys && slot == 0) thomas_column<C2W>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
+  __syncthreads();
+  // ---------------- phase C: pressure update, filter, the w average
+  if (phys && kb <= ke) {
+    float rw[CH];
+#pragma unroll
+    for (int kk = 0; kk < CH; ++kk)
+      if (a.avg && kb + kk <= ke)
+        rw[kk] = n <= a.avg ? a.wa[(int64_t)(kb + kk) * wst + wc] * a.beta : a.rrw[(int64_t)(kb + kk) * wst + wc];
+#pragma unroll
+    for (int kk = 0; kk < CH; ++kk) {
+      const int k = kb + kk;
+      if (k <= ke) {
+        const int64_t p = pix(k, pj, pi, ni, nj);
+        const float wk = (k == 1) ? lw1[c] : Ldd[at(k)];
+        if (k >= 2) w[(int64_t)k * wst + wc] = wk;
+        const float w1 = (k == 1) ? 0.0f : wk;
+        const float w2 = (k == nk) ? 0.0f : Ldd[at(k + 1)];
+        const float old = rpp[kk];
+        const float vt = w1 * Ls1[at(k)] + w2 * Ls2[at(k)];
+        float up = (old + rfpk[kk]) + a.alph * vt;
+        if (fabsf(up) < smeps) up = 0.0f;
+        a.pp3d[p] = up;
+        const float tend = a.kdiv * (up - old);
+        a.ppd[p] = up + tend;
+        if (a.nrk == 3 && last) a.ppx[p] = tend;
+        if (a.avg) {
+          const float vw = (a.avg == AVG_PAIR ? rw[kk] + rwo[kk] : rw[kk]) + (last ? wk * a.alph : wk);
+          a.rrw[(int64_t)k * wst + wc] = last ? vw * tavg : vw;
+        }
+      }
+    }
+  } else if (inside) {
+    for (int k = kb; k <= ke; ++k) {
+      const int64_t pw = (int64_t)k * wst + wc;
+      const float wk = a.w_in ? a.w_in[pw] : w[pw];
+      if (a.w_in) w[pw] = wk;  // the east column's and north row's w, copied on the first step
+      if (a.avg) {  // (this w is the same in every small step)
+        const float r0 = n <= a.avg ? a.wa[pw] * a.beta : a.rrw[pw];
+        const float vw = (a.avg == AVG_PAIR ? r0 + wk : r0) + (last ? wk * a.alph : wk);
+        a.rrw[pw] = last ? vw * tavg : vw;
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------ radiation
 // Durran-Klemp phase speed of one edge row/column, averaged over k in order.
 // One workgroup per edge position: its lanes form the levels' phase speeds
@@ -1896,6 +2253,25 @@ static void launch_column3(bool narrow, const SoundArgs& a, int n, hipStream_t s
   }
 }
 
+// the resident terrain pass, likewise
+template <int C2W, int C2T>
+static void launch_column4_tile(int chunk, dim3 grid, int lds, const SoundArgs& a, int n, hipStream_t s) {
+  if (chunk <= 3) hipLaunchKernelGGL((k_snd_column4<C2W, C2T, 3>), grid, dim3(C2T), lds, s, a, n);
+  else if (chunk <= 4) hipLaunchKernelGGL((k_snd_column4<C2W, C2T, 4>), grid, dim3(C2T), lds, s, a, n);
+  else if (chunk <= 5) hipLaunchKernelGGL((k_snd_column4<C2W, C2T, 5>), grid, dim3(C2T), lds, s, a, n);
+  else if (chunk <= 6) hipLaunchKernelGGL((k_snd_column4<C2W, C2T, 6>), grid, dim3(C2T), lds, s, a, n);
+  else hipLaunchKernelGGL((k_snd_column4<C2W, C2T, 8>), grid, dim3(C2T), lds, s, a, n);
+}
+
+static void launch_column4(bool narrow, const SoundArgs& a, int n, hipStream_t s) {
+  const int cw = narrow ? 16 : 32, slots = 16;
+  const dim3 grid(((a.ni + 1 + cw - 1) / cw) * (a.nj + 1));
+  const int lds = column4_lds_bytes(a.nk, cw, slots);
+  const int chunk = (a.nk + slots - 1) / slots;
+  if (narrow) launch_column4_tile<16, 256>(chunk, grid, lds, a, n, s);
+  else launch_column4_tile<32, 512>(chunk, grid, lds, a, n, s);
+}
+
 static int psolver3_stage(
     float* ppi, float* pp3d, float* ppx, float* ppd, const float* piadv, const float* ppterm, const float* ppten,
     const float* thv, float* qk, float* pk1, float* pk2, float* mm, float* fpk, float* elim_c, float* elim_d,
@@ -1955,8 +2331,12 @@ static int psolver3_stage(
     return (int)hipErrorInvalidValue;
   // flags & 128: the flat pass with its own levels' pressure words in registers
   // (16 level slots of at most 8 levels: nk <= 128)
-  const bool resident = (flags & 128) != 0;
-  if (resident && (!flat || fuse || nk > 128 || column3_lds_bytes(nk, cw, 16) > lds_max ||
+  // (the terrain column's pipelined request runs its resident pass where the column fits it)
+  const bool resident = flat ? (flags & 128) != 0
+                             : pipe && nk <= 128 && column4_lds_bytes(nk, cw, 16) <= lds_max &&
+                                   span < ((int64_t)1 << 32);
+  if ((flags & 128) && !flat) return (int)hipErrorInvalidValue;
+  if (resident && flat && (fuse || nk > 128 || column3_lds_bytes(nk, cw, 16) > lds_max ||
                    span >= ((int64_t)1 << 32)))
     return (int)hipErrorInvalidValue;
   a.fresh_averages = resident ? 1 : 0;
@@ -1969,7 +2349,7 @@ static int psolver3_stage(
   const bool start_alt = fuse && (nloop & 1);
   if (fuse) a.ppd_twin = ppd_alt;
   if (start_alt) { a.u_start = u_alt; a.v_start = v_alt; }
-  if (resident && a.skip_ppd)
+  if (resident && a.skip_ppd && flat)
     hipLaunchKernelGGL(k_snd_prepare_ring, dim3((2 * (ni + 2) + 2 * nj + 255) / 256, nk), dim3(256), 0, s, a);
   else
     hipLaunchKernelGGL(k_snd_prepare, dim3((ni + 2 + 63) / 64, nj + 2, nk), dim3(64), 0, s, a);
@@ -2037,25 +2417,37 @@ static int psolver3_stage(
     }
   }
   for (int n = 1; n <= nloop && !flat; ++n) {
-    if (any_open) {
-      if (nk <= SS_MAXK) hipLaunchKernelGGL(k_snd_ssopen2, dim3(edge), dim3(SS_T), 0, s, a);
-      else hipLaunchKernelGGL(k_snd_ssopen, dim3((edge + 63) / 64), dim3(64), 0, s, a);
+    SoundArgs b = a;
+    first_step(b, n);
+    if (resident) {
+      b.avg = (n % 2 == 0) ? AVG_PAIR : (n == nloop) ? AVG_SINGLE : AVG_NONE;
+      b.map_ppd = (n > 1 && all_sides) ? 1 : 0;
     }
+    if (any_open) {
+      if (nk <= SS_MAXK) hipLaunchKernelGGL(k_snd_ssopen2, dim3(edge), dim3(SS_T), 0, s, b);
+      else hipLaunchKernelGGL(k_snd_ssopen, dim3((edge + 63) / 64), dim3(64), 0, s, b);
+    }
+    SoundArgs pg = b;
+    if (a.skip_ppd && n == 1) pg.ppd = ppx;  // ppd = ppx until the first small step writes it
     // flags & 32: the caller states the terrain slopes gxu, gyv are +0 everywhere
-    const dim3 pgrid(((ni + 1 + PG_TX - 1) / PG_TX) * ((nj + 1 + PG_TY - 1) / PG_TY) * nk);
+    const int ptiles = ((ni + 1 + PG_TX - 1) / PG_TX) * ((nj + 1 + PG_TY - 1) / PG_TY);
     GM1_TIMED(TK_ACOUSTIC_SMALL_STEP, s, {
       if (flags & 32)
-        GM1_TIMED(TK_ACOUSTIC_PGRAD, s, hipLaunchKernelGGL(k_snd_pgrad<true>, pgrid, dim3(PG_TX * PG_TY), 0, s, a));
+        GM1_TIMED(TK_ACOUSTIC_PGRAD, s,
+                  hipLaunchKernelGGL(k_snd_pgrad<true>, dim3(ptiles * ((nk + 1) / 2)), dim3(PG_TX * PG_TY), 0, s, pg, n));
       else
-        GM1_TIMED(TK_ACOUSTIC_PGRAD, s, hipLaunchKernelGGL(k_snd_pgrad<false>, pgrid, dim3(PG_TX * PG_TY), 0, s, a));
-      if (staged)
+        GM1_TIMED(TK_ACOUSTIC_PGRAD, s,
+                  hipLaunchKernelGGL(k_snd_pgrad<false>, dim3(ptiles * ((nk + 3) / 4)), dim3(PG_TX * PG_TY), 0, s, pg, n));
+      if (resident)
+        GM1_TIMED(TK_ACOUSTIC_COLUMN, s, launch_column4(narrow, b, n, s));
+      else if (staged)
         GM1_TIMED(TK_ACOUSTIC_COLUMN, s, launch_column2<false>(narrow, pipe, a, n, s));
       else
         GM1_TIMED(TK_ACOUSTIC_COLUMN, s,
                   hipLaunchKernelGGL(k_snd_column, dim3((ni + 1 + 63) / 64, nj + 1), dim3(64), 0, s, a, n));
     });
     GM1_LAUNCH_CHECK();
-    if (n < nloop) {
+    if (n < nloop && (!(resident && all_sides) || n == nloop - 1)) {
       int rc = fill_pressure(ppd, sides, ni, nj, nk, s);
       if (rc) return rc;
     }

@@ -127,8 +127,9 @@ def verify_terrain_slopes_zero(metrics: Mapping[str, Any]) -> bool:
 
 # column pass name -> the stage call's flag bits: "staged" is 32 columns x 512
 # threads per workgroup, "staged16" 16 x 256; the "pipelined" forms issue each
-# level's loads a level ahead and run the u/v time averages beside the
-# recurrence; "register" walks each column in one thread
+# level's loads a level ahead and, up to 128 levels, keep the pressure words of a
+# thread's own levels in registers and leave the u/v time averages to the
+# pressure-gradient pass; "register" walks each column in one thread
 COLUMN_PASSES = {"staged": 0, "pipelined": 16, "staged16": 8, "pipelined16": 24, "register": 4}
 # the flat column runs the LDS-staged passes (the register pass is the terrain text); its
 # "fused" forms also step u and v inside the pipelined pass (one pass per small step instead

@@ -52,3 +52,39 @@ def test_gpu_flat_resident_stage_equals_the_staged_one(device, monkeypatch, nloo
             for n in OUT:
                 assert_bits_equal(got[n], want[n], f"{column_pass} stage {nrk} {n}")
     assert np.isfinite(runs["staged"][1]["w3d"]).all() and np.abs(runs["staged"][1]["w3d"]).max() > 0.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nloop", [1, 2, 3, 6])
+@pytest.mark.parametrize("sides,ni,nj,nk,slopes", [((2, 2, 2, 2), 33, 9, 18, True), ((1, 1, 2, 2), 32, 11, 49, False),
+                                                   ((2, 4, 1, 1), 31, 8, 65, True), ((4, 2, 2, 4), 64, 9, 81, False),
+                                                   ((1, 1, 1, 1), 9, 33, 128, True), ((2, 2, 1, 1), 40, 8, 130, True)])
+def test_gpu_terrain_pipelined_stage_equals_the_staged_one(device, monkeypatch, nloop, sides, ni, nj, nk, slopes):
+    """The resident terrain pass (up to 128 levels; beyond, the seven-plane one) and the pressure gradient's levels,
+    averages and mapped halo words, with and without slopes, on every chunk of levels a thread may own."""
+    import torch
+    from helpers import to_dev
+    from test_sound import _acoustic_case
+
+    from gm1_amd import psolver3
+
+    print(f"terrain stage {ni}x{nj}x{nk} sides {sides} nloop {nloop}", flush=True)
+    a0, m0 = _acoustic_case(np.random.default_rng(nk + nloop), ni, nj, nk, terrain=slopes)
+    m = to_dev(m0, device)
+    monkeypatch.setattr(psolver3, "sound3_stage_schedule_f32", lambda dt, ns, nrk: (nloop, float(np.float32(dt / ns))))
+    runs = {}
+    for column_pass in ("staged", "pipelined", "pipelined16"):
+        a = to_dev(a0, device)
+        out = []
+        for nrk in (1, 3):
+            psolver3.launch_cuda_psolver3_terrain_open_stage(a, m, ni=ni, nj=nj, nk=nk, nrk=nrk, dt=0.5, nsound=8,
+                                                             dx=250.0, dy=200.0, dz=150.0, lateral_sides=sides,
+                                                             column_pass=column_pass, terrain_slopes_zero=not slopes)
+            torch.cuda.synchronize()
+            out.append({n: to_host(a[n]) for n in OUT + ("qk", "pk1", "pk2", "mm")})
+        runs[column_pass] = out
+    for column_pass in ("pipelined", "pipelined16"):
+        for got, want, nrk in zip(runs[column_pass], runs["staged"], (1, 3)):
+            for n in got:
+                assert_bits_equal(got[n], want[n], f"{column_pass} stage {nrk} {n}")
+    assert np.isfinite(runs["staged"][1]["w3d"]).all()
