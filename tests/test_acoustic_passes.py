@@ -88,3 +88,26 @@ def test_gpu_terrain_pipelined_stage_equals_the_staged_one(device, monkeypatch, 
             for n in got:
                 assert_bits_equal(got[n], want[n], f"{column_pass} stage {nrk} {n}")
     assert np.isfinite(runs["staged"][1]["w3d"]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ni,nj,nk,nsound", [(17, 5, 3, 4), (16, 4, 32, 6), (15, 3, 33, 4), (33, 6, 65, 8), (48, 3, 97, 4),
+                                             (9, 4, 128, 6), (8, 3, 130, 4)])
+def test_gpu_periodic_column_passes_equal_the_oracle(ni, nj, nk, nsound):
+    """Every chunk of levels a slot may own (1 to 4 levels of 32 slots), ragged tiles, both parities of the averages'
+    pairs, and a column too tall for the staged pass: every compared output, after each stage, word for word."""
+    from test_sound3_periodic import _to_device, differing, seeded_case
+
+    from gm1_amd.sound3_periodic import launch_cuda_sound3_periodic_stage
+    from oracle import sound3_periodic as osp
+
+    a = seeded_case(ni, nj, nk, nk)
+    for n in ("tri_aa", "tri_bb", "tri_cc", "tri_dd", "tri_pivot", "tri_residual", "divh", "hadvp", "elim_c", "elim_d"):
+        a[n][...] = np.float32(7.0)  # words that a stage zeroes or writes
+    d = _to_device(a, "cuda")
+    params = dict(dt=2.0, nsound=nsound, rdx=1e-3, rdy=1e-3, rdz=1 / 500)
+    print(f"periodic stage {ni}x{nj}x{nk} nsound {nsound}", flush=True)
+    for nrk in (1, 2, 3):
+        launch_cuda_sound3_periodic_stage(d, ni=ni, nj=nj, nk=nk, nrk=nrk, **params)
+        osp.stage(a, ni=ni, nj=nj, nk=nk, nrk=nrk, **params)
+        assert differing({n: d[n].cpu().numpy() for n in osp.COMPARE_OUTPUT_NAMES}, a) == {}, f"stage {nrk}"
