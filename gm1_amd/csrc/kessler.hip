@@ -52,8 +52,95 @@ GM1_DEV KesConst kes_const() {
   return c;
 }
 
-GM1_DEV float exp_r(float x) { return (float)exp((double)x); }
-GM1_DEV float pow_r(float b, float e) { return (float)pow((double)b, (double)e); }
+// exp and pow in binary64 rounded once to binary32, by Ziv's method (A. Ziv,
+// ACM TOMS 17, 1991): a short binary64 evaluation whose relative error is below
+// 2^-44 decides the binary32 word unless it lies within 2^-41 of the midpoint of
+// two binary32 numbers; there (about one value in 2^17), and where argument or
+// result leaves the normal range, the library's binary64 function does.  The
+// words are therefore the library's rounded words everywhere.  The cell and column
+// passes were bound by these functions and by the registers the library's pow
+// holds (it is called, not inlined, so the usual path's registers decide): at
+// 320x320x80 with cloud and rain in two cells of five the cell pass takes 292 ->
+// 184 us and the column pass 221 -> 141; on a storm of 640x768x80, where HBM
+// bounds them (5.3 TB/s a copy), 1187 -> 899 and 862 -> 680.
+//
+// log(m) = 2 artanh(s), s = (m-1)/(m+1), |s| <= 0.1716: the artanh series to
+// s^17 (the next term is below 2^-51 of the sum); exp(x) = exp(x/2)^2 with the
+// Taylor series to the 10th power on |x/2| <= 0.1733 (next term below 2^-53).
+struct Near {
+  double log_m;  // natural logarithm of the significand in [sqrt(1/2), sqrt(2))
+  double ex;     // and the power of two
+  bool ok;       // a positive normal number
+};
+
+// binary64 rounded once: the words that decide where the short forms do not
+__device__ __attribute__((noinline)) float pow_library(float b, float e) { return (float)pow((double)b, (double)e); }
+__device__ __attribute__((noinline)) float exp_library(float x) { return (float)exp((double)x); }
+
+GM1_DEV Near log_near(float b) {
+  const unsigned u = __float_as_uint(b);
+  Near r;
+  r.ok = u - 0x00800000u < 0x7f000000u;
+  const bool up = (u & 0x007fffffu) > 0x003504f3u;
+  const double m = (double)__uint_as_float((u & 0x007fffffu) | (up ? 0x3f000000u : 0x3f800000u));
+  r.ex = (double)((int)(u >> 23) - (up ? 126 : 127));
+  const double n = m - 1.0, d = m + 1.0;
+  double y = (double)__builtin_amdgcn_rcpf((float)d);
+  y = fma(y, fma(-d, y, 1.0), y);
+  double s = n * y;
+  s = fma(y, fma(-d, s, n), s);
+  const double z = s * s;
+  double p = 1.0 / 17.0;
+  p = fma(p, z, 1.0 / 15.0);
+  p = fma(p, z, 1.0 / 13.0);
+  p = fma(p, z, 1.0 / 11.0);
+  p = fma(p, z, 1.0 / 9.0);
+  p = fma(p, z, 1.0 / 7.0);
+  p = fma(p, z, 1.0 / 5.0);
+  p = fma(p, z, 1.0 / 3.0);
+  r.log_m = 2.0 * fma(s * z, p, s);
+  return r;
+}
+
+constexpr double LOG2E = 1.4426950408889634, HALF_LN2 = 0.34657359027997264;
+
+// 2^t, |t| < 1000
+GM1_DEV double exp2_near(double t) {
+  const double n = rint(t);
+  const double x = (t - n) * HALF_LN2;
+  double p = 1.0 / 3628800.0;
+  p = fma(p, x, 1.0 / 362880.0);
+  p = fma(p, x, 1.0 / 40320.0);
+  p = fma(p, x, 1.0 / 5040.0);
+  p = fma(p, x, 1.0 / 720.0);
+  p = fma(p, x, 1.0 / 120.0);
+  p = fma(p, x, 1.0 / 24.0);
+  p = fma(p, x, 1.0 / 6.0);
+  p = fma(p, x, 0.5);
+  p = fma(p, x, 1.0);
+  p = fma(p, x, 1.0);
+  return ldexp(p * p, (int)n);
+}
+
+// y, an approximation within 2^-44 of a value, rounds to the value's binary32 word
+GM1_DEV bool rounds_safely(double y) {
+  const long long b = __double_as_longlong(y);
+  const int tail = (int)(b & 0x1fffffff) - 0x10000000;  // the bits below binary32's last, from the midpoint
+  return y > 1.2e-38 && y < 3.0e38 && (tail > 2048 || tail < -2048);
+}
+
+GM1_DEV float exp_r(float x) {
+  const double y = exp2_near((double)fminf(fmaxf(x, -200.0f), 200.0f) * LOG2E);
+  return (rounds_safely(y)) ? (float)y : exp_library(x);
+}
+
+GM1_DEV float pow_of(const Near& l, float b, float e) {
+  const double t = fma(l.ex, (double)e, l.log_m * ((double)e * LOG2E));
+  const double y = exp2_near(fmin(fmax(t, -200.0), 200.0));
+  return (l.ok && rounds_safely(y)) ? (float)y : pow_library(b, e);
+}
+
+GM1_DEV float pow_r(float b, float e) { return pow_of(log_near(b), b, e); }
 
 GM1_DEV float sat_qv(const KesConst& c, float t, float prs_cap, float pden) {
   float esl = 611.2f * exp_r((17.67f * (t - 273.15f)) / (t - 29.65f));
@@ -85,8 +172,10 @@ struct KesArgs {
 // ------------------------------------------------------------------ column phase
 // Column loops load KB levels at a time (independent loads in flight) and
 // then run the level arithmetic in k order, so every binary64 sum and every
-// carried value is the sequential one.
-constexpr int KB = 8;
+// carried value is the sequential one.  (KB = 4 runs two waves a SIMD, 8 one:
+// 141 against 192 us at 320x320x80 and 680 against 766 at 640x768x80, but 56
+// against 51 at 97x61x50; 2 takes 167, 746 and 68.)
+constexpr int KB = 4;
 
 __global__ __launch_bounds__(64) void k_kes_column(KesArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -323,9 +412,10 @@ __global__ __launch_bounds__(64) void k_kes_cell(KesArgs a) {
       if (qv < qvs) {
         word |= 8u;
         const float rhoqr = rho * qr;
-        const float vent = 1.6f + 30.3922f * pow_r(rhoqr, 0.2046f);
+        const Near lrq = log_near(rhoqr);
+        const float vent = 1.6f + 30.3922f * pow_of(lrq, rhoqr, 0.2046f);
         const float deficit = 1.0f - qv / qvs;
-        const float num = (vent * deficit) * pow_r(rhoqr, 0.525f);
+        const float num = (vent * deficit) * pow_of(lrq, rhoqr, 0.525f);
         const float den = (2.03e4f + 9.584e6f / (qvs * prs)) * rho;
         er = fminf((num / den) * dt, qr);
         if (qv + er > qvs) {
