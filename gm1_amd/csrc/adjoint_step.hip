@@ -69,12 +69,14 @@ struct W {
   double weps;
   Consts c;
   Cols col;
-  // index of (level l, row j, column i), levels 1-based
-  __device__ __forceinline__ int64_t at(int l, int j, int i) const {
-    return ((int64_t)(l - 1) * nj + j) * ni + i;
-  }
-  __device__ __forceinline__ int X(int i, int o) const { return (i + o + 4 * ni) % ni; }
-  __device__ __forceinline__ int Y(int j, int o) const { return (j + o + 4 * nj) % nj; }
+  // index of (level l, row j, column i), levels 1-based (a field holds fewer than 2^31 words,
+  // checked before the first launch, so indices are 32-bit)
+  __device__ __forceinline__ int at(int l, int j, int i) const { return ((l - 1) * nj + j) * ni + i; }
+  // periodic neighbours; i + o and j + o lie within one period of the grid (stencils reach at
+  // most four points past it, and ni, nj >= 6)
+  __device__ __forceinline__ int X(int i, int o) const { return wrap(i + o, ni); }
+  __device__ __forceinline__ int Y(int j, int o) const { return wrap(j + o, nj); }
+  static __device__ __forceinline__ int wrap(int v, int n) { return v < 0 ? v + n : v >= n ? v - n : v; }
   __device__ __forceinline__ int64_t plane() const { return (int64_t)nk * nj * ni; }
   __device__ __forceinline__ int64_t wplane() const { return (int64_t)(nk + 1) * nj * ni; }
   // substep snapshot n of a cell/u/v array or of w
@@ -109,7 +111,7 @@ Cols make_cols(const float* col, int nk) {
 __global__ __launch_bounds__(64) void k_terms(W w) {
   CELL_INDEX
   const Consts& c = w.c;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float th = w.p[XTH][q], pp = w.p[XPP][q];
   const float theta = w.col.th0[l - 1] + th;
   float b = th * w.col.rth[l - 1] + c.repsm1 * (0.0f - w.col.qv0[l - 1]);
@@ -124,7 +126,7 @@ __global__ __launch_bounds__(64) void k_terms(W w) {
 
 __global__ __launch_bounds__(64) void k_mass(W w) {
   CELL_INDEX
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float den = 0.5f * (w.col.rho[l - 1] + w.col.rho[l - 1]);
   w.p[RRU][q] = den * w.p[XU][q];
   w.p[RRV][q] = den * w.p[XV][q];
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(64) void k_coef(W w) {
   CELL_INDEX
   const Consts& c = w.c;
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float tem = c.dts * w.col.rdsf[l];
   w.p[QK][q] = (tem * w.p[PPTERM][q]) * 1.0f;
   const float tem2 = ((c.dts * 1.0f) * w.col.rdsf[l]) * w.col.rr0[l - 1];
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(64) void k_rows(W w);
 
 __global__ __launch_bounds__(64) void k_ac_start(W w) {
   CELL_INDEX
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const bool first = w.nrk == 1;
   w.snap(SPPD, 0)[q] = w.p[PPX][q];
   w.snap(SPP, 0)[q] = first ? w.p[XPP][q] : w.p[API][q];
@@ -527,7 +529,7 @@ __global__ __launch_bounds__(64) void k_ac_start(W w) {
   w.p[ARV][q] = 0.0f;
   w.p[ARW][q] = w.p[AW][q] * w.c.beta;
   if (l == w.nk) {
-    const int64_t top = w.at(w.nk + 1, j, i);
+    const int top = w.at(w.nk + 1, j, i);
     w.wsnap(0)[top] = w.p[XW][top];
     w.p[ARW][top] = 0.0f;
   }
@@ -540,16 +542,16 @@ __global__ __launch_bounds__(64) void k_ss_pgrad(W w, int n) {
   const bool last = n == w.nloop;
   const float* thv = w.p[THV];
   const float* ppd = w.snap(SPPD, n - 1);
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   {
-    const int64_t qw = w.at(l, j, w.X(i, -1));
+    const int qw = w.at(l, j, w.X(i, -1));
     const float pg = (c.halfcp * (thv[q] + thv[qw])) * ((ppd[q] - ppd[qw]) * c.rdx);
     const float u1 = w.snap(SU, n - 1)[q] + c.dts * (w.p[UTEN][q] - pg);
     w.snap(SU, n)[q] = u1;
     w.p[ARU][q] = last ? (w.p[ARU][q] + u1) * c.tavg : w.p[ARU][q] + u1;
   }
   {
-    const int64_t qs = w.at(l, w.Y(j, -1), i);
+    const int qs = w.at(l, w.Y(j, -1), i);
     const float pg = (c.halfcp * (thv[q] + thv[qs])) * ((ppd[q] - ppd[qs]) * c.rdy);
     const float v1 = w.snap(SV, n - 1)[q] + c.dts * (w.p[VTEN][q] - pg);
     w.snap(SV, n)[q] = v1;
@@ -565,8 +567,8 @@ __device__ __forceinline__ float column_fpk(const W& w, int n, int l, int j, int
   const float* v1 = w.snap(SV, n);
   const float* ws = w.wsnap(n - 1);
   const float* pia = w.p[PIADV];
-  const int64_t q = w.at(l, j, i);
-  const int64_t qe = w.at(l, j, w.X(i, 1)), qn = w.at(l, w.Y(j, 1), i);
+  const int q = w.at(l, j, i);
+  const int qe = w.at(l, j, w.X(i, 1)), qn = w.at(l, w.Y(j, 1), i);
   const float hz = (u1[qe] - u1[q]) * c.rdx + (v1[qn] - v1[q]) * c.rdy;
   float div = 1.0f * (hz + 0.0f);
   div = fabsf(div) < 1.0e-20f ? 0.0f : div;
@@ -598,7 +600,7 @@ __device__ __forceinline__ Row thomas_row(const W& w, int k, int j, int i) {
   const int nk = w.nk;
   const float asq = w.c.asq;
   const float *qk = w.p[QK], *pk1 = w.p[PK1], *pk2 = w.p[PK2], *mm = w.p[MM];
-  const int64_t q = w.at(k, j, i), qd = w.at(k - 1, j, i);
+  const int q = w.at(k, j, i), qd = w.at(k - 1, j, i);
   Row r;
   r.aa = k >= 3 ? (-asq) * (mm[q] * (pk1[qd] + qk[qd])) : 0.0f;
   r.cc = k < nk ? (-asq) * ((-mm[q]) * (pk2[q] - qk[q])) : 0.0f;
@@ -612,7 +614,7 @@ __global__ __launch_bounds__(64) void k_rows(W w) {
   CELL_INDEX
   if (l < 2) return;
   const Row r = thomas_row(w, l, j, i);
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   w.p[RA][q] = r.aa;
   w.p[RB][q] = r.bb;
   w.p[RC][q] = r.cc;
@@ -626,7 +628,7 @@ __global__ __launch_bounds__(64) void k_ss_rhs(W w, int n) {
   const float* ws = w.wsnap(n - 1);
   const float* pp = w.snap(SPP, n - 1);
   const float* fpk = w.p[FPK];
-  const int64_t q = w.at(l, j, i), qd = w.at(l - 1, j, i);
+  const int q = w.at(l, j, i), qd = w.at(l - 1, j, i);
   const float mmk = w.p[MM][q];
   const float pdelta = pp[q] - pp[qd];
   const float fwk = c.dts * w.p[WTEN][q] + c.beta * ((-mmk) * pdelta);
@@ -662,7 +664,7 @@ __global__ __launch_bounds__(64) void k_ss_thomas(W w, int n) {
 #pragma unroll
     for (int u = 0; u < TH_CHUNK; ++u) {
       const int k = k0 + u;
-      const int64_t q = w.at(k <= nk ? k : nk, j, i);
+      const int q = w.at(k <= nk ? k : nk, j, i);
       a[u] = ra[q];
       bb[u] = rb[q];
       c[u] = rc[q];
@@ -672,7 +674,7 @@ __global__ __launch_bounds__(64) void k_ss_thomas(W w, int n) {
     for (int u = 0; u < TH_CHUNK; ++u) {
       const int k = k0 + u;
       if (k > nk) break;
-      const int64_t q = w.at(k, j, i);
+      const int q = w.at(k, j, i);
       const float pivot = k == 2 ? bb[u] : a[u] * ecd + bb[u];
       const float inv = 1.0f / pivot;
       if (k < nk) {
@@ -692,7 +694,7 @@ __global__ __launch_bounds__(64) void k_ss_thomas(W w, int n) {
 #pragma unroll
     for (int u = 0; u < TH_CHUNK; ++u) {
       const int k = k1 - u;
-      const int64_t q = w.at(k >= 2 ? k : 2, j, i);
+      const int q = w.at(k >= 2 ? k : 2, j, i);
       e[u] = ec[q];
       f[u] = ed[q];
     }
@@ -716,7 +718,7 @@ __global__ __launch_bounds__(64) void k_ss_update(W w, int n) {
   const bool last = n == w.nloop;
   const float* wn = w.wsnap(n);
   const float* pp = w.snap(SPP, n - 1);
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float wlo = l == 1 ? 0.0f : wn[q];
   const float whi = l == nk ? 0.0f : wn[w.at(l + 1, j, i)];
   const float vt = wlo * (w.p[PK1][q] + w.p[QK][q]) + whi * (w.p[PK2][q] - w.p[QK][q]);
@@ -728,6 +730,146 @@ __global__ __launch_bounds__(64) void k_ss_update(W w, int n) {
   if (w.nrk == 3 && last) w.p[PPXO][q] = tend;
   float* arw = w.p[ARW];
   arw[q] = last ? (arw[q] + wn[q] * c.alph) * c.tavg : arw[q] + wn[q];
+}
+
+// ------------------------------------------------------------------ staged columns
+// One substep's column work in one pass: a workgroup owns CW columns of one row
+// and all levels, CS level slots a chunk of at most CH levels each.  Every slot
+// forms its levels' words at once (registers), the recurrence runs out of LDS
+// with one lane a column, and every slot finishes its levels.  What the passes
+// above hand each other through HBM (fpk, the right side, ec, ed) stays in
+// registers and LDS: 16 words a cell forward instead of 36.  At 192x192x64 (a
+// field is 9.4 MB, most of the working set stays in the last-level cache) a
+// forward substep's column takes 52 us against 85 in four passes, and its adjoint
+// (k_b_ss_column) 104 against 191 in three; the adjoint of a step 7.75 -> 6.06 ms,
+// with the neighbour indices wrapped by compares instead of a modulo (k_advu, v, w
+// 46 -> 27 us, k_theta 87 -> 69).
+constexpr int CW = 32, CS = 16, MAX_STAGED_NK = 8 * CS;
+
+int staged_lds_bytes(int nk) { return (4 * (nk + 2) + 2 * CS) * CW * (int)sizeof(float); }
+
+// substep n: fpk, the right side, the Thomas solve, the pressure update, filter, ppx and w running sum
+template <int CH>
+__global__ __launch_bounds__(CW* CS) void k_ss_column(W w, int n) {
+  extern __shared__ float lds[];
+  const Consts& c = w.c;
+  const int nk = w.nk, lane = threadIdx.x % CW, slot = threadIdx.x / CW;
+  const int i = (int)blockIdx.x * CW + lane, j = blockIdx.y;
+  const int chunk = (nk + CS - 1) / CS, kb = 1 + slot * chunk, ke = min(nk, kb + chunk - 1);
+  const bool col = i < w.ni, mine = col && kb <= ke;
+  const bool last = n == w.nloop;
+  const int L = (nk + 2) * CW;
+  float *Laa = lds, *Lbb = lds + L, *Lcc = lds + 2 * L, *Ldd = lds + 3 * L;
+  float *Lbf = lds + 4 * L, *Lbp = Lbf + CS * CW;  // fpk and pp of each slot's last level
+  auto at = [&](int k) { return k * CW + lane; };
+  const float* ws = w.wsnap(n - 1);
+  float* wn = w.wsnap(n);
+  const float* pp = w.snap(SPP, n - 1);
+  float rpp[CH], rf[CH], rs1[CH], rs2[CH], rmm[CH], rar[CH], wt[CH], wo[CH];
+  if (mine) {
+    float s1m = 0.0f, s2m = 0.0f;
+    if (kb > 1) {
+      const int qd = w.at(kb - 1, j, i);
+      const float qk = w.p[QK][qd];
+      s1m = w.p[PK1][qd] + qk;
+      s2m = w.p[PK2][qd] - qk;
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int k = kb + u;
+      if (k <= ke) {
+        const int q = w.at(k, j, i);
+        const float qk = w.p[QK][q];
+        rs1[u] = w.p[PK1][q] + qk;
+        rs2[u] = w.p[PK2][q] - qk;
+        rmm[u] = w.p[MM][q];
+        rpp[u] = pp[q];
+        wt[u] = w.p[WTEN][q];
+        wo[u] = ws[q];
+        rar[u] = w.p[ARW][q];
+        rf[u] = column_fpk(w, n, k, j, i, nullptr);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int k = kb + u;
+      if (k <= ke) {
+        const float s1d = u ? rs1[u - 1] : s1m, s2d = u ? rs2[u - 1] : s2m;
+        Laa[at(k)] = k >= 3 ? (-c.asq) * (rmm[u] * s1d) : 0.0f;
+        Lcc[at(k)] = k < nk ? (-c.asq) * ((-rmm[u]) * rs2[u]) : 0.0f;
+        const float diag = (-rs1[u]) + s2d;
+        Lbb[at(k)] = 1.0f - c.asq * (rmm[u] * diag);
+        if (k == ke) {
+          Lbf[slot * CW + lane] = rf[u];
+          Lbp[slot * CW + lane] = rpp[u];
+        }
+      }
+    }
+  }
+  __syncthreads();
+  if (mine) {
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int k = kb + u;
+      if (k >= 2 && k <= ke) {
+        const float ppd = u ? rpp[u - 1] : Lbp[(slot - 1) * CW + lane], fd = u ? rf[u - 1] : Lbf[(slot - 1) * CW + lane];
+        const float pdelta = rpp[u] - ppd;
+        const float fwk = c.dts * wt[u] + c.beta * ((-rmm[u]) * pdelta);
+        const float udelta = (rpp[u] + rf[u]) - (ppd + fd);
+        Ldd[at(k)] = (wo[u] + fwk) + c.alph * ((-rmm[u]) * udelta);
+      }
+    }
+  }
+  __syncthreads();
+  if (col && slot == 0) {
+    float ec = 0.0f, ed = 0.0f;
+    float an = Laa[at(2)], bn = Lbb[at(2)], cn = Lcc[at(2)], dn = Ldd[at(2)];
+    for (int k = 2; k <= nk; ++k) {
+      const float a = an, b = bn, cc = cn, d = dn;
+      if (k < nk) {
+        an = Laa[at(k + 1)];
+        bn = Lbb[at(k + 1)];
+        cn = Lcc[at(k + 1)];
+        dn = Ldd[at(k + 1)];
+      }
+      const float pivot = k == 2 ? b : a * ec + b;
+      const float inv = 1.0f / pivot;
+      ed = (k == 2 ? d : d - a * ed) * inv;
+      Ldd[at(k)] = ed;
+      if (k < nk) {
+        ec = (-cc) * inv;
+        Lcc[at(k)] = ec;
+      }
+    }
+    float x = ed;
+    for (int k = nk - 1; k >= 2; --k) {
+      x = Lcc[at(k)] * x + Ldd[at(k)];
+      Ldd[at(k)] = x;
+    }
+  }
+  __syncthreads();
+  if (!mine) return;
+#pragma unroll
+  for (int u = 0; u < CH; ++u) {
+    const int k = kb + u;
+    if (k <= ke) {
+      const int q = w.at(k, j, i);
+      const float wk = k == 1 ? 0.0f : Ldd[at(k)], wu = k == nk ? 0.0f : Ldd[at(k + 1)];
+      const float vt = wk * rs1[u] + wu * rs2[u];
+      float up = (rpp[u] + rf[u]) + c.alph * vt;
+      up = fabsf(up) < 1.0e-20f ? 0.0f : up;
+      const float tend = c.kdiv * (up - rpp[u]);
+      wn[q] = wk;
+      w.snap(SPP, n)[q] = up;
+      w.snap(SPPD, n)[q] = up + tend;
+      if (w.nrk == 3 && last) w.p[PPXO][q] = tend;
+      w.p[ARW][q] = last ? (rar[u] + wk * c.alph) * c.tavg : rar[u] + wk;
+      if (k == nk) {
+        const int top = w.at(nk + 1, j, i);
+        wn[top] = ws[top];
+      }
+    }
+  }
 }
 
 // ------------------------------------------------------------------ post-acoustic and theta (forward)
@@ -748,7 +890,7 @@ __global__ __launch_bounds__(64) void k_post(W w) {
   CELL_INDEX
   const Consts& c = w.c;
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const int ie = w.X(i, 1), jn = w.Y(j, 1);
   const float *aru = w.p[ARU], *arv = w.p[ARV], *arw = w.p[ARW];
   // getdiv
@@ -806,7 +948,7 @@ __global__ __launch_bounds__(64) void k_theta(W w) {
   if (l == 1) az = (-fz(2)) * c.rdz;
   else if (l == nk) az = fz(nk) * c.rdz;
   else az = (fz(l) - fz(l + 1)) * c.rdz;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   float total = (ax + ay) + az;
   total = total + S(l, j, i) * w.p[DIVX2][q];
   const float adv = (total * w.col.rr0[l - 1]) * 1.0f;
@@ -816,7 +958,7 @@ __global__ __launch_bounds__(64) void k_theta(W w) {
 
 __global__ __launch_bounds__(64) void k_solve3(W w) {
   CELL_INDEX
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   w.p[PPXO][q] = w.snap(SPP, w.nloop)[q] + w.p[PPXO][q];
 }
 
@@ -841,7 +983,7 @@ __global__ __launch_bounds__(256) void k_b_fill(FillList f) {
 __global__ __launch_bounds__(64) void k_b_theta_cell(W w) {
   CELL_INDEX
   const Consts& c = w.c;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float thb = w.p[B_OTH][q];
   w.p[B_ATH][q] += thb;
   const float tdb = -c.dttmp * thb;
@@ -886,7 +1028,7 @@ __global__ __launch_bounds__(64) void k_b_theta_xy(W w, int dir) {
   const float rb = fb * m;
   for (int n = 0; n < 5; ++n) {
     const int o = o0 + step * n;
-    const int64_t t = dir == 0 ? w.at(l, j, w.X(i, o)) : w.at(l, w.Y(j, o), i);
+    const int t = dir == 0 ? w.at(l, j, w.X(i, o)) : w.at(l, w.Y(j, o), i);
     aadd(&w.p[B_SC][t], cf[n] * rb);
   }
 }
@@ -928,11 +1070,11 @@ __global__ __launch_bounds__(64) void k_b_post(W w) {
   if (l <= nk) {
     const float rho = w.col.rho[l - 1];
     const float den = 0.5f * (rho + rho);
-    const int64_t q = w.at(l, j, i), qw = w.at(l, j, w.X(i, -1)), qs = w.at(l, w.Y(j, -1), i);
+    const int q = w.at(l, j, i), qw = w.at(l, j, w.X(i, -1)), qs = w.at(l, w.Y(j, -1), i);
     w.p[B_ARU][q] = den * (w.p[B_MU][q] + c.rdx * (dx2[qw] - dx2[q])) + c.rdx * (db[qw] - db[q]);
     w.p[B_ARV][q] = den * (w.p[B_MV][q] + c.rdy * (dx2[qs] - dx2[q])) + c.rdy * (db[qs] - db[q]);
   }
-  const int64_t qw = w.at(l, j, i);
+  const int qw = w.at(l, j, i);
   if (l >= 2 && l <= nk) {
     const int64_t lo = w.at(l - 1, j, i);
     w.p[B_ARW][qw] = w.col.rf0[l - 1] * (w.p[B_MW][qw] + c.rdz * (dx2[lo] - dx2[qw])) + c.rdz * (db[lo] - db[qw]);
@@ -944,7 +1086,7 @@ __global__ __launch_bounds__(64) void k_b_post(W w) {
 // acoustic adjoint state from the stage-output adjoints (grid level l = 1..nk+1)
 __global__ __launch_bounds__(64) void k_b_ac_init(W w) {
   CELL_INDEX
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   w.p[B_W][q] = w.p[B_OW][q];
   if (l > w.nk) return;
   w.p[B_U][q] = w.p[B_OU][q];
@@ -963,11 +1105,11 @@ __global__ __launch_bounds__(64) void k_b_ssA(W w, int n) {
   const bool last = n == w.nloop;
   const bool last3 = last && w.nrk == 3;
   const float* wn = w.wsnap(n);
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   float dv;
   w.p[FPK][q] = column_fpk(w, n, l, j, i, &dv);
   w.p[DIV][q] = dv;
-  auto upb_at = [&](int64_t qq) {
+  auto upb_at = [&](int qq) {
     float u = w.p[B_PP][qq] + (1.0f + c.kdiv) * w.p[B_PPD][qq];
     if (last3) u = u + c.kdiv * w.p[B_PPX][qq];
     return u;
@@ -989,7 +1131,7 @@ __global__ __launch_bounds__(64) void k_b_ssA(W w, int n) {
   w.p[B_QK][q] += vtb * (wlo - whi);
   w.p[B_PK2][q] += vtb * whi;
   if (l >= 2) {
-    const int64_t qd = w.at(l - 1, j, i);
+    const int qd = w.at(l - 1, j, i);
     bw += vtb * (pk1[q] + qk[q]) + (c.alph * upb_at(qd)) * (pk2[qd] - qk[qd]);
   }
   w.p[B_W][q] = bw;
@@ -1023,7 +1165,7 @@ __global__ __launch_bounds__(64) void k_b_ssB(W w) {
     for (int u = 0; u < TH_CHUNK; ++u) {
       const int k = k0 + u;
       if (k > nk) break;
-      const int64_t q = w.at(k, j, i);
+      const int q = w.at(k, j, i);
       const float piv = dg[u] - lo[u] * cprev;
       const float cpk = up[u] / piv;
       const float dpk = (rh[u] - lo[u] * dprev) / piv;
@@ -1038,7 +1180,7 @@ __global__ __launch_bounds__(64) void k_b_ssB(W w) {
     float e[TH_CHUNK], f[TH_CHUNK];
 #pragma unroll
     for (int u = 0; u < TH_CHUNK; ++u) {
-      const int64_t q = w.at(k1 - u >= 2 ? k1 - u : 2, j, i);
+      const int q = w.at(k1 - u >= 2 ? k1 - u : 2, j, i);
       e[u] = bec[q];
       f[u] = bed[q];
     }
@@ -1058,7 +1200,7 @@ __global__ __launch_bounds__(64) void k_b_ssC(W w, int n) {
   CELL_INDEX
   const Consts& c = w.c;
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   if (l == nk + 1) return;  // the lid level's adjoint passes through (pk2(nk) = 0)
   const float* ws = w.wsnap(n - 1);
   const float* wn = w.wsnap(n);
@@ -1076,7 +1218,7 @@ __global__ __launch_bounds__(64) void k_b_ssC(W w, int n) {
   // bb's and aa's, cc's adjoints of row k
   auto diagb = [&](int k) {
     if (k < 2 || k > nk) return 0.0f;
-    const int64_t qq = w.at(k, j, i);
+    const int qq = w.at(k, j, i);
     return (-c.asq * mm[qq]) * (-LAM(k) * wn[qq]);
   };
   auto aab = [&](int k) { return (k >= 3 && k <= nk) ? -LAM(k) * wn[w.at(k - 1, j, i)] : 0.0f; };
@@ -1086,7 +1228,7 @@ __global__ __launch_bounds__(64) void k_b_ssC(W w, int n) {
   float bw = LAM(l);
   if (l >= 2) bw += c.beta * (f * pk1[q]) + qk[q] * (c.beta * f);
   if (l >= 2) {
-    const int64_t qd = w.at(l - 1, j, i);
+    const int qd = w.at(l - 1, j, i);
     const float fd = F(l - 1);
     bw += c.beta * (fd * pk2[qd]);
     if (l - 1 <= nk - 1) bw += -qk[qd] * (c.beta * fd);
@@ -1095,7 +1237,7 @@ __global__ __launch_bounds__(64) void k_b_ssC(W w, int n) {
   if (l >= 2) {
     const float lk = LAM(l);
     w.p[B_WTEN][q] += c.dts * lk;
-    const int64_t qd = w.at(l - 1, j, i);
+    const int qd = w.at(l - 1, j, i);
     const float pdelta = PP(l) - PP(l - 1);
     const float udelta = (PP(l) + FP(l)) - (PP(l - 1) + FP(l - 1));
     float mmb = (-(c.beta * pdelta + c.alph * udelta)) * lk;
@@ -1139,6 +1281,179 @@ __global__ __launch_bounds__(64) void k_b_ssC(W w, int n) {
   w.p[B_XA][q] = -(f * w.col.rr0[l - 1]);
 }
 
+// A, B and C in one pass (the staged columns above): the substep's fpk, the rows and their adjoints stay in
+// registers and LDS, the coefficients' accumulators are read and written once, and the first substep
+// reversed (n = nloop) starts them.
+template <int CH>
+__global__ __launch_bounds__(CW* CS) void k_b_ss_column(W w, int n) {
+  extern __shared__ float lds[];
+  const Consts& c = w.c;
+  const int nk = w.nk, lane = threadIdx.x % CW, slot = threadIdx.x / CW;
+  const int i = (int)blockIdx.x * CW + lane, j = blockIdx.y;
+  const int chunk = (nk + CS - 1) / CS, kb = 1 + slot * chunk, ke = min(nk, kb + chunk - 1);
+  const bool col = i < w.ni, mine = col && kb <= ke;
+  const bool last = n == w.nloop, last3 = last && w.nrk == 3;
+  const int L = (nk + 2) * CW;
+  float *Laa = lds, *Lbb = lds + L, *Lcc = lds + 2 * L, *Lr = lds + 3 * L;
+  float* Lbf = lds + 4 * L;  // fpk of each slot's last level
+  auto at = [&](int k) { return k * CW + lane; };
+  const float *ws = w.wsnap(n - 1), *wn = w.wsnap(n), *pp = w.snap(SPP, n - 1);
+  auto upb_at = [&](int q) {
+    float v = w.p[B_PP][q] + (1.0f + c.kdiv) * w.p[B_PPD][q];
+    if (last3) v = v + c.kdiv * w.p[B_PPX][q];
+    return v;
+  };
+  // own levels, and level kb-1 in element 0
+  float qk[CH + 1], pk1[CH + 1], pk2[CH + 1], mm[CH + 1], upb[CH + 1], rpp[CH + 1], rf[CH + 1], rwn[CH + 1];
+  float div[CH], rws[CH];
+  if (mine) {
+    {
+      const int q = w.at(max(kb - 1, 1), j, i);
+      qk[0] = w.p[QK][q];
+      pk1[0] = w.p[PK1][q];
+      pk2[0] = w.p[PK2][q];
+      mm[0] = w.p[MM][q];
+      rpp[0] = pp[q];
+      rwn[0] = wn[q];
+      upb[0] = upb_at(q);
+      rf[0] = 0.0f;
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int k = kb + u;
+      if (k <= ke) {
+        const int q = w.at(k, j, i);
+        qk[u + 1] = w.p[QK][q];
+        pk1[u + 1] = w.p[PK1][q];
+        pk2[u + 1] = w.p[PK2][q];
+        mm[u + 1] = w.p[MM][q];
+        rpp[u + 1] = pp[q];
+        rwn[u + 1] = wn[q];
+        rws[u] = ws[q];
+        upb[u + 1] = upb_at(q);
+        rf[u + 1] = column_fpk(w, n, k, j, i, &div[u]);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int k = kb + u;
+      if (k <= ke) {
+        const int q = w.at(k, j, i);
+        const float s1 = pk1[u + 1] + qk[u + 1], s2 = pk2[u + 1] - qk[u + 1];
+        const float s1d = pk1[u] + qk[u], s2d = pk2[u] - qk[u];
+        Laa[at(k)] = k >= 3 ? (-c.asq) * (mm[u + 1] * s1d) : 0.0f;
+        Lcc[at(k)] = k >= 2 && k < nk ? (-c.asq) * ((-mm[u + 1]) * s2) : 0.0f;
+        const float diag = (-s1) + s2d;
+        Lbb[at(k)] = 1.0f - c.asq * (mm[u + 1] * diag);
+        const float barw = w.p[B_ARW][q];
+        float bw = w.p[B_W][q];
+        if (last) {
+          bw += (barw * c.tavg) * c.alph;
+          w.p[B_ARW][q] = barw * c.tavg;
+        } else {
+          bw += barw;
+        }
+        if (k >= 2) bw += (c.alph * upb[u + 1]) * s1 + (c.alph * upb[u]) * s2d;
+        Lr[at(k)] = bw;
+        if (k == ke) Lbf[slot * CW + lane] = rf[u + 1];
+      }
+    }
+  }
+  __syncthreads();
+  if (col && slot == 0) {  // T^T lam = wbar(2..nk): row k has cc(k-1) below and aa(k+1) above its diagonal
+    float cp = 0.0f, dp = 0.0f, lo = 0.0f;
+    float un = nk > 2 ? Laa[at(3)] : 0.0f, gn = Lbb[at(2)], rn = Lr[at(2)], cn = Lcc[at(2)];
+    for (int k = 2; k <= nk; ++k) {
+      const float up = un, dg = gn, rh = rn, cc = cn;
+      if (k < nk) {
+        un = k + 2 <= nk ? Laa[at(k + 2)] : 0.0f;
+        gn = Lbb[at(k + 1)];
+        rn = Lr[at(k + 1)];
+        cn = Lcc[at(k + 1)];
+      }
+      const float piv = dg - lo * cp;
+      cp = up / piv;
+      dp = (rh - lo * dp) / piv;
+      Lbb[at(k)] = cp;
+      Lr[at(k)] = dp;
+      lo = cc;
+    }
+    float x = dp;
+    for (int k = nk - 1; k >= 2; --k) {
+      x = Lr[at(k)] - Lbb[at(k)] * x;
+      Lr[at(k)] = x;
+    }
+  }
+  __syncthreads();
+  if (!mine) return;
+  if (kb > 1) rf[0] = Lbf[(slot - 1) * CW + lane];
+  // the words of level ke+1 that its row's adjoints need
+  const int qt = w.at(min(ke + 1, nk), j, i);
+  const float mmt = w.p[MM][qt], wnt = wn[qt], wst = ws[w.at(ke + 1, j, i)];
+  auto LAM = [&](int k) { return (k >= 2 && k <= nk) ? Lr[at(k)] : 0.0f; };
+#pragma unroll
+  for (int u = 0; u < CH; ++u) {
+    const int k = kb + u;
+    if (k <= ke) {
+      const int q = w.at(k, j, i);
+      const float mk = mm[u + 1], wk = rwn[u + 1], md = mm[u], wd = rwn[u];
+      const bool top = k == ke;
+      const float mu = top ? mmt : mm[u + 2 <= CH ? u + 2 : CH], wu = top ? wnt : rwn[u + 2 <= CH ? u + 2 : CH];
+      const float wsu = top ? wst : rws[u + 1 < CH ? u + 1 : CH - 1];
+      const float ld = LAM(k - 1), lk = LAM(k), lu = LAM(k + 1);
+      const float udk = c.alph * (-mk) * lk, udu = c.alph * (-mu) * lu, udd = c.alph * (-md) * ld;
+      const float pdk = c.beta * (-mk) * lk, pdu = c.beta * (-mu) * lu;
+      const float f = upb[u + 1] + udk - udu;
+      const float fd = upb[u] + udd - udk;
+      const float diagk = k >= 2 ? (-c.asq * mk) * (-lk * wk) : 0.0f;
+      const float diagu = k < nk ? (-c.asq * mu) * (-lu * wu) : 0.0f;
+      const float aak = k >= 3 ? -lk * wd : 0.0f, aau = (k < nk && k >= 2) ? -lu * wk : 0.0f;
+      const float cck = (k >= 2 && k < nk) ? -lk * wu : 0.0f;
+      float bw = lk;
+      if (k >= 2) {
+        bw += c.beta * (f * pk1[u + 1]) + qk[u + 1] * (c.beta * f);
+        bw += c.beta * (fd * pk2[u]);
+        bw += -qk[u] * (c.beta * fd);
+        w.p[B_WTEN][q] = (last ? 0.0f : w.p[B_WTEN][q]) + c.dts * lk;
+        const float pdelta = rpp[u + 1] - rpp[u];
+        const float udelta = (rpp[u + 1] + rf[u + 1]) - (rpp[u] + rf[u]);
+        float mmb = (-(c.beta * pdelta + c.alph * udelta)) * lk;
+        const float diag = (-(pk1[u + 1] + qk[u + 1])) + (pk2[u] - qk[u]);
+        mmb += (-c.asq * diag) * (-lk * wk);
+        mmb += (-c.asq) * (pk1[u] + qk[u]) * aak;
+        mmb += c.asq * (pk2[u + 1] - qk[u + 1]) * cck;
+        w.p[B_MM][q] = (last ? 0.0f : w.p[B_MM][q]) + mmb;
+      }
+      w.p[B_W][q] = k == 1 ? 0.0f : bw;
+      {
+        float ppb = -c.kdiv * w.p[B_PPD][q];
+        if (last3) {
+          ppb = ppb - c.kdiv * w.p[B_PPX][q];
+          w.p[B_PPX][q] = 0.0f;
+        }
+        w.p[B_PP][q] = (ppb + upb[u + 1]) + ((pdk + udk) - (pdu + udu));
+      }
+      const float vtb = c.alph * upb[u + 1];
+      const float wnlo = k == 1 ? 0.0f : wk, wnhi = k == nk ? 0.0f : wu;
+      const float wlo = k == 1 ? 0.0f : rws[u], whi = k == nk ? 0.0f : wsu;
+      float bpk1 = -diagk + f * (c.beta * wlo);
+      float bqk = -diagk - diagu - (c.beta * f) * (whi - wlo);
+      float bpk2 = diagu + f * (c.beta * wsu);
+      const float ma = (-c.asq) * mu * aau, mc = c.asq * mk * cck;
+      bpk1 += ma;
+      bqk += ma;
+      bpk2 += mc;
+      bqk -= mc;
+      w.p[B_PK1][q] = ((last ? 0.0f : w.p[B_PK1][q]) + vtb * wnlo) + bpk1;
+      w.p[B_QK][q] = ((last ? 0.0f : w.p[B_QK][q]) + vtb * (wnlo - wnhi)) + bqk;
+      w.p[B_PK2][q] = ((last ? 0.0f : w.p[B_PK2][q]) + vtb * wnhi) + bpk2;
+      w.p[B_PPTERM][q] = (last ? 0.0f : w.p[B_PPTERM][q]) - c.dts * (div[u] * f);
+      w.p[B_DIV][q] = -c.dts * (w.p[PPTERM][q] * f);
+      w.p[B_XA][q] = -(f * w.col.rr0[k - 1]);
+    }
+  }
+}
+
 // u and v faces of substep n: averages, pressure advection and divergence adjoints, forcing
 __global__ __launch_bounds__(64) void k_b_ss_faces(W w, int n) {
   CELL_INDEX
@@ -1147,9 +1462,9 @@ __global__ __launch_bounds__(64) void k_b_ss_faces(W w, int n) {
   const float* pia = w.p[PIADV];
   const float *xa = w.p[B_XA], *db = w.p[B_DIV];
   const float rho = w.col.rho[l - 1];
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   {
-    const int64_t qw = w.at(l, j, w.X(i, -1));
+    const int qw = w.at(l, j, w.X(i, -1));
     float ub = w.p[B_U][q];
     if (last) {
       ub += w.p[B_ARU][q] * c.tavg;
@@ -1165,7 +1480,7 @@ __global__ __launch_bounds__(64) void k_b_ss_faces(W w, int n) {
     w.p[B_U][q] = ub;
   }
   {
-    const int64_t qs = w.at(l, w.Y(j, -1), i);
+    const int qs = w.at(l, w.Y(j, -1), i);
     float vb = w.p[B_V][q];
     if (last) {
       vb += w.p[B_ARV][q] * c.tavg;
@@ -1192,9 +1507,9 @@ __global__ __launch_bounds__(64) void k_b_ss_cells(W w, int n) {
   const float* v1 = w.snap(SV, n);
   const float *bu = w.p[B_U], *bv = w.p[B_V], *xa = w.p[B_XA];
   const float rho = w.col.rho[l - 1];
-  const int64_t q = w.at(l, j, i);
-  const int64_t qe = w.at(l, j, w.X(i, 1)), qw = w.at(l, j, w.X(i, -1));
-  const int64_t qn = w.at(l, w.Y(j, 1), i), qs = w.at(l, w.Y(j, -1), i);
+  const int q = w.at(l, j, i);
+  const int qe = w.at(l, j, w.X(i, 1)), qw = w.at(l, j, w.X(i, -1));
+  const int qn = w.at(l, w.Y(j, 1), i), qs = w.at(l, w.Y(j, -1), i);
   // u faces i (cell i is the right cell) and i+1 (left cell)
   const float pgx0 = -c.dts * bu[q], pgx1 = -c.dts * bu[qe];
   const float A0 = c.halfcp * (thv[q] + thv[qw]), A1 = c.halfcp * (thv[qe] + thv[q]);
@@ -1207,10 +1522,10 @@ __global__ __launch_bounds__(64) void k_b_ss_cells(W w, int n) {
   tb += c.halfcp * (pgy0 * By0) + c.halfcp * (pgy1 * By1);
   w.p[B_THV][q] += tb;
   // pressure advection: t2(c) = xa(c)*temx*rho*u1(c+1), t1(c) = xa(c)*temx*rho*u1(c)
-  auto t2x = [&](int64_t cell, int64_t east) { return xa[cell] * (c.temx * (rho * u1[east])); };
-  auto t1x = [&](int64_t cell) { return xa[cell] * (c.temx * (rho * u1[cell])); };
-  auto t2y = [&](int64_t cell, int64_t north) { return xa[cell] * (c.temy * (rho * v1[north])); };
-  auto t1y = [&](int64_t cell) { return xa[cell] * (c.temy * (rho * v1[cell])); };
+  auto t2x = [&](int cell, int east) { return xa[cell] * (c.temx * (rho * u1[east])); };
+  auto t1x = [&](int cell) { return xa[cell] * (c.temx * (rho * u1[cell])); };
+  auto t2y = [&](int cell, int north) { return xa[cell] * (c.temy * (rho * v1[north])); };
+  auto t1y = [&](int cell) { return xa[cell] * (c.temy * (rho * v1[cell])); };
   float pb = (t2x(qw, q) - t2x(q, qe)) + (t1x(q) - t1x(qe));
   pb += (t2y(qs, q) - t2y(q, qn)) + (t1y(q) - t1y(qn));
   w.p[B_PIADV][q] += pb;
@@ -1221,7 +1536,7 @@ __global__ __launch_bounds__(64) void k_b_coef(W w) {
   CELL_INDEX
   const Consts& c = w.c;
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   auto tem2 = [&](int k) { return ((c.dts * 1.0f) * w.col.rdsf[k]) * w.col.rr0[k - 1]; };
   auto b2b = [&](int k) { return (tem2(k) * w.col.rf0[k]) * w.p[B_PK2][w.at(k, j, i)]; };      // k < nk
   auto b1b = [&](int k) { return (tem2(k) * w.col.rf0[k - 1]) * w.p[B_PK1][w.at(k, j, i)]; };  // k > 1
@@ -1243,7 +1558,7 @@ __global__ __launch_bounds__(64) void k_b_coef(W w) {
 __global__ __launch_bounds__(64) void k_b_ac_end(W w) {
   CELL_INDEX
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   if (l <= nk) {
     w.p[B_PPX][q] = w.p[B_PPD][q] + w.p[B_PPX][q];
     w.p[B_AW][q] += w.c.beta * w.p[B_ARW][q];
@@ -1277,10 +1592,10 @@ __global__ __launch_bounds__(64) void k_b_adv_local(W w) {
     return btv[qq] * (1.0f / (0.5f * (rho + rho)));
   };
   auto totw = [&](int kf, int64_t qq) { return btw[qq] * (w.col.rrf0[kf - 1] * 1.0f); };
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   if (l <= nk) {
-    const int64_t qw = w.at(l, j, w.X(i, -1)), qe = w.at(l, j, w.X(i, 1));
-    const int64_t qs = w.at(l, w.Y(j, -1), i), qn = w.at(l, w.Y(j, 1), i);
+    const int qw = w.at(l, j, w.X(i, -1)), qe = w.at(l, j, w.X(i, 1));
+    const int qs = w.at(l, w.Y(j, -1), i), qn = w.at(l, w.Y(j, 1), i);
     const float tu = totu(q, l), tv = totv(q, l);
     w.p[B_XU][q] += tu * (0.5f * (dx[q] + dx[qw]));
     w.p[B_XV][q] += tv * (0.5f * (dx[q] + dx[qs]));
@@ -1291,7 +1606,7 @@ __global__ __launch_bounds__(64) void k_b_adv_local(W w) {
     g += 0.5f * (tv * v[q]) + 0.5f * (totv(qn, l) * v[qn]);
     if (l >= 2) g += w.col.c2[l - 1] * (totw(l, q) * ww[q]);
     if (l + 1 <= nk) {
-      const int64_t qu = w.at(l + 1, j, i);
+      const int qu = w.at(l + 1, j, i);
       g += (1.0f - w.col.c2[l]) * (totw(l + 1, qu) * ww[qu]);
     }
     w.p[B_DIVX][q] += g;
@@ -1314,7 +1629,7 @@ __global__ __launch_bounds__(64) void k_b_advh_flux(W w, int comp) {
   CELL_INDEX
   const Consts& c = w.c;
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float *ru = w.p[RRU], *rv = w.p[RRV];
   float *g0 = w.p[G0], *g1 = w.p[G1], *g2 = w.p[G2], *g3 = w.p[G3], *g4 = w.p[G4], *g5 = w.p[G5];
   if (comp == 2 && (l < 2 || l > nk)) {
@@ -1374,7 +1689,7 @@ __global__ __launch_bounds__(64) void k_b_advh_flux(W w, int comp) {
 __global__ __launch_bounds__(64) void k_b_advh_gather(W w, int comp) {
   CELL_INDEX
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float *g0 = w.p[G0], *g1 = w.p[G1], *g2 = w.p[G2], *g3 = w.p[G3], *g4 = w.p[G4], *g5 = w.p[G5];
   const float cf[5] = {gm1::C2_60, gm1::CM13_60, gm1::C47_60, gm1::C27_60, gm1::CM3_60};
   auto at = [&](int ll, int jj, int ii) { return w.at(ll, w.Y(jj, 0), w.X(ii, 0)); };
@@ -1410,7 +1725,7 @@ __global__ __launch_bounds__(64) void k_b_advh_gather(W w, int comp) {
     }
     if (l + 1 <= nk) {
       const float c2h = 0.5f * (w.col.c2[l] + w.col.c2[l]);
-      const int64_t qu = w.at(l + 1, j, i);
+      const int qu = w.at(l + 1, j, i);
       gu += (1.0f - c2h) * g2[qu];
       gv += (1.0f - c2h) * g5[qu];
     }
@@ -1425,7 +1740,7 @@ __global__ __launch_bounds__(64) void k_b_advz_flux(W w, int comp) {
   CELL_INDEX
   const Consts& c = w.c;
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   float *g0 = w.p[G0], *g1 = w.p[G1], *g2 = w.p[G2];
   const float* rw = w.p[RRW];
   const bool live = comp == 2 ? (l <= nk) : (l >= 2 && l <= nk);
@@ -1444,7 +1759,7 @@ __global__ __launch_bounds__(64) void k_b_advz_flux(W w, int comp) {
     };
     const int kf = l;
     fb = c.rdz * tot(kf) - c.rdz * tot(kf - 1);
-    const int64_t qo = comp == 0 ? w.at(kf, j, w.X(i, -1)) : w.at(kf, w.Y(j, -1), i);
+    const int qo = comp == 0 ? w.at(kf, j, w.X(i, -1)) : w.at(kf, w.Y(j, -1), i);
     m = 0.5f * (rw[q] + rw[qo]);
     const float c2h = 0.5f * (w.col.c2[kf - 1] + w.col.c2[kf - 1]);
     Stencil ps, ng;
@@ -1472,7 +1787,7 @@ __global__ __launch_bounds__(64) void k_b_advz_flux(W w, int comp) {
 __global__ __launch_bounds__(64) void k_b_advz_gather(W w, int comp) {
   CELL_INDEX
   const int nk = w.nk;
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   const float *g0 = w.p[G0], *g1 = w.p[G1], *g2 = w.p[G2];
   auto Q0 = [&](int) { return 0.0f; };
   float acc = 0.0f;
@@ -1484,7 +1799,7 @@ __global__ __launch_bounds__(64) void k_b_advz_gather(W w, int comp) {
 #pragma unroll
     for (int d = -2; d <= 2; ++d) acc += cf5[2 + d] * g1[w.at(l + d, j, i)];
     (comp == 0 ? w.p[B_XU] : w.p[B_XV])[q] += acc;
-    const int64_t qn = comp == 0 ? w.at(l, j, w.X(i, 1)) : w.at(l, w.Y(j, 1), i);
+    const int qn = comp == 0 ? w.at(l, j, w.X(i, 1)) : w.at(l, w.Y(j, 1), i);
     w.p[B_RRW][q] += 0.5f * g2[q] + 0.5f * g2[qn];
     return;
   }
@@ -1506,7 +1821,7 @@ __global__ __launch_bounds__(64) void k_b_advz_gather(W w, int comp) {
         Stencil ps, ng;
         uvz_branch(kf, nk, ps, ng);
         float cf[5];
-        const int64_t qf = w.at(kf, j, i);
+        const int qf = w.at(kf, j, i);
         int nc = branch_coefs(ps, Q0, c2h, 1.0f - c2h, 0.0f, cf);
         for (int n = 0; n < nc; ++n)
           if (ps.lev[n] == l) acc += cf[n] * g0[qf];
@@ -1518,7 +1833,7 @@ __global__ __launch_bounds__(64) void k_b_advz_gather(W w, int comp) {
     }
     // rrw at w level l (2..nk) from the fluxes at this point and its +x / +y neighbour
     if (l >= 2 && l <= nk) {
-      const int64_t qn = comp == 0 ? w.at(l, j, w.X(i, 1)) : w.at(l, w.Y(j, 1), i);
+      const int qn = comp == 0 ? w.at(l, j, w.X(i, 1)) : w.at(l, w.Y(j, 1), i);
       w.p[B_RRW][q] += 0.5f * g2[q] + 0.5f * g2[qn];
     }
   } else {
@@ -1527,7 +1842,7 @@ __global__ __launch_bounds__(64) void k_b_advz_gather(W w, int comp) {
       Stencil ps, ng;
       wz_branch(k, nk, ps, ng);
       float cf[5];
-      const int64_t qf = w.at(k, j, i);
+      const int qf = w.at(k, j, i);
       int nc = branch_coefs(ps, Q0, 0.0f, 0.0f, 0.0f, cf);
       for (int n = 0; n < nc; ++n)
         if (ps.lev[n] == l) acc += cf[n] * g0[qf];
@@ -1549,11 +1864,11 @@ __global__ __launch_bounds__(64) void k_b_mass_terms(W w) {
   const Consts& c = w.c;
   const int nk = w.nk;
   const float* dxb = w.p[B_DIVX];
-  const int64_t q = w.at(l, j, i);
+  const int q = w.at(l, j, i);
   if (l <= nk) {
     const float rho = w.col.rho[l - 1];
     const float den = 0.5f * (rho + rho);
-    const int64_t qw = w.at(l, j, w.X(i, -1)), qs = w.at(l, w.Y(j, -1), i);
+    const int qw = w.at(l, j, w.X(i, -1)), qs = w.at(l, w.Y(j, -1), i);
     w.p[B_XU][q] += den * (w.p[B_RRU][q] + (dxb[qw] * c.rdx - dxb[q] * c.rdx));
     w.p[B_XV][q] += den * (w.p[B_RRV][q] + (dxb[qs] * c.rdy - dxb[q] * c.rdy));
     w.p[B_XTH][q] += ((w.p[B_THV][q] * 1.0f + w.p[B_DUM8][q] * (c.g * w.col.rth[l - 1])) +
@@ -1561,7 +1876,7 @@ __global__ __launch_bounds__(64) void k_b_mass_terms(W w) {
     w.p[B_XPP][q] += w.p[B_PPTERM][q] * ((c.rovcp * c.cpm) * c.cvm) + w.p[B_PIADV][q];
   }
   if (l >= 2 && l <= nk) {
-    const int64_t qd = w.at(l - 1, j, i);
+    const int qd = w.at(l - 1, j, i);
     w.p[B_XW][q] += w.col.rf0[l - 1] * (w.p[B_RRW][q] + (dxb[qd] * c.rdz - dxb[q] * c.rdz));
   }
 }
@@ -1590,6 +1905,7 @@ int gm1hip_dry_stage_forward(void* const* table, const float* consts, int ni, in
                              double weps, void* stream) {
   if (!table || !consts || ni < 6 || nj < 6 || nk < 6 || nrk < 1 || nrk > 3 || nloop < 1)
     return (int)hipErrorInvalidValue;
+  if ((int64_t)ni * nj * (nk + 1) >= ((int64_t)1 << 31)) return (int)hipErrorInvalidValue;
   hipStream_t s = (hipStream_t)stream;
   const W w = make_w(table, consts, ni, nj, nk, nrk, nloop, weps);
   const dim3 b(64), g((ni + 63) / 64, nj, nk), gw((ni + 63) / 64, nj, nk + 1), gc((ni + 63) / 64, nj);
@@ -1600,11 +1916,19 @@ int gm1hip_dry_stage_forward(void* const* table, const float* consts, int ni, in
   hipLaunchKernelGGL(k_advv, g, b, 0, s, w);
   hipLaunchKernelGGL(k_advw, gw, b, 0, s, w);
   hipLaunchKernelGGL(k_coef, g, b, 0, s, w);
-  hipLaunchKernelGGL(k_rows, g, b, 0, s, w);
+  const bool staged = nk <= MAX_STAGED_NK;  // (a taller column takes the passes of one thread a cell)
+  const dim3 gs((ni + CW - 1) / CW, nj);
+  const int lds = staged_lds_bytes(nk);
+  if (!staged) hipLaunchKernelGGL(k_rows, g, b, 0, s, w);
   hipLaunchKernelGGL(k_ac_start, g, b, 0, s, w);
   GM1_LAUNCH_CHECK();
   for (int n = 1; n <= nloop; ++n) {
     hipLaunchKernelGGL(k_ss_pgrad, g, b, 0, s, w, n);
+    if (staged) {
+      if (nk <= 4 * CS) hipLaunchKernelGGL(k_ss_column<4>, gs, dim3(CW * CS), lds, s, w, n);
+      else hipLaunchKernelGGL(k_ss_column<8>, gs, dim3(CW * CS), lds, s, w, n);
+      continue;
+    }
     hipLaunchKernelGGL(k_ss_fpk, g, b, 0, s, w, n);
     hipLaunchKernelGGL(k_ss_rhs, g, b, 0, s, w, n);
     hipLaunchKernelGGL(k_ss_thomas, gc, b, 0, s, w, n);
@@ -1621,6 +1945,7 @@ int gm1hip_dry_stage_adjoint(void* const* table, const float* consts, int ni, in
                              double weps, void* stream) {
   if (!table || !consts || ni < 6 || nj < 6 || nk < 6 || nrk < 1 || nrk > 3 || nloop < 1)
     return (int)hipErrorInvalidValue;
+  if ((int64_t)ni * nj * (nk + 1) >= ((int64_t)1 << 31)) return (int)hipErrorInvalidValue;
   hipStream_t s = (hipStream_t)stream;
   const W w = make_w(table, consts, ni, nj, nk, nrk, nloop, weps);
   const int64_t cells = (int64_t)ni * nj * nk, wcells = (int64_t)ni * nj * (nk + 1);
@@ -1650,10 +1975,18 @@ int gm1hip_dry_stage_adjoint(void* const* table, const float* consts, int ni, in
   // acoustic stage
   hipLaunchKernelGGL(k_b_ac_init, gw, b, 0, s, w);
   GM1_LAUNCH_CHECK();
+  const bool staged = nk <= MAX_STAGED_NK;
+  const dim3 gs((ni + CW - 1) / CW, nj);
+  const int lds = staged_lds_bytes(nk);
   for (int n = nloop; n >= 1; --n) {
-    hipLaunchKernelGGL(k_b_ssA, g, b, 0, s, w, n);
-    hipLaunchKernelGGL(k_b_ssB, gc, b, 0, s, w);
-    hipLaunchKernelGGL(k_b_ssC, g, b, 0, s, w, n);
+    if (staged) {
+      if (nk <= 4 * CS) hipLaunchKernelGGL(k_b_ss_column<4>, gs, dim3(CW * CS), lds, s, w, n);
+      else hipLaunchKernelGGL(k_b_ss_column<8>, gs, dim3(CW * CS), lds, s, w, n);
+    } else {
+      hipLaunchKernelGGL(k_b_ssA, g, b, 0, s, w, n);
+      hipLaunchKernelGGL(k_b_ssB, gc, b, 0, s, w);
+      hipLaunchKernelGGL(k_b_ssC, g, b, 0, s, w, n);
+    }
     hipLaunchKernelGGL(k_b_ss_faces, g, b, 0, s, w, n);
     hipLaunchKernelGGL(k_b_ss_cells, g, b, 0, s, w, n);
   }
