@@ -2,7 +2,7 @@
 //
 // Replaces the kernel family of cuda_advection5.py (terrain mass flux,
 // divergence, scalar face fluxes and tendency).  Design:
-//   * one fused tendency kernel per scalar: a 64x4 (i,j) tile marches up its
+//   * one fused tendency kernel per scalar: a 64x8 (i,j) tile marches up its
 //     column chunk; x- and y-face fluxes of each level are formed once into
 //     LDS and shared by the two cells on either side, the z-face flux is
 //     carried in a register from one level to the next.  Face fluxes never
@@ -135,9 +135,10 @@ __device__ __forceinline__ float zflux_g(Get S, float m, float cc1, float cc2, i
   } else if (k == nk - 1) {
     if (m >= 0.0f) r = recon5(S(k - 3), S(k - 2), S(k - 1), S(k), S(k + 1), WENO, weps);
     else r = WENO ? upstrpd(S(k + 1), S(k), S(k - 1), wf) : flx3(S(k + 1), S(k), S(k - 1));
-  } else {
-    if (m >= 0.0f) r = recon5(S(k - 3), S(k - 2), S(k - 1), S(k), S(k + 1), WENO, weps);
-    else r = recon5(S(k + 2), S(k + 1), S(k), S(k - 1), S(k - 2), WENO, weps);
+  } else {  // one reconstruction of the upwind words, whichever way the lanes' fluxes point
+    const bool up = m >= 0.0f;
+    const float q0 = S(k - 3), q1 = S(k - 2), q2 = S(k - 1), q3 = S(k), q4 = S(k + 1), q5 = S(k + 2);
+    r = recon5(up ? q0 : q5, up ? q1 : q4, up ? q2 : q3, up ? q3 : q2, up ? q4 : q1, WENO, weps);
   }
   return m * r;
 }
@@ -159,9 +160,9 @@ __device__ __forceinline__ float zflux_pdef_g(Get S, float m, float cc1, float c
     if (low) {
       r = (k == 3) ? upstrpd(S(k - 2), S(k - 1), S(k), wf) : upstrpd(S(k + 1), S(k), S(k - 1), wf);
     } else {
-      float s1, s2, s3, s4, s5;
-      if (m >= 0.0f) { s1 = S(k - 3); s2 = S(k - 2); s3 = S(k - 1); s4 = S(k); s5 = S(k + 1); }
-      else { s1 = S(k + 2); s2 = S(k + 1); s3 = S(k); s4 = S(k - 1); s5 = S(k - 2); }
+      const bool up = m >= 0.0f;
+      const float q0 = S(k - 3), q1 = S(k - 2), q2 = S(k - 1), q3 = S(k), q4 = S(k + 1), q5 = S(k + 2);
+      const float s1 = up ? q0 : q5, s2 = up ? q1 : q4, s3 = up ? q2 : q3, s4 = up ? q3 : q2, s5 = up ? q4 : q1;
       if (pdefweno && !((double)max5(s1, s2, s3, s4, s5) > weps)) return 0.0f;
       r = weno5(s1, s2, s3, s4, s5, weps);
     }
@@ -256,12 +257,12 @@ template <bool WENO, int MODE, bool FLAT, bool SRC>
 __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
   constexpr bool GATE = (MODE == MODE_PDEF);
   constexpr int PS = ((TY + 6) * LQ + NT - 1) / NT;
-  __shared__ float lfx[TY][TX + 1];
-  __shared__ float lfy[TY + 1][TX];
-  __shared__ float lp[PS * NT];       // the level plane, TY+6 rows of LQ (slots past them unread)
+  __shared__ float lfx2[2][TY][TX + 1];  // (the fluxes and the plane each in two buffers, levels taking turns)
+  __shared__ float lfy2[2][TY + 1][TX];
+  __shared__ float lp2[2][PS * NT];   // the level plane, TY+6 rows of LQ (slots past them unread)
   __shared__ uint32_t lpo[PS * NT];   // each plane slot's byte offset within a level
   const int ni = a.ni, nj = a.nj, nk = a.nk;
-  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+  const int tx = threadIdx.x % TX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / TX);  // (a wavefront is one row)
   // tiles ordered i fastest, then j, then column chunk; each XCD sweeps a
   // contiguous range so the y-halo rows a tile shares stay in one L2
   const int gxt = (ni + TX - 1) / TX, gyt = (nj + TY - 1) / TY;
@@ -279,11 +280,11 @@ __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
   const int x = i + NG, y = j + NG;
   const int64_t st = (int64_t)nys * nxs, ust = (int64_t)nys * nxu, vst = (int64_t)nyv * nxs;
   const int64_t mst = (int64_t)nj * ni;
-  const uint32_t o_s = (uint32_t)(y * nxs + x) * 4u;  // padded scalar, w and v (south face) families
+  const uint32_t o_s = live ? (uint32_t)(y * nxs + x) * 4u : 0u;  // padded scalar, w and v (south face) families
   const uint32_t o_u = (uint32_t)(y * nxu + x) * 4u;  // u family (west face)
-  const uint32_t o_m = (uint32_t)(j * ni + i) * 4u;   // unpadded cells
+  const uint32_t o_m = live ? (uint32_t)(j * ni + i) * 4u : 0u;   // unpadded cells
   const uint32_t o_fu = (i <= ni && j < nj) ? o_u : 0u;  // the own west x face
-  const uint32_t o_fv = (i < ni && j <= nj) ? o_s : 0u;  // the own south y face
+  const uint32_t o_fv = (i < ni && j <= nj) ? (uint32_t)(y * nxs + x) * 4u : 0u;  // the own south y face
   const bool xe = (ty == TY - 1), yn = (ty == TY - 2);   // the wavefronts forming the east / north faces
   uint32_t o_ex = 0u;
   if (xe && tx < TY && i0 + TX <= ni && j0 + tx < nj) o_ex = (uint32_t)((j0 + tx + NG) * nxu + i0 + TX + NG) * 4u;
@@ -312,86 +313,103 @@ __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
   // holds level k-3+q (0 outside the padded column; those words are never
   // read by a face's stencil, which stays within levels 1..nk).
   float win[7];
-  auto colword = [&](int lev) {  // the column's word at a level, 0 where no stencil reads
+  // The column's word at a level, as loaded (levels clipped to the column) and as the
+  // window holds it: the two are apart so that no load is waited for where it is issued.
+  auto colload = [&](int lev) {
+    // (from an unpadded carrier the own column is a physical cell, which needs no lateral image)
+    if constexpr (SRC) return ldo(a.src + (int64_t)(min(max(lev, 1), nk) - 1) * mst, o_m);
+    return ldo(a.s + (int64_t)min(max(lev, 0), nk + 1) * st, o_s);
+  };
+  auto colword = [&](int lev, float v) {  // 0 where no stencil reads
     if constexpr (SRC) {
-      // the own column is a physical cell, so its unpadded word needs no lateral image
       if (lev < 1 || lev > nk) return 0.0f;
-      const float v = ldo(a.src + (int64_t)(lev - 1) * mst, o_m);
       return a.th0 ? (a.th0[lev - 1] - 300.0f) + v : v;
     }
-    return (lev >= 0 && lev <= nk + 1) ? ldo(a.s + (int64_t)lev * st, o_s) : 0.0f;
+    return (lev >= 0 && lev <= nk + 1) ? v : 0.0f;
   };
 #pragma unroll
-  for (int q = 0; q < 7; ++q) win[q] = live ? colword(kb - 3 + q) : 0.0f;
-  // z-face flux at face kf from the window b, b[0] = S(kf-3).
-  auto zf = [&](int kf, const float* b) {
-    const float m = ldo(a.rrw + (int64_t)kf * st, o_s);
-    const float* p1 = a.c1 + (int64_t)(kf - 1) * mst;
-    const float* p2 = a.c2 + (int64_t)(kf - 1) * mst;
-    const float cc1 = a.c12col ? p1[0] : ldo(p1, o_m), cc2 = a.c12col ? p2[0] : ldo(p2, o_m);
+  for (int q = 0; q < 7; ++q) win[q] = colload(kb - 3 + q);
+#pragma unroll
+  for (int q = 0; q < 7; ++q) win[q] = colword(kb - 3 + q, win[q]);
+  // z-face flux at face kf from the window b, b[0] = S(kf-3), and the face's mass flux m
+  auto zmass = [&](int kf) { return ldo(a.rrw + (int64_t)kf * st, o_s); };
+  auto zf = [&](int kf, const float* b, float m) {
+    float cc1 = 0.0f, cc2 = 0.0f;
+    if (kf == 2 || kf == nk) {  // (the centred closures only)
+      const float* p1 = a.c1 + (int64_t)(kf - 1) * mst;
+      const float* p2 = a.c2 + (int64_t)(kf - 1) * mst;
+      cc1 = a.c12col ? p1[0] : ldo(p1, o_m);
+      cc2 = a.c12col ? p2[0] : ldo(p2, o_m);
+    }
     auto S = [&](int level) { return b[level - (kf - 3)]; };
     if (MODE == MODE_PDEF) return zflux_pdef_g(S, m, cc1, cc2, kf, nk, a.weps, a.pdefweno != 0);
     return zflux_g<WENO>(S, m, cc1, cc2, kf, nk, a.weps);
   };
   float fzb = 0.0f;
-  if (live && kb >= 2) fzb = zf(kb, win);  // S(kb-3..)
+  if (live && kb >= 2) fzb = zf(kb, win, zmass(kb));  // S(kb-3..)
   const float gzc = (!FLAT && owned && MODE != MODE_PDEF) ? ldo(a.gz, o_m) : 0.0f;
-  // A level's plane slots and own faces' mass fluxes are requested one level
-  // ahead into registers, and its cell words at the top of the level, so they
-  // arrive while the level before it (or its fluxes) is formed.
+  // One barrier a level: a level's fluxes are formed from its plane while the plane
+  // above it, requested a level earlier, is stored to the other buffer.  The own
+  // faces' mass fluxes (the top z face's included) are requested a level ahead too,
+  // and the cell words at the top of the level, so all arrive behind a level's work.
   struct Lv {
-    float plane[PS];
-    float mu, mv, mx;
+    float mu, mv, mx, mz;
     float snext;
   };
   auto fetch = [&](int k) {
     Lv v;
-    v.snext = live ? colword(k + 4) : 0.0f;  // the level entering the window after level k
-    const float* pl = SRC ? a.src + (int64_t)(k - 1) * mst : a.s + (int64_t)k * st;
-    const float pack = (SRC && a.th0) ? a.th0[k - 1] - 300.0f : 0.0f;
-#pragma unroll
-    for (int u = 0; u < PS; ++u) {
-      const float w = ldo(pl, lpo[threadIdx.x + u * NT]);
-      v.plane[u] = (SRC && a.th0) ? pack + w : w;
-    }
+    v.snext = colload(k + 4);  // the level entering the window after level k
     const float* pu = a.rru + (int64_t)k * ust;
     const float* pv = a.rrv + (int64_t)k * vst;
     v.mu = ldo(pu, o_fu);
     v.mv = ldo(pv, o_fv);
-    v.mx = xe ? ldo(pu, o_ex) : (yn ? ldo(pv, o_ex) : 0.0f);
+    v.mx = ldo(xe ? pu : pv, o_ex);
+    v.mz = zmass(min(k + 1, nk));
     return v;
   };
+  float pln[PS];  // a plane in flight
+  auto fetch_plane = [&](int k) {
+    const float* pl = SRC ? a.src + (int64_t)(k - 1) * mst : a.s + (int64_t)k * st;
+#pragma unroll
+    for (int u = 0; u < PS; ++u) pln[u] = ldo(pl, lpo[threadIdx.x + u * NT]);
+  };
+  auto store_plane = [&](int k) {
+    const float pack = (SRC && a.th0) ? a.th0[k - 1] - 300.0f : 0.0f;
+#pragma unroll
+    for (int u = 0; u < PS; ++u) lp2[k & 1][threadIdx.x + u * NT] = (SRC && a.th0) ? pack + pln[u] : pln[u];
+  };
+  fetch_plane(kb);
   Lv nx = fetch(kb);
+  store_plane(kb);
+  fetch_plane(min(kb + 1, ke));
+  __syncthreads();
   for (int k = kb; k <= ke; ++k) {
+    const float* lp = lp2[k & 1];
+    auto& lfx = lfx2[k & 1];
+    auto& lfy = lfy2[k & 1];
     const Lv cu = nx;
-    if (k < ke) nx = fetch(k + 1);
-    const float snext = cu.snext;
     const int64_t lm = (int64_t)(k - 1) * mst;  // the unpadded families' level k
     // this level's cell words, consumed after its fluxes
     float c_uw = 0.0f, c_ue = 0.0f, c_vs = 0.0f, c_vn = 0.0f, c_divx = 0.0f, c_rr0 = 0.0f, c_a0 = 0.0f,
           c_held = 0.0f, c_divterm = 0.0f;
-    if (owned) {
-      if (MODE != MODE_PDEF) {
-        c_divx = ldo(a.divx + lm, o_m);
-        c_rr0 = FLAT ? a.rr0[lm] : ldo(a.rr0 + lm, o_m);
-        if (MODE == MODE_COMPOSE) {
-          c_a0 = ldo(a.a0 + lm, o_m);
-          c_held = ldo(a.held + lm, o_m);
-          if (a.divterm) c_divterm = ldo(a.divterm + lm, o_m);
-        }
-      }
-      if (edge) {
-        const float* pu = a.rru + (int64_t)k * ust;
-        const float* pv = a.rrv + (int64_t)k * vst;
-        c_uw = ldo(pu, o_u);
-        c_ue = ldo(pu, o_u + 4u);
-        c_vs = ldo(pv, o_s);
-        c_vn = ldo(pv, o_s + (uint32_t)nxs * 4u);
+    if (MODE != MODE_PDEF) {
+      c_divx = ldo(a.divx + lm, o_m);
+      c_rr0 = FLAT ? a.rr0[lm] : ldo(a.rr0 + lm, o_m);
+      if (MODE == MODE_COMPOSE) {
+        c_a0 = ldo(a.a0 + lm, o_m);
+        c_held = ldo(a.held + lm, o_m);
+        c_divterm = ldo((a.divterm ? a.divterm : a.held) + lm, o_m);  // (unread without a divterm)
       }
     }
-#pragma unroll
-    for (int u = 0; u < PS; ++u) lp[threadIdx.x + u * NT] = cu.plane[u];
-    __syncthreads();
+    if (edge) {
+      const float* pu = a.rru + (int64_t)k * ust;
+      const float* pv = a.rrv + (int64_t)k * vst;
+      c_uw = ldo(pu, o_u);
+      c_ue = ldo(pu, o_u + 4u);
+      c_vs = ldo(pv, o_s);
+      c_vn = ldo(pv, o_s + (uint32_t)nxs * 4u);
+    }
+    nx = fetch(min(k + 1, ke));
     {  // the own faces: x face i0+tx of row j0+ty, y face j0+ty of column i0+tx
       const float* q = lp + (ty + 3) * LQ + tx;
       const float fx = face_flux<WENO, GATE>(cu.mu, q[0], q[1], q[2], q[3], q[4], q[5], a.weps);
@@ -401,7 +419,7 @@ __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
       lfy[ty][tx] = fy;
       if (MODE == MODE_TENDENCY) {
         if (a.fx && i <= ni && j < nj) sto(a.fx + (int64_t)k * ust, o_u, fx);
-        if (a.fy && i < ni && j <= nj) sto(a.fy + (int64_t)k * vst, o_s, fy);
+        if (a.fy && i < ni && j <= nj) sto(a.fy + (int64_t)k * vst, o_fv, fy);
       }
     }
     if (xe) {  // face i0+TX of row j0+tx
@@ -419,7 +437,9 @@ __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
       if (MODE == MODE_TENDENCY && a.fy && j0 + TY == nj && i0 + tx < ni) sto(a.fy + (int64_t)k * vst, o_ex, fy);
     }
     float fzt = 0.0f;
-    if (live && k + 1 <= nk) fzt = zf(k + 1, win + 1);  // S(k-2..)
+    if (live && k + 1 <= nk) fzt = zf(k + 1, win + 1, cu.mz);  // S(k-2..)
+    if (k < ke) store_plane(k + 1);  // (the buffer was last read before the barrier below of the level below)
+    fetch_plane(min(k + 2, ke));
     __syncthreads();
     if (MODE == MODE_TENDENCY && live && a.fz) {
       if (k == 1) sto(a.fz + st, o_s, 0.0f);
@@ -429,7 +449,7 @@ __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
     if (owned) {
       float fw = lfx[ty][tx], fe = lfx[ty][tx + 1];
       float fs = lfy[ty][tx], fn = lfy[ty + 1][tx];
-      const float sv = lp[(ty + 3) * LQ + tx + 3];
+      const float sv = win[3];
       float ax, ay, az;
       if (obc != 0u) {
         const float uw = c_uw, ue = c_ue, vs = c_vs, vn = c_vn;  // zero off the edges, where no closure applies
@@ -480,19 +500,23 @@ __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
     fzb = fzt;
 #pragma unroll
     for (int q = 0; q < 6; ++q) win[q] = win[q + 1];
-    win[6] = snext;
-    __syncthreads();
+    win[6] = colword(k + 4, cu.snext);
   }
 }
 
 
-// Held to six waves per SIMD (three 512-lane workgroups per CU): more
-// waves in flight hide more of each level's load latency.  Measured at
-// 640x768x80 against the unconstrained register budget (four waves): the
-// pdef tendencies 641 -> 585 us and the WENO compose 1025 -> 964 us, though
-// both spill a few registers.
+// What bounds the pass is the latency of a level's words behind its barriers: no lane
+// skips a load (a word it has no use for is read at a clipped place and dropped, so a
+// wait leaves exactly the younger loads in flight), every word is requested a level
+// ahead and a level has one barrier.  Measured against guarded loads, the z face's words
+// loaded where they are used and three barriers a level: at 640x768x80 (flat) the WENO
+// compose 927 -> 675 us and the pdef tendencies 727 -> 605, at 320x320x80 (terrain)
+// 254 -> 154 and 182 -> 140.  Six waves per SIMD (three 512-lane workgroups a CU), except the
+// terrain WENO forms, which spill at six: four waves, 154 against 165 us at 320x320x80
+// (the flat form 720 against 675 at 640x768x80).
+constexpr int adv5_waves(bool weno, int mode, bool flat) { return weno && mode != MODE_PDEF && !flat ? 4 : 6; }
 template <bool WENO, int MODE, bool FLAT, bool SRC>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(6))) void k_scalar_adv5(ScalarAdvArgs a) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(adv5_waves(WENO, MODE, FLAT)))) void k_scalar_adv5(ScalarAdvArgs a) {
   scalar_adv5_body_lanes<WENO, MODE, FLAT, SRC>(a);
 }
 
@@ -512,14 +536,14 @@ struct ScalarBatch {
 };
 
 template <int NS, bool FLAT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_scalar_compose_batch(ScalarAdvArgs a, ScalarBatch b) {
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NS == 1 ? 6 : 4))) void k_scalar_compose_batch(ScalarAdvArgs a, ScalarBatch b) {
   constexpr int PS = ((TY + 6) * LQ + NT - 1) / NT;
-  __shared__ float lfx[NS][TY][TX + 1];
-  __shared__ float lfy[NS][TY + 1][TX];
-  __shared__ float lp[NS][PS * NT];
+  __shared__ float lfx2[2][NS][TY][TX + 1];  // (two buffers each, one barrier a level, as the one-scalar pass)
+  __shared__ float lfy2[2][NS][TY + 1][TX];
+  __shared__ float lp2[2][NS][PS * NT];
   __shared__ uint32_t lpo[PS * NT];
   const int ni = a.ni, nj = a.nj, nk = a.nk;
-  const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
+  const int tx = threadIdx.x % TX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / TX);
   const int gxt = (ni + TX - 1) / TX, gyt = (nj + TY - 1) / TY;
   const int tile = xcd_tile((int)blockIdx.x, gxt * gyt * a.nchunks);
   const int i0 = (tile % gxt) * TX, j0 = ((tile / gxt) % gyt) * TY;
@@ -534,11 +558,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const int x = i + NG, y = j + NG;
   const int64_t st = (int64_t)nys * nxs, ust = (int64_t)nys * nxu, vst = (int64_t)nyv * nxs;
   const int64_t mst = (int64_t)nj * ni;
-  const uint32_t o_s = (uint32_t)(y * nxs + x) * 4u;
+  const uint32_t o_s = live ? (uint32_t)(y * nxs + x) * 4u : 0u;
   const uint32_t o_u = (uint32_t)(y * nxu + x) * 4u;
-  const uint32_t o_m = (uint32_t)(j * ni + i) * 4u;
+  const uint32_t o_m = live ? (uint32_t)(j * ni + i) * 4u : 0u;
   const uint32_t o_fu = (i <= ni && j < nj) ? o_u : 0u;
-  const uint32_t o_fv = (i < ni && j <= nj) ? o_s : 0u;
+  const uint32_t o_fv = (i < ni && j <= nj) ? (uint32_t)(y * nxs + x) * 4u : 0u;
   const bool xe = (ty == TY - 1), yn = (ty == TY - 2);
   uint32_t o_ex = 0u;
   if (xe && tx < TY && i0 + TX <= ni && j0 + tx < nj) o_ex = (uint32_t)((j0 + tx + NG) * nxu + i0 + TX + NG) * 4u;
@@ -556,19 +580,26 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
     }
     lpo[slot] = off;
   }
-  auto colword = [&](int q, int lev) {  // scalar q's own column at a level, 0 where no stencil reads
+  // scalar q's own column at a level: as loaded, and as the window holds it
+  auto colload = [&](int q, int lev) { return ldo(b.src[q] + (int64_t)(min(max(lev, 1), nk) - 1) * mst, o_m); };
+  auto colword = [&](int q, int lev, float v) {  // 0 where no stencil reads
     if (lev < 1 || lev > nk) return 0.0f;
-    const float v = ldo(b.src[q] + (int64_t)(lev - 1) * mst, o_m);
     return b.th0[q] ? (b.th0[q][lev - 1] - 300.0f) + v : v;
   };
   float win[NS][7];
 #pragma unroll
   for (int q = 0; q < NS; ++q)
 #pragma unroll
-    for (int l = 0; l < 7; ++l) win[q][l] = live ? colword(q, kb - 3 + l) : 0.0f;
+    for (int l = 0; l < 7; ++l) win[q][l] = colload(q, kb - 3 + l);
+#pragma unroll
+  for (int q = 0; q < NS; ++q)
+#pragma unroll
+    for (int l = 0; l < 7; ++l) win[q][l] = colword(q, kb - 3 + l, win[q][l]);
   // the z face kf's mass flux and weights, shared by the scalars
-  auto zmass = [&](int kf, float& m, float& cc1, float& cc2) {
-    m = ldo(a.rrw + (int64_t)kf * st, o_s);
+  auto zmass = [&](int kf) { return ldo(a.rrw + (int64_t)kf * st, o_s); };
+  auto zweights = [&](int kf, float& cc1, float& cc2) {  // (the centred closures only)
+    cc1 = cc2 = 0.0f;
+    if (kf != 2 && kf != nk) return;
     const float* p1 = a.c1 + (int64_t)(kf - 1) * mst;
     const float* p2 = a.c2 + (int64_t)(kf - 1) * mst;
     cc1 = a.c12col ? p1[0] : ldo(p1, o_m);
@@ -578,8 +609,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
   for (int q = 0; q < NS; ++q) fzb[q] = 0.0f;
   if (live && kb >= 2) {
-    float m, cc1, cc2;
-    zmass(kb, m, cc1, cc2);
+    const float m = zmass(kb);
+    float cc1, cc2;
+    zweights(kb, cc1, cc2);
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
       const float* w = win[q];
@@ -588,62 +620,68 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   }
   const float gzc = (!FLAT && owned) ? ldo(a.gz, o_m) : 0.0f;
   struct Lv {
-    float plane[NS][PS];
     float snext[NS];
-    float mu, mv, mx;
+    float mu, mv, mx, mz;
   };
   auto fetch = [&](int k) {
     Lv v;
 #pragma unroll
-    for (int q = 0; q < NS; ++q) {
-      v.snext[q] = live ? colword(q, k + 4) : 0.0f;
-      const float* pl = b.src[q] + (int64_t)(k - 1) * mst;
-      const float pack = b.th0[q] ? b.th0[q][k - 1] - 300.0f : 0.0f;
-#pragma unroll
-      for (int u = 0; u < PS; ++u) {
-        const float w = ldo(pl, lpo[threadIdx.x + u * NT]);
-        v.plane[q][u] = b.th0[q] ? pack + w : w;
-      }
-    }
+    for (int q = 0; q < NS; ++q) v.snext[q] = colload(q, k + 4);
     const float* pu = a.rru + (int64_t)k * ust;
     const float* pv = a.rrv + (int64_t)k * vst;
     v.mu = ldo(pu, o_fu);
     v.mv = ldo(pv, o_fv);
-    v.mx = xe ? ldo(pu, o_ex) : (yn ? ldo(pv, o_ex) : 0.0f);
+    v.mx = ldo(xe ? pu : pv, o_ex);
+    v.mz = zmass(min(k + 1, nk));
     return v;
   };
+  float pln[NS][PS];
+  auto fetch_plane = [&](int k) {
+#pragma unroll
+    for (int q = 0; q < NS; ++q)
+#pragma unroll
+      for (int u = 0; u < PS; ++u) pln[q][u] = ldo(b.src[q] + (int64_t)(k - 1) * mst, lpo[threadIdx.x + u * NT]);
+  };
+  auto store_plane = [&](int k) {
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+      const float pack = b.th0[q] ? b.th0[q][k - 1] - 300.0f : 0.0f;
+#pragma unroll
+      for (int u = 0; u < PS; ++u) lp2[k & 1][q][threadIdx.x + u * NT] = b.th0[q] ? pack + pln[q][u] : pln[q][u];
+    }
+  };
+  fetch_plane(kb);
   Lv nx = fetch(kb);
+  store_plane(kb);
+  fetch_plane(min(kb + 1, ke));
+  __syncthreads();
   for (int k = kb; k <= ke; ++k) {
+    auto& lp = lp2[k & 1];
+    auto& lfx = lfx2[k & 1];
+    auto& lfy = lfy2[k & 1];
     const Lv cu = nx;
-    if (k < ke) nx = fetch(k + 1);
     const int64_t lm = (int64_t)(k - 1) * mst;
     float c_uw = 0.0f, c_ue = 0.0f, c_vs = 0.0f, c_vn = 0.0f, c_divx = 0.0f, c_rr0 = 0.0f;
     float c_a0[NS], c_held[NS], c_divterm[NS];
 #pragma unroll
     for (int q = 0; q < NS; ++q) c_a0[q] = c_held[q] = c_divterm[q] = 0.0f;
-    if (owned) {
-      c_divx = ldo(a.divx + lm, o_m);
-      c_rr0 = FLAT ? a.rr0[lm] : ldo(a.rr0 + lm, o_m);
+    c_divx = ldo(a.divx + lm, o_m);
+    c_rr0 = FLAT ? a.rr0[lm] : ldo(a.rr0 + lm, o_m);
 #pragma unroll
-      for (int q = 0; q < NS; ++q) {
-        c_a0[q] = ldo(b.a0[q] + lm, o_m);
-        c_held[q] = ldo(b.held[q] + lm, o_m);
-        if (b.divterm[q]) c_divterm[q] = ldo(b.divterm[q] + lm, o_m);
-      }
-      if (edge) {
-        const float* pu = a.rru + (int64_t)k * ust;
-        const float* pv = a.rrv + (int64_t)k * vst;
-        c_uw = ldo(pu, o_u);
-        c_ue = ldo(pu, o_u + 4u);
-        c_vs = ldo(pv, o_s);
-        c_vn = ldo(pv, o_s + (uint32_t)nxs * 4u);
-      }
+    for (int q = 0; q < NS; ++q) {
+      c_a0[q] = ldo(b.a0[q] + lm, o_m);
+      c_held[q] = ldo(b.held[q] + lm, o_m);
+      c_divterm[q] = ldo((b.divterm[q] ? b.divterm[q] : b.held[q]) + lm, o_m);  // (unread without a divterm)
     }
-#pragma unroll
-    for (int q = 0; q < NS; ++q)
-#pragma unroll
-      for (int u = 0; u < PS; ++u) lp[q][threadIdx.x + u * NT] = cu.plane[q][u];
-    __syncthreads();
+    if (edge) {
+      const float* pu = a.rru + (int64_t)k * ust;
+      const float* pv = a.rrv + (int64_t)k * vst;
+      c_uw = ldo(pu, o_u);
+      c_ue = ldo(pu, o_u + 4u);
+      c_vs = ldo(pv, o_s);
+      c_vn = ldo(pv, o_s + (uint32_t)nxs * 4u);
+    }
+    nx = fetch(min(k + 1, ke));
 #pragma unroll
     for (int q = 0; q < NS; ++q) {
       const float* P = lp[q];
@@ -667,21 +705,24 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
 #pragma unroll
     for (int q = 0; q < NS; ++q) fzt[q] = 0.0f;
     if (live && k + 1 <= nk) {
-      float m, cc1, cc2;
-      zmass(k + 1, m, cc1, cc2);
+      const float m = cu.mz;
+      float cc1, cc2;
+      zweights(k + 1, cc1, cc2);
 #pragma unroll
       for (int q = 0; q < NS; ++q) {
         const float* w = win[q] + 1;  // S(k-2..)
         fzt[q] = zflux_g<false>([&](int level) { return w[level - (k - 2)]; }, m, cc1, cc2, k + 1, nk, a.weps);
       }
     }
+    if (k < ke) store_plane(k + 1);
+    fetch_plane(min(k + 2, ke));
     __syncthreads();
     if (owned) {
 #pragma unroll
       for (int q = 0; q < NS; ++q) {
         float fw = lfx[q][ty][tx], fe = lfx[q][ty][tx + 1];
         float fs = lfy[q][ty][tx], fn = lfy[q][ty + 1][tx];
-        const float sv = lp[q][(ty + 3) * LQ + tx + 3];
+        const float sv = win[q][3];
         float ax, ay, az;
         if (obc != 0u) {
           const float uw = c_uw, ue = c_ue, vs = c_vs, vn = c_vn;  // zero off the edges, where no closure applies
@@ -725,9 +766,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
       fzb[q] = fzt[q];
 #pragma unroll
       for (int l = 0; l < 6; ++l) win[q][l] = win[q][l + 1];
-      win[q][6] = cu.snext[q];
+      win[q][6] = colword(q, k + 4, cu.snext[q]);
     }
-    __syncthreads();
   }
 }
 
@@ -782,20 +822,19 @@ GM1_DEV float donor_ratio(float lo, float c, float hi) {
   return (sum > 1.0e-30f) ? fmaxf(c, -sum) / sum : 0.0f;
 }
 
-// mass change and flag of the centre of five consecutive values v[0..4]
-GM1_DEV void row_mass(const float v[5], float& mass, bool& flag) {
+// mass change and flag of the centre c of five consecutive values v0, v1, c, v3, v4
+GM1_DEV void row_mass(float v0, float v1, float c, float v3, float v4, float& mass, bool& flag) {
   mass = 0.0f;
   flag = false;
-  const float c = v[2];
   if (c < 0.0f) {
-    const float r = donor_ratio(v[1], c, v[3]);
+    const float r = donor_ratio(v1, c, v3);
     if (r != 0.0f) {
-      const float sum = fmaxf(0.0f, v[1]) + fmaxf(0.0f, v[3]);
+      const float sum = fmaxf(0.0f, v1) + fmaxf(0.0f, v3);
       mass = 0.0f - sum * r;
       flag = true;
     }
   } else if (c > 1.0e-30f) {
-    const float rl = donor_ratio(v[0], v[1], v[2]), rr = donor_ratio(v[2], v[3], v[4]);
+    const float rl = donor_ratio(v0, v1, c), rr = donor_ratio(c, v3, v4);
     if (rl != 0.0f) { mass = mass + c * rl; flag = true; }
     if (rr != 0.0f) { mass = mass + c * rr; flag = true; }
   }
@@ -806,13 +845,19 @@ GM1_DEV void row_mass(const float v[5], float& mass, bool& flag) {
 // those of the lateral family's image), wavefronts 0-3 the tile's south and
 // north halo rows' y candidates and wavefront 4 the west and east halo
 // columns' x candidates; the z candidates ride in a five-level register
-// window.  Every word a level needs is requested one level ahead.
+// window.  Every word a level needs is requested one level ahead, by loads no lane
+// skips (a word a lane has no use for is read at a clipped place and dropped): a
+// wait then leaves exactly the loads issued after it in flight.  The candidates
+// take two buffers in turn, one barrier a level, and the column's own words, loaded
+// as those of level k+2 for the z candidates, are carried down to level k (measured
+// against loading them again there: 123 -> 111 us at 320x320x80, 583 -> 537 at
+// 640x768x80; a register budget for six waves spills it, 324 and 1100 us).
 template <bool FLAT>
 __global__ __launch_bounds__(RT) void k_pdef_repair(PdefArgs a) {
-  __shared__ float lcx[RY][RX + 4];
-  __shared__ float lcy[RY + 4][RX];
+  __shared__ float lcx2[2][RY][RX + 4];
+  __shared__ float lcy2[2][RY + 4][RX];
   const int ni = a.ni, nj = a.nj, nk = a.nk;
-  const int tx = threadIdx.x % RX, ty = threadIdx.x / RX;
+  const int tx = threadIdx.x % RX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / RX);  // (a wavefront is one row)
   const int gxt = (ni + RX - 1) / RX, gyt = (nj + RY - 1) / RY;
   const int tile = xcd_tile((int)blockIdx.x, gxt * gyt * a.nchunks);
   const int i0 = (tile % gxt) * RX, j0 = ((tile / gxt) % gyt) * RY;
@@ -823,19 +868,17 @@ __global__ __launch_bounds__(RT) void k_pdef_repair(PdefArgs a) {
   const unsigned wbc = side_of(a.obc, 0), ebc = side_of(a.obc, 1), sbc = side_of(a.obc, 2), nbc = side_of(a.obc, 3);
   const int nxs = sx(ni), nys = sy(nj), nxu = ux(ni), nyv = vy(nj);
   const int64_t st = (int64_t)nys * nxs, ust = (int64_t)nys * nxu, vst = (int64_t)nyv * nxs, mst = (int64_t)nj * ni;
-  // a cell's words: unpadded (m), padded scalar / v / w families (s), u family (u)
+  // a cell's words: unpadded (m), padded scalar / v / w families (s), u family (u), the scalar's (w)
   struct Cell {
-    uint32_t m, s, u;
+    uint32_t m, s, u, w;
   };
+  const uint32_t from_src = a.src ? ~0u : 0u;
   auto cell = [&](int ci, int cj) {
-    Cell c;
-    c.m = (uint32_t)(cj * ni + ci) * 4u;
-    c.s = (uint32_t)((cj + NG) * nxs + ci + NG) * 4u;
-    c.u = (uint32_t)((cj + NG) * nxu + ci + NG) * 4u;
-    return c;
+    const uint32_t m = (uint32_t)(cj * ni + ci) * 4u, s = (uint32_t)((cj + NG) * nxs + ci + NG) * 4u;
+    return Cell{m, s, (uint32_t)((cj + NG) * nxu + ci + NG) * 4u, (m & from_src) | (s & ~from_src)};
   };
   auto word = [&](int k, const Cell& c) {  // the scalar's current value
-    return a.src ? ldo(a.src + (int64_t)(k - 1) * mst, c.m) : ldo(a.s + (int64_t)k * st, c.s);
+    return ldo(a.src ? a.src + (int64_t)(k - 1) * mst : a.s + (int64_t)k * st, c.w);
   };
   auto rho_at = [&](int k, const Cell& c) {
     return FLAT ? a.rho0[(int64_t)(k - 1) * mst] : ldo(a.rho0 + (int64_t)(k - 1) * mst, c.m);
@@ -873,6 +916,8 @@ __global__ __launch_bounds__(RT) void k_pdef_repair(PdefArgs a) {
   const Cell hc = cell(hi, hj);
   const bool h_lo = hk == 1 ? (hi == 0 && wbc == 2u) : (hj == 0 && sbc == 2u);
   const bool h_hi = hk == 1 ? (hi + 1 == ni && ebc == 2u) : (hj + 1 == nj && nbc == 2u);
+  const bool hx = ty == 4;  // (the wavefront's halo candidates are x candidates)
+  const uint32_t ho = hx ? hc.u : hc.s;
   const float hgz = (!FLAT && hk) ? ldo(a.gz, hc.m) : 1.0f;
   // z candidate of the own column at level k (0 outside 1..nk) from its words
   auto zcand = [&](int k, float rho, float qa, float az, float sv, float wb, float wt) {
@@ -881,134 +926,129 @@ __global__ __launch_bounds__(RT) void k_pdef_repair(PdefArgs a) {
     if constexpr (FLAT) return rho * qa + a.dt * (az + ((sv * d) * a.rdz) * a.mh[k]);
     return rho * qa + (a.dt * (az + (sv * d) * a.rdz)) * gzc;
   };
-  auto zwords = [&](int k) {  // the own column's z candidate at level k from memory
-    if (!live || k < 1 || k > nk) return 0.0f;
-    const int64_t lm = (int64_t)(k - 1) * mst;
-    return zcand(k, rho_at(k, oc), ldo(a.qa + lm, oc.m), ldo(a.advz + lm, oc.m), word(k, oc),
-                 ldo(a.rrw + (int64_t)k * st, oc.s), ldo(a.rrw + (int64_t)(k + 1) * st, oc.s));
-  };
+  const float rgc = (!FLAT && live) ? ldo(a.rgz, oc.m) : 1.0f;
   float cz[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};  // candidates at k-2..k+2
-  for (int d = 0; d < 4; ++d) cz[d + 1] = zwords(kb - 2 + d);
+  // the own column's words at levels k and k+1 (loaded once, as level k+2's, and carried) and rrw at k..k+2
+  struct Own {
+    float qa, sv, az, rho;
+  };
+  Own c0, c1;
+  float w0, w1, w2;
+  {  // below and beside the first level, all words requested before the first is used
+    float q[4], z[4], w[4], m0[4], m1[4], r[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      const int k = min(max(kb - 2 + d, 1), nk);
+      const int64_t lm = (int64_t)(k - 1) * mst;
+      r[d] = rho_at(k, oc);
+      q[d] = ldo(a.qa + lm, oc.m);
+      z[d] = ldo(a.advz + lm, oc.m);
+      w[d] = word(k, oc);
+      m0[d] = ldo(a.rrw + (int64_t)k * st, oc.s);
+      m1[d] = ldo(a.rrw + (int64_t)(k + 1) * st, oc.s);
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) cz[d + 1] = zcand(kb - 2 + d, r[d], q[d], z[d], w[d], m0[d], m1[d]);
+    c0 = Own{q[2], w[2], z[2], r[2]};
+    c1 = Own{q[3], w[3], z[3], r[3]};
+    w0 = m0[2];
+    w1 = m1[2];
+    w2 = m1[3];
+  }
   struct Lv {
-    float qa, ax, ay, az, sv, divx, held, uw, ue, vs, vn, wb, wt, rho, rr0;  // the own cell at level k
-    float zqa, zaz, zsv, zwb, zwt, zrho;                                      // the own column at level k+2
+    float ax, ay, divx, held, uw, ue, vs, vn, rr0;  // the own cell at level k
+    float zqa, zaz, zsv, zwt, zrho;                 // the own column at level k+2
     float hqa, hadv, hsv, hm0, hm1, hrho;                                     // the halo cell at level k
   };
   auto fetch = [&](int k) {
-    Lv v{};
+    Lv v;
     const int64_t lm = (int64_t)(k - 1) * mst;
-    if (xc || yc) {
-      v.qa = ldo(a.qa + lm, oc.m);
-      v.sv = word(k, oc);
-      v.rho = rho_at(k, oc);
-      if (xc) {
-        v.ax = ldo(a.advx + lm, oc.m);
-        v.uw = ldo(a.rru + (int64_t)k * ust, oc.u);
-        v.ue = ldo(a.rru + (int64_t)k * ust, oc.u + 4u);
-      }
-      if (yc) {
-        v.ay = ldo(a.advy + lm, oc.m);
-        v.vs = ldo(a.rrv + (int64_t)k * vst, oc.s);
-        v.vn = ldo(a.rrv + (int64_t)k * vst, oc.s + (uint32_t)nxs * 4u);
-      }
-    }
-    if (live) {
-      v.az = ldo(a.advz + lm, oc.m);
-      v.divx = ldo(a.divx + lm, oc.m);
-      v.held = ldo(a.held + lm, oc.m);
-      v.wb = ldo(a.rrw + (int64_t)k * st, oc.s);
-      v.wt = ldo(a.rrw + (int64_t)(k + 1) * st, oc.s);
-      v.rr0 = FLAT ? a.rr0[lm] : ldo(a.rr0 + lm, oc.m);
-      const int kz = k + 2;
-      if (kz <= nk) {
-        const int64_t lz = (int64_t)(kz - 1) * mst;
-        v.zqa = ldo(a.qa + lz, oc.m);
-        v.zaz = ldo(a.advz + lz, oc.m);
-        v.zsv = word(kz, oc);
-        v.zwb = ldo(a.rrw + (int64_t)kz * st, oc.s);
-        v.zwt = ldo(a.rrw + (int64_t)(kz + 1) * st, oc.s);
-        v.zrho = rho_at(kz, oc);
-      }
-    }
-    if (hk) {
-      v.hqa = ldo(a.qa + lm, hc.m);
-      v.hsv = word(k, hc);
-      v.hrho = rho_at(k, hc);
-      if (hk == 1) {
-        v.hadv = ldo(a.advx + lm, hc.m);
-        v.hm0 = ldo(a.rru + (int64_t)k * ust, hc.u);
-        v.hm1 = ldo(a.rru + (int64_t)k * ust, hc.u + 4u);
-      } else {
-        v.hadv = ldo(a.advy + lm, hc.m);
-        v.hm0 = ldo(a.rrv + (int64_t)k * vst, hc.s);
-        v.hm1 = ldo(a.rrv + (int64_t)k * vst, hc.s + (uint32_t)nxs * 4u);
-      }
-    }
+    v.ax = ldo(a.advx + lm, oc.m);
+    v.uw = ldo(a.rru + (int64_t)k * ust, oc.u);
+    v.ue = ldo(a.rru + (int64_t)k * ust, oc.u + 4u);
+    v.ay = ldo(a.advy + lm, oc.m);
+    v.vs = ldo(a.rrv + (int64_t)k * vst, oc.s);
+    v.vn = ldo(a.rrv + (int64_t)k * vst, oc.s + (uint32_t)nxs * 4u);
+    v.divx = ldo(a.divx + lm, oc.m);
+    v.held = ldo(a.held + lm, oc.m);
+    v.rr0 = FLAT ? a.rr0[lm] : ldo(a.rr0 + lm, oc.m);
+    const int kz = min(k + 2, nk);
+    const int64_t lz = (int64_t)(kz - 1) * mst;
+    v.zqa = ldo(a.qa + lz, oc.m);
+    v.zaz = ldo(a.advz + lz, oc.m);
+    v.zsv = word(kz, oc);
+    v.zwt = ldo(a.rrw + (int64_t)(kz + 1) * st, oc.s);
+    v.zrho = rho_at(kz, oc);
+    v.hqa = ldo(a.qa + lm, hc.m);
+    v.hsv = word(k, hc);
+    v.hrho = rho_at(k, hc);
+    const float* hm = hx ? a.rru + (int64_t)k * ust : a.rrv + (int64_t)k * vst;
+    v.hadv = ldo((hx ? a.advx : a.advy) + lm, hc.m);
+    v.hm0 = ldo(hm, ho);
+    v.hm1 = ldo(hm, ho + (hx ? 4u : (uint32_t)nxs * 4u));
     return v;
   };
   Lv nx = fetch(kb);
   for (int k = kb; k <= ke; ++k) {
     const Lv cu = nx;
-    if (k < ke) nx = fetch(k + 1);
-    if (xc) lcx[ty][tx + 2] = pdef_cand<FLAT>(cu.rho * cu.qa, cu.ax, cu.sv, cu.uw, cu.ue, a.rdx, a.dt, gzc, x_lo, x_hi);
-    if (yc) lcy[ty + 2][tx] = pdef_cand<FLAT>(cu.rho * cu.qa, cu.ay, cu.sv, cu.vs, cu.vn, a.rdy, a.dt, gzc, y_lo, y_hi);
+    nx = fetch(min(k + 1, ke));
+    auto& lcx = lcx2[k & 1];
+    auto& lcy = lcy2[k & 1];
+    if (xc) lcx[ty][tx + 2] = pdef_cand<FLAT>(c0.rho * c0.qa, cu.ax, c0.sv, cu.uw, cu.ue, a.rdx, a.dt, gzc, x_lo, x_hi);
+    if (yc) lcy[ty + 2][tx] = pdef_cand<FLAT>(c0.rho * c0.qa, cu.ay, c0.sv, cu.vs, cu.vn, a.rdy, a.dt, gzc, y_lo, y_hi);
     if (hk) {
       const float c = pdef_cand<FLAT>(cu.hrho * cu.hqa, cu.hadv, cu.hsv, cu.hm0, cu.hm1, hk == 1 ? a.rdx : a.rdy, a.dt,
                                       hgz, h_lo, h_hi);
       if (hk == 1) lcx[hr][ht] = c;
       else lcy[hr][ht] = c;
     }
+#pragma unroll
     for (int d = 0; d < 4; ++d) cz[d] = cz[d + 1];
-    cz[4] = live ? zcand(k + 2, cu.zrho, cu.zqa, cu.zaz, cu.zsv, cu.zwb, cu.zwt) : 0.0f;
+    cz[4] = live ? zcand(k + 2, cu.zrho, cu.zqa, cu.zaz, cu.zsv, w2, cu.zwt) : 0.0f;
     __syncthreads();
     if (live) {
       const int64_t lm = (int64_t)(k - 1) * mst;
-      const float sv = cu.sv;
+      const float sv = c0.sv;
       constexpr bool flat = FLAT;
-      const float r0a = cu.rho * cu.qa;
-      const float rg = flat ? 1.0f : ldo(a.rgz, oc.m);
-      float ax = cu.ax, ay = cu.ay, az = cu.az;
+      const float r0a = c0.rho * c0.qa;
+      const float rg = rgc;
+      float ax = cu.ax, ay = cu.ay, az = c0.az;
       float v[5], mass;
       bool flag;
+#pragma unroll
       for (int d = 0; d < 5; ++d) v[d] = lcx[ty][tx + d];
-      row_mass(v, mass, flag);
+      row_mass(v[0], v[1], v[2], v[3], v[4], mass, flag);
       if (flag) {
         const float du = cu.ue - cu.uw;
         const float first = flat ? ((v[2] + mass) - r0a) * a.rdt : (((v[2] + mass) - r0a) * a.rdt) * rg;
         ax = first - (sv * du) * a.rdx;
       }
+#pragma unroll
       for (int d = 0; d < 5; ++d) v[d] = lcy[ty + d][tx];
-      row_mass(v, mass, flag);
+      row_mass(v[0], v[1], v[2], v[3], v[4], mass, flag);
       if (flag) {
         const float dv = cu.vn - cu.vs;
         const float first = flat ? ((v[2] + mass) - r0a) * a.rdt : (((v[2] + mass) - r0a) * a.rdt) * rg;
         ay = first - (sv * dv) * a.rdy;
       }
-      row_mass(cz, mass, flag);
+      row_mass(cz[0], cz[1], cz[2], cz[3], cz[4], mass, flag);
       if (flag) {
-        const float dw = cu.wt - cu.wb;
+        const float dw = w1 - w0;
         if (flat) az = ((cz[2] + mass) - r0a) * a.rdt - ((sv * dw) * a.rdz) * a.mh[k];
         else az = (((cz[2] + mass) - r0a) * a.rdt) * rg - (sv * dw) * a.rdz;
       }
       float t = (ax + ay) + az;
       t = t + sv * cu.divx;
       const float adv = flat ? t * cu.rr0 : (t * cu.rr0) * gzc;
-      const float o = cu.qa + a.dt * (cu.held + adv);
+      const float o = c0.qa + a.dt * (cu.held + adv);
       sto(a.out + lm, oc.m, (fabsf(o) < 1.0e-30f) ? 0.0f : o);
     }
-    __syncthreads();
+    c0 = c1;
+    c1 = Own{cu.zqa, cu.zsv, cu.zaz, cu.zrho};
+    w0 = w1;
+    w1 = w2;
+    w2 = cu.zwt;
   }
-}
-
-int chunks_for(int tiles, int nk, int* kchunk) {
-  // enough column chunks to put >= 1024 tiles in flight on 256 CUs (measured at
-  // 640x768x80 against 2048 and 4096: the paired compose 764 -> 744 us, the
-  // pdef repair 521 -> 508 us)
-  int chunks = (1024 + tiles - 1) / tiles;
-  if (chunks > nk) chunks = nk;
-  if (chunks < 1) chunks = 1;
-  *kchunk = (nk + chunks - 1) / chunks;
-  return (nk + *kchunk - 1) / *kchunk;
 }
 
 template <bool FLAT, bool SRC>
@@ -1035,7 +1075,7 @@ void launch_scalar_variant(const ScalarAdvArgs& a, int use_weno, int mode, dim3 
 
 int launch_scalar_tile(ScalarAdvArgs& a, int use_weno, int mode, hipStream_t s) {
   const int tiles = ((a.ni + TX - 1) / TX) * ((a.nj + TY - 1) / TY);
-  const int chunks = chunks_for(tiles, a.nk, &a.kchunk);
+  const int chunks = tile_chunks(tiles, a.nk, adv5_waves(use_weno || mode == MODE_PDEF, mode, a.mh != nullptr) / 2, &a.kchunk);
   a.nchunks = chunks;
   dim3 grid(tiles * chunks);
   if (a.mh) {
@@ -1145,7 +1185,7 @@ static int pdef_stage(const float* scalar, const float* src, const float* rru, c
   p.dt = dttmp; p.rdt = 1.0f / dttmp; p.rdx = 1.0f / dx; p.rdy = 1.0f / dy; p.rdz = rdzv;
   p.obc = obc & 0xFFFFu;
   const int tiles = ((ni + RX - 1) / RX) * ((nj + RY - 1) / RY);
-  const int chunks = chunks_for(tiles, nk, &p.kchunk);
+  const int chunks = tile_chunks(tiles, nk, 2, &p.kchunk);
   p.nchunks = chunks;
   if (p.mh) hipLaunchKernelGGL(k_pdef_repair<true>, dim3(tiles * chunks), dim3(RT), 0, s, p);
   else hipLaunchKernelGGL(k_pdef_repair<false>, dim3(tiles * chunks), dim3(RT), 0, s, p);
@@ -1217,7 +1257,7 @@ int gm1hip_scalar_rk_stage_src_batch(int ns, const float* const* srcs, const flo
     b.divterm[q] = divterms ? divterms[q] : nullptr; b.out[q] = outs[q];
   }
   const int tiles = ((ni + TX - 1) / TX) * ((nj + TY - 1) / TY);
-  a.nchunks = chunks_for(tiles, nk, &a.kchunk);
+  a.nchunks = tile_chunks(tiles, nk, ns == 1 ? 3 : 2, &a.kchunk);
   const dim3 grid(tiles * a.nchunks);
   hipStream_t s = (hipStream_t)stream;
   const bool flat = flat_column != nullptr;

@@ -9,6 +9,7 @@
 #pragma once
 #pragma clang fp contract(off)
 
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -44,6 +45,28 @@ GM1_DEV int xcd_tile(int linear, int n) {
   const int per = n / X, rem = n % X;
   const int x = linear % X, r = linear / X;
   return (x < rem) ? x * (per + 1) + r : rem * (per + 1) + (x - rem) * per + r;
+}
+
+// Level chunks of a kernel of `tiles` 512-lane tiles marching nk levels, per_cu
+// workgroups resident on each of the 256 CUs: the count whose estimated time is
+// least (of counts within a hundredth, the largest).  A chunk takes a level more than
+// it has (its window and first plane), full rounds of resident workgroups take a
+// chunk's time each, and a last round takes 0.5 + 0.5 f of it where its fullest CU
+// holds a fraction f of per_cu (fewer waves on a CU each run faster).  The rule follows
+// the measured minima: 200 tiles of 80 levels at two per CU, 5 chunks 154 us, 10 160,
+// 16 173, 4 179; 200 of 80 at three, 5 140, 10 142, 3 152, 4 167; 48 of 64 at three,
+// 16 36 us, 10 40, 5 44; 960 of 80 at three, 4 604 us, 5 612, 10 640, 2 625.
+inline int tile_chunks(int tiles, int nk, int per_cu, int* kchunk) {
+  auto cost = [&](int kc) {
+    const int64_t groups = (int64_t)tiles * ((nk + kc - 1) / kc), slots = 256 * per_cu;
+    const int64_t last = (groups % slots + 255) / 256;  // workgroups on the last round's fullest CU
+    return (kc + 1) * ((double)(groups / slots) + (last ? 0.5 + 0.5 * (double)last / per_cu : 0.0));
+  };
+  double least = cost(nk);
+  for (int kc = 1; kc < nk; ++kc) least = std::min(least, cost(kc));
+  *kchunk = 1;
+  while (cost(*kchunk) > 1.01 * least) ++*kchunk;
+  return (nk + *kchunk - 1) / *kchunk;
 }
 
 // The word at a 32-bit byte offset from a base the whole workgroup shares:

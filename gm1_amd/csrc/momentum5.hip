@@ -214,30 +214,48 @@ __global__ __launch_bounds__(256) void k_mom_mass_flat(
   }
 }
 
-// vertical flux of u (stag 0) or v (stag 1) at w level kf of column (j, i)
-template <int STAG, class Get>
-GM1_DEV float uvz_g(const MomArgs& a, int kf, int j, int i, Get Q) {
+// the words a column's vertical flux of u (stag 0) or v (stag 1) at w level kf
+// takes beside its own: the pair of rrw and, where the face has a centred closure
+// (kf = 2 and nk), the pair of c2
+struct UvzWords { float r0, r1, c0, c1; };
+
+template <int STAG>
+GM1_DEV void uvz_c2(const MomArgs& a, int kf, int j, int i, UvzWords& w) {
+  const int ni = a.ni, nj = a.nj;
+  const float* c2k = a.c2 + (int64_t)(kf - 1) * nj * ni;
+  const int jl = STAG == 0 ? clampi(j, nj) : clampi(j - 1, nj), jh = clampi(j, nj);
+  const int il = STAG == 0 ? clampi(i - 1, ni) : clampi(i, ni), ih = clampi(i, ni);
+  w.c0 = ldo(c2k, (uint32_t)(jl * ni + il) * 4u);
+  w.c1 = ldo(c2k, (uint32_t)(jh * ni + ih) * 4u);
+}
+
+template <int STAG>
+GM1_DEV UvzWords uvz_words(const MomArgs& a, int kf, int j, int i) {
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const int nxs = sx(ni), nys = sy(nj);
-  float m, c2h;
+  UvzWords w;
   // the level's planes, each word at a 32-bit byte offset
-  const float* c2k = a.c2 + (int64_t)(kf - 1) * nj * ni;
   const float* R = a.rrw + (int64_t)kf * nys * nxs;
   if (STAG == 0) {
     const bool pw = per(a.obc, 0), pe = per(a.obc, 1);
     const int rb = (j + NG) * nxs + NG;
-    m = 0.5f * (ldo(R, (uint32_t)(rb + wc(i, ni, pw, pe)) * 4u) + ldo(R, (uint32_t)(rb + wc(i - 1, ni, pw, pe)) * 4u));
-    const int jc = clampi(j, nj);
-    c2h = 0.5f * (ldo(c2k, (uint32_t)(jc * ni + clampi(i - 1, ni)) * 4u) +
-                  ldo(c2k, (uint32_t)(jc * ni + clampi(i, ni)) * 4u));
+    w.r0 = ldo(R, (uint32_t)(rb + wc(i, ni, pw, pe)) * 4u);
+    w.r1 = ldo(R, (uint32_t)(rb + wc(i - 1, ni, pw, pe)) * 4u);
   } else {
     const bool ps = per(a.obc, 2), pn = per(a.obc, 3);
-    m = 0.5f * (ldo(R, (uint32_t)((wc(j, nj, ps, pn) + NG) * nxs + i + NG) * 4u) +
-                ldo(R, (uint32_t)((wc(j - 1, nj, ps, pn) + NG) * nxs + i + NG) * 4u));
-    const int ic = clampi(i, ni);
-    c2h = 0.5f * (ldo(c2k, (uint32_t)(clampi(j - 1, nj) * ni + ic) * 4u) +
-                  ldo(c2k, (uint32_t)(clampi(j, nj) * ni + ic) * 4u));
+    w.r0 = ldo(R, (uint32_t)((wc(j, nj, ps, pn) + NG) * nxs + i + NG) * 4u);
+    w.r1 = ldo(R, (uint32_t)((wc(j - 1, nj, ps, pn) + NG) * nxs + i + NG) * 4u);
   }
+  w.c0 = w.c1 = 0.0f;
+  if (kf == 2 || kf == nk) uvz_c2<STAG>(a, kf, j, i, w);
+  return w;
+}
+
+// the flux from those words and the column's (Q(level))
+template <class Get>
+GM1_DEV float uvz_g(const UvzWords& w, int kf, int nk, Get Q) {
+  const float m = 0.5f * (w.r0 + w.r1);
+  const float c2h = 0.5f * (w.c0 + w.c1);
   const float c1h = 1.0f - c2h;
   float r;
   if (kf == 2) {
@@ -249,9 +267,10 @@ GM1_DEV float uvz_g(const MomArgs& a, int kf, int j, int i, Get Q) {
   } else if (kf == nk - 1) {
     r = (m >= 0.0f) ? flx5(Q(kf - 3), Q(kf - 2), Q(kf - 1), Q(kf), Q(kf + 1))
                     : flx3(Q(kf + 1), Q(kf), Q(kf - 1));
-  } else {
-    r = (m >= 0.0f) ? flx5(Q(kf - 3), Q(kf - 2), Q(kf - 1), Q(kf), Q(kf + 1))
-                    : flx5(Q(kf + 2), Q(kf + 1), Q(kf), Q(kf - 1), Q(kf - 2));
+  } else {  // one value of the upwind words, whichever way the lanes' fluxes point
+    const bool up = m >= 0.0f;
+    const float q0 = Q(kf - 3), q1 = Q(kf - 2), q2 = Q(kf - 1), q3 = Q(kf), q4 = Q(kf + 1), q5 = Q(kf + 2);
+    r = flx5(up ? q0 : q5, up ? q1 : q4, up ? q2 : q3, up ? q3 : q2, up ? q4 : q1);
   }
   return m * r;
 }
@@ -265,7 +284,7 @@ GM1_DEV float uvz(const MomArgs& a, int kf, int j, int i) {
   const int nyq = (STAG == 0) ? sy(nj) : vy(nj);
   const int64_t st = (int64_t)nyq * nxq;
   const float* col = q + (int64_t)(j + NG) * nxq + (i + NG);
-  return uvz_g<STAG>(a, kf, j, i, [&](int lev) { return col[(int64_t)lev * st]; });
+  return uvz_g(uvz_words<STAG>(a, kf, j, i), kf, a.nk, [&](int lev) { return col[(int64_t)lev * st]; });
 }
 
 
@@ -286,15 +305,6 @@ constexpr int MTX = 64, MTY = 8, MNT = MTX * MTY, MPX = MTX + 6;
 constexpr int MPS = ((MTY + 6) * MPX + MNT - 1) / MNT;  // plane slots a lane
 static_assert(MTX == 64, "a wavefront is one tile row");
 
-int mom_chunks(int tiles, int nk, int* kchunk) {
-  // >= 4096 tiles in flight (measured at 640x768x80 against 2048: v 415 -> 405 us, w 432 -> 420 us)
-  int chunks = (4096 + tiles - 1) / tiles;
-  if (chunks > nk) chunks = nk;
-  if (chunks < 1) chunks = 1;
-  *kchunk = (nk + chunks - 1) / chunks;
-  return (nk + *kchunk - 1) / *kchunk;
-}
-
 // fifth-order upwind value of the six words q0..q5 around a flux point (q2|q3
 // straddle it), times the mass flux m
 GM1_DEV float point_flux(float m, float q0, float q1, float q2, float q3, float q4, float q5) {
@@ -303,19 +313,26 @@ GM1_DEV float point_flux(float m, float q0, float q1, float q2, float q3, float 
 }
 
 // u-momentum: faces f0 .. f0+nf-1 (tile columns), rows 0..nj-1 (tile rows).
-// The u and v tiles are held to six waves per SIMD (three workgroups a CU):
-// measured at 640x768x80, u 472 -> 427 us and v 492 -> 416 us against four
-// waves, though both spill a few registers; the w tile, which spills far
-// more at six, stays at four.
+// What bounds the three tiles is the latency of a level's words behind its barriers,
+// so no lane skips a load (a word it has no use for is read at a clipped place and
+// dropped: a wait then leaves exactly the younger loads in flight), every word is
+// requested a level ahead, and a level has one barrier.  Measured against guarded
+// loads, the z fluxes' words loaded where they are used and three barriers a level:
+// u 442 -> 333, v 401 -> 340, w 420 -> 410 us at 640x768x80 (flat), 124 -> 78, 120 -> 78
+// and 111 -> 77 at 320x320x80 (terrain).  Six waves per SIMD (three workgroups a CU), where only the u
+// tile spills a few registers; on the terrain family, whose u tile needs more, four
+// waves are faster (82 -> 78 us at 320x320x80; flat, 364 against 333 at 640x768x80).
+constexpr int advu_waves(bool flat) { return flat ? 6 : 4; }
 template <bool FLAT>
-__global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k_mom_advu_tile(MomArgs a, int f0, int nf, int kchunk, int nchunks) {
-  __shared__ float lp[MPS * MNT];      // u: row r = padded row ja + r, col c = padded x fa + c (pitch MPX)
-  __shared__ float lfx[MTY][MTX + 1];  // x flux at centre fa - 1 + t
-  __shared__ float lfy[MTY + 1][MTX];  // y flux at corner row ja + r of face fa + t
+__global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(advu_waves(FLAT)))) void k_mom_advu_tile(MomArgs a, int f0, int nf, int kchunk, int nchunks) {
+  // (plane and fluxes each in two buffers, levels taking turns)
+  __shared__ float lp2[2][MPS * MNT];  // u: row r = padded row ja + r, col c = padded x fa + c (pitch MPX)
+  __shared__ float lfx2[2][MTY][MTX + 1];  // x flux at centre fa - 1 + t
+  __shared__ float lfy2[2][MTY + 1][MTX];  // y flux at corner row ja + r of face fa + t
   __shared__ uint32_t lpo[MPS * MNT];  // plane slot offsets within a level (read back by their own lane)
   __shared__ uint32_t lmo[6][MNT];     // mass-flux pairs: own x centre, own y corner, extra point
   const int ni = a.ni, nj = a.nj, nk = a.nk;
-  const int tx = threadIdx.x % MTX, ty = threadIdx.x / MTX;
+  const int tx = threadIdx.x % MTX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / MTX);  // (a wavefront is one row)
   const int gx = (nf + MTX - 1) / MTX, gy = (nj + MTY - 1) / MTY;
   const int tile = xcd_tile((int)blockIdx.x, gx * gy * nchunks);
   const int fa = f0 + (tile % gx) * MTX, ja = ((tile / gx) % gy) * MTY;
@@ -357,51 +374,71 @@ __global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k
     else lmo[4][threadIdx.x] = lmo[5][threadIdx.x] = 0u;
   }
   // a level's words sit at 32-bit byte offsets from the level's base
-  const uint32_t ocol = (uint32_t)(y * nxu + x) * 4u;  // this face in the u family
+  const uint32_t ocol = live ? (uint32_t)(y * nxu + x) * 4u : 0u;  // this face in the u family
   float win[7];  // u(k-3 .. k+3) of this face's column
 #pragma unroll
   for (int q = 0; q < 7; ++q) {
     const int lev = kb - 3 + q;
     win[q] = (live && lev >= 0 && lev <= nk + 1) ? ldo(a.u + (int64_t)lev * ust, ocol) : 0.0f;
   }
-  auto zf = [&](int kf, const float* b) {  // b[0] = u(kf - 3)
-    return uvz_g<0>(a, kf, j, f, [&](int lev) { return b[lev - (kf - 3)]; });
+  auto zf = [&](int kf, const float* b, const UvzWords& z) {  // b[0] = u(kf - 3)
+    return uvz_g(z, kf, nk, [&](int lev) { return b[lev - (kf - 3)]; });
   };
-  float zlo = (live && kb >= 2) ? zf(kb, win) : 0.0f;
-  // A level's u plane and the rru / rrv pairs its points average are
-  // requested one level ahead into registers (Lv), so they arrive while the
-  // level before it is formed.
+  auto zwords = [&](int kf, float r0, float r1) {
+    UvzWords z{r0, r1, 0.0f, 0.0f};
+    if (kf == 2 || kf == nk) uvz_c2<0>(a, kf, j, f, z);
+    return z;
+  };
+  float zlo = (live && kb >= 2) ? zf(kb, win, uvz_words<0>(a, kb, j, f)) : 0.0f;
+  // the top z face's pair of rrw words
+  const uint32_t oz0 = live ? (uint32_t)((j + NG) * nxv + NG + wc(f, ni, pw, pe)) * 4u : 0u;
+  const uint32_t oz1 = live ? (uint32_t)((j + NG) * nxv + NG + wc(f - 1, ni, pw, pe)) * 4u : 0u;
+  // One barrier a level: a level's fluxes are formed from its u plane while the
+  // plane above it, requested a level earlier, is stored to the other buffer; the
+  // mass-flux pairs (the top z face's included) are requested a level ahead too.
+  // the scalar cells west and east of the face
+  const uint32_t olo = live ? (uint32_t)(j * ni + wc(f - 1, ni, pw, pe)) * 4u : 0u;
+  const uint32_t ohi = live ? (uint32_t)(j * ni + wc(f, ni, pw, pe)) * 4u : 0u;
+  const float gzl = (!FLAT && live) ? a.gzu[(int64_t)j * (ni + 1) + f] : 0.0f;
   struct Lv {
-    float plane[MPS], m[6];
+    float m[6];
     float unext;
+    float z0, z1;
+  };
+  float pln[MPS];  // a plane in flight
+  auto fetch_plane = [&](int k) {
+    const float* plane = a.u + (int64_t)k * ust;
+#pragma unroll
+    for (int q = 0; q < MPS; ++q) pln[q] = ldo(plane, lpo[threadIdx.x + q * MNT]);
+  };
+  auto store_plane = [&](int k) {
+#pragma unroll
+    for (int q = 0; q < MPS; ++q) lp2[k & 1][threadIdx.x + q * MNT] = pln[q];
   };
   auto fetch = [&](int k) {
     Lv v;
     const int lnext = k + 4;
-    v.unext = (live && lnext <= nk + 1) ? ldo(a.u + (int64_t)lnext * ust, ocol) : 0.0f;
-    const float* plane = a.u + (int64_t)k * ust;
-#pragma unroll
-    for (int q = 0; q < MPS; ++q) v.plane[q] = ldo(plane, lpo[threadIdx.x + q * MNT]);
+    v.unext = ldo(a.u + (int64_t)min(lnext, nk + 1) * ust, ocol);
+    const float* Rw = a.rrw + (int64_t)min(k + 1, nk) * nyu * nxv;
+    v.z0 = ldo(Rw, oz0);
+    v.z1 = ldo(Rw, oz1);
     const float* Ru = a.rru + (int64_t)k * ust;
     const float* Rv = a.rrv + (int64_t)k * vst;
     v.m[0] = ldo(Ru, lmo[0][threadIdx.x]);
     v.m[1] = ldo(Ru, lmo[1][threadIdx.x]);
     v.m[2] = ldo(Rv, lmo[2][threadIdx.x]);
     v.m[3] = ldo(Rv, lmo[3][threadIdx.x]);
-    v.m[4] = v.m[5] = 0.0f;
-    if (xe || yn) {
-      const float* R = xe ? Ru : Rv;
-      v.m[4] = ldo(R, lmo[4][threadIdx.x]);
-      v.m[5] = ldo(R, lmo[5][threadIdx.x]);
-    }
+    const float* R = xe ? Ru : Rv;
+    v.m[4] = ldo(R, lmo[4][threadIdx.x]);
+    v.m[5] = ldo(R, lmo[5][threadIdx.x]);
     return v;
   };
   // x point (row r, centre fa-1+t): the mean of the two rru faces times u's
   // fifth-order upwind value
-  auto xflux = [&](int r, int t, float m0, float m1) {
+  auto xflux = [&](int k, int r, int t, float m0, float m1) {
     const float m = 0.5f * (m0 + m1);
-    const float* L = lp + (r + 3) * MPX + t;  // L[c] = u at padded x (cc + NG) - 2 + c
-    lfx[r][t] = point_flux(m, L[0], L[1], L[2], L[3], L[4], L[5]);
+    const float* L = lp2[k & 1] + (r + 3) * MPX + t;  // L[c] = u at padded x (cc + NG) - 2 + c
+    lfx2[k & 1][r][t] = point_flux(m, L[0], L[1], L[2], L[3], L[4], L[5]);
   };
   // y point (corner row p = ja+r of face ff = fa+t); on an open south/north
   // side an inflowing edge corner takes the next row's flux
@@ -421,49 +458,49 @@ __global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k
                                 ldo(Rb, (uint32_t)(rb + wc(ff - 1, ni, pw, pe)) * 4u))
                       : 0.0f;
     }
-    const float* L = lp + (pb - ja) * MPX + t + 3;  // u at padded row pb + NG - 3 + q
-    lfy[r][t] = point_flux(m, L[0], L[MPX], L[2 * MPX], L[3 * MPX], L[4 * MPX], L[5 * MPX]);
+    const float* L = lp2[k & 1] + (pb - ja) * MPX + t + 3;  // u at padded row pb + NG - 3 + q
+    lfy2[k & 1][r][t] = point_flux(m, L[0], L[MPX], L[2 * MPX], L[3 * MPX], L[4 * MPX], L[5 * MPX]);
   };
+  fetch_plane(kb);
   Lv nx = fetch(kb);
+  store_plane(kb);
+  fetch_plane(min(kb + 1, ke));
+  __syncthreads();
   for (int k = kb; k <= ke; ++k) {
+    const auto& lfx = lfx2[k & 1];
+    const auto& lfy = lfy2[k & 1];
     const Lv cu = nx;
-    if (k < ke) nx = fetch(k + 1);
-    const float unext = cu.unext;
     // this level's point words, requested before its fluxes are formed
     float e_dxe = 0.0f, e_dxw = 0.0f, e_sc0 = 0.0f, e_rw = 0.0f, e_re = 0.0f, e_ten = 0.0f;
-    if (live) {
-      const int west = wc(f - 1, ni, pw, pe), east = wc(f, ni, pw, pe);
-      const int64_t lm = (int64_t)(k - 1) * mst;
-      const uint32_t ow = (uint32_t)(j * ni + west) * 4u, oe = (uint32_t)(j * ni + east) * 4u;
-      e_dxe = ldo(a.divx + lm, oe);
-      e_dxw = ldo(a.divx + lm, ow);
-      if (FLAT) {
-        e_sc0 = a.rr0[lm];
-      } else {
-        e_sc0 = a.gzu[(int64_t)j * (ni + 1) + f];
-        e_rw = ldo(a.rho0 + lm, ow);
-        e_re = ldo(a.rho0 + lm, oe);
-      }
-      e_ten = a.zero_held ? 0.0f : ldo((a.u1 ? a.u1 : a.uten) + (int64_t)k * ust, ocol);
+    const int64_t lm = (int64_t)(k - 1) * mst;
+    e_dxe = ldo(a.divx + lm, ohi);
+    e_dxw = ldo(a.divx + lm, olo);
+    if (FLAT) {
+      e_sc0 = a.rr0[lm];
+    } else {
+      e_sc0 = gzl;
+      e_rw = ldo(a.rho0 + lm, olo);
+      e_re = ldo(a.rho0 + lm, ohi);
     }
-#pragma unroll
-    for (int q = 0; q < MPS; ++q) lp[threadIdx.x + q * MNT] = cu.plane[q];
-    __syncthreads();
-    xflux(ty, tx, cu.m[0], cu.m[1]);
+    e_ten = ldo((a.zero_held ? a.u : a.u1 ? a.u1 : a.uten) + (int64_t)k * ust, ocol);  // (unread when the held tendencies are zero)
+    nx = fetch(min(k + 1, ke));
+    xflux(k, ty, tx, cu.m[0], cu.m[1]);
     yflux(k, ty, tx, cu.m[2], cu.m[3]);
     if (xe) {
-      if (tx < MTY) xflux(tx, MTX, cu.m[4], cu.m[5]);
+      if (tx < MTY) xflux(k, tx, MTX, cu.m[4], cu.m[5]);
     } else if (yn) {
       yflux(k, MTY, tx, cu.m[4], cu.m[5]);
     }
     float zhi = 0.0f;
-    if (live && k + 1 <= nk) zhi = zf(k + 1, win + 1);
+    if (live && k + 1 <= nk) zhi = zf(k + 1, win + 1, zwords(k + 1, cu.z0, cu.z1));
+    if (k < ke) store_plane(k + 1);  // (the buffer was last read before the barrier below of the level below)
+    fetch_plane(min(k + 2, ke));
     __syncthreads();
     if (live) {
       const int west = wc(f - 1, ni, pw, pe), east = wc(f, ni, pw, pe);
       float ax = (-(lfx[ty][tx + 1] - lfx[ty][tx])) * a.rdx;
       float ay = (-(lfy[ty + 1][tx] - lfy[ty][tx])) * a.rdy;
-      const float uc = lp[(ty + 3) * MPX + tx + 3];
+      const float uc = win[3];
       if (j == 0 && opn(a.obc, 2)) {
         const float* R0 = a.rrv + ix3(k, NG, 0, nyv, nxv);
         const float* R1 = a.rrv + ix3(k, NG + 1, 0, nyv, nxv);
@@ -490,26 +527,26 @@ __global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k
       float tot = (ax + ay) + az;
       tot = tot + uc * (0.5f * (e_dxe + e_dxw));
       const float sc = FLAT ? e_sc0 : e_sc0 / (0.5f * (e_rw + e_re));
-      sto(a.uten + (int64_t)k * ust, ocol, e_ten + tot * sc);
+      sto(a.uten + (int64_t)k * ust, ocol, (a.zero_held ? 0.0f : e_ten) + tot * sc);
     }
     zlo = zhi;
 #pragma unroll
     for (int q = 0; q < 6; ++q) win[q] = win[q + 1];
-    win[6] = unext;
-    __syncthreads();
+    win[6] = (k + 4 <= nk + 1) ? cu.unext : 0.0f;
   }
 }
 
 // v-momentum: faces g0 .. g0+nr-1 (tile rows), columns 0..ni-1 (tile columns)
 template <bool FLAT>
 __global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k_mom_advv_tile(MomArgs a, int g0, int nr, int kchunk, int nchunks) {
-  __shared__ float lp[MPS * MNT];      // v: row r = padded row ga + r, col c = padded x ia + c (pitch MPX)
-  __shared__ float lfx[MTY][MTX + 1];  // x flux at corner column ia + t of face row ga + r
-  __shared__ float lfy[MTY + 1][MTX];  // y flux at centre ga - 1 + r of column ia + t
+  // (plane and fluxes each in two buffers, levels taking turns)
+  __shared__ float lp2[2][MPS * MNT];  // v: row r = padded row ga + r, col c = padded x ia + c (pitch MPX)
+  __shared__ float lfx2[2][MTY][MTX + 1];  // x flux at corner column ia + t of face row ga + r
+  __shared__ float lfy2[2][MTY + 1][MTX];  // y flux at centre ga - 1 + r of column ia + t
   __shared__ uint32_t lpo[MPS * MNT];  // plane slot offsets within a level (read back by their own lane)
   __shared__ uint32_t lmo[6][MNT];     // mass-flux pairs: own x corner, own y centre, extra point
   const int ni = a.ni, nj = a.nj, nk = a.nk;
-  const int tx = threadIdx.x % MTX, ty = threadIdx.x / MTX;
+  const int tx = threadIdx.x % MTX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / MTX);  // (a wavefront is one row)
   const int gx = (ni + MTX - 1) / MTX, gy = (nr + MTY - 1) / MTY;
   const int tile = xcd_tile((int)blockIdx.x, gx * gy * nchunks);
   const int ia = (tile % gx) * MTX, ga = g0 + ((tile / gx) % gy) * MTY;
@@ -550,42 +587,61 @@ __global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k
     else lmo[4][threadIdx.x] = lmo[5][threadIdx.x] = 0u;
   }
   // a level's words sit at 32-bit byte offsets from the level's base
-  const uint32_t ocol = (uint32_t)(y * nxv + x) * 4u;  // this face in the v family
+  const uint32_t ocol = live ? (uint32_t)(y * nxv + x) * 4u : 0u;  // this face in the v family
   float win[7];
 #pragma unroll
   for (int q = 0; q < 7; ++q) {
     const int lev = kb - 3 + q;
     win[q] = (live && lev >= 0 && lev <= nk + 1) ? ldo(a.v + (int64_t)lev * vst, ocol) : 0.0f;
   }
-  auto zf = [&](int kf, const float* b) {
-    return uvz_g<1>(a, kf, g, i, [&](int lev) { return b[lev - (kf - 3)]; });
+  auto zf = [&](int kf, const float* b, const UvzWords& z) {  // b[0] = v(kf - 3)
+    return uvz_g(z, kf, nk, [&](int lev) { return b[lev - (kf - 3)]; });
   };
-  float zlo = (live && kb >= 2) ? zf(kb, win) : 0.0f;
-  // A level's v plane and the rru / rrv pairs its points average are
-  // requested one level ahead into registers (Lv), as in the u tile.
+  auto zwords = [&](int kf, float r0, float r1) {
+    UvzWords z{r0, r1, 0.0f, 0.0f};
+    if (kf == 2 || kf == nk) uvz_c2<1>(a, kf, g, i, z);
+    return z;
+  };
+  float zlo = (live && kb >= 2) ? zf(kb, win, uvz_words<1>(a, kb, g, i)) : 0.0f;
+  // the top z face's pair of rrw words
+  const uint32_t oz0 = live ? (uint32_t)((wc(g, nj, ps, pn) + NG) * nxv + i + NG) * 4u : 0u;
+  const uint32_t oz1 = live ? (uint32_t)((wc(g - 1, nj, ps, pn) + NG) * nxv + i + NG) * 4u : 0u;
+  // One barrier a level and the words requested a level ahead, as in the u tile.
+  // the scalar cells south and north of the face
+  const uint32_t olo = live ? (uint32_t)(wc(g - 1, nj, ps, pn) * ni + i) * 4u : 0u;
+  const uint32_t ohi = live ? (uint32_t)(wc(g, nj, ps, pn) * ni + i) * 4u : 0u;
+  const float gzl = (!FLAT && live) ? a.gzv[(int64_t)g * ni + i] : 0.0f;
   struct Lv {
-    float plane[MPS], m[6];
+    float m[6];
     float vnext;
+    float z0, z1;
+  };
+  float pln[MPS];  // a plane in flight
+  auto fetch_plane = [&](int k) {
+    const float* plane = a.v + (int64_t)k * vst;
+#pragma unroll
+    for (int q = 0; q < MPS; ++q) pln[q] = ldo(plane, lpo[threadIdx.x + q * MNT]);
+  };
+  auto store_plane = [&](int k) {
+#pragma unroll
+    for (int q = 0; q < MPS; ++q) lp2[k & 1][threadIdx.x + q * MNT] = pln[q];
   };
   auto fetch = [&](int k) {
     Lv v;
     const int lnext = k + 4;
-    v.vnext = (live && lnext <= nk + 1) ? ldo(a.v + (int64_t)lnext * vst, ocol) : 0.0f;
-    const float* plane = a.v + (int64_t)k * vst;
-#pragma unroll
-    for (int q = 0; q < MPS; ++q) v.plane[q] = ldo(plane, lpo[threadIdx.x + q * MNT]);
+    v.vnext = ldo(a.v + (int64_t)min(lnext, nk + 1) * vst, ocol);
+    const float* Rw = a.rrw + (int64_t)min(k + 1, nk) * nyu * nxv;
+    v.z0 = ldo(Rw, oz0);
+    v.z1 = ldo(Rw, oz1);
     const float* Ru = a.rru + (int64_t)k * ust;
     const float* Rv = a.rrv + (int64_t)k * vst;
     v.m[0] = ldo(Ru, lmo[0][threadIdx.x]);
     v.m[1] = ldo(Ru, lmo[1][threadIdx.x]);
     v.m[2] = ldo(Rv, lmo[2][threadIdx.x]);
     v.m[3] = ldo(Rv, lmo[3][threadIdx.x]);
-    v.m[4] = v.m[5] = 0.0f;
-    if (xe || yn) {
-      const float* R = xe ? Ru : Rv;
-      v.m[4] = ldo(R, lmo[4][threadIdx.x]);
-      v.m[5] = ldo(R, lmo[5][threadIdx.x]);
-    }
+    const float* R = xe ? Ru : Rv;
+    v.m[4] = ldo(R, lmo[4][threadIdx.x]);
+    v.m[5] = ldo(R, lmo[5][threadIdx.x]);
     return v;
   };
   // x point (face row gg = ga+r, corner column p = ia+t); on an open
@@ -606,56 +662,56 @@ __global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k
                                 ldo(R, (uint32_t)(rs * nxu + pb + NG) * 4u))
                       : 0.0f;
     }
-    const float* L = lp + (r + 3) * MPX + (pb - ia);  // L[c] = v at padded x (pb + NG) - 3 + c
-    lfx[r][t] = point_flux(m, L[0], L[1], L[2], L[3], L[4], L[5]);
+    const float* L = lp2[k & 1] + (r + 3) * MPX + (pb - ia);  // L[c] = v at padded x (pb + NG) - 3 + c
+    lfx2[k & 1][r][t] = point_flux(m, L[0], L[1], L[2], L[3], L[4], L[5]);
   };
   // y point (centre pc = ga-1+r of column ia+t)
-  auto yflux = [&](int r, int t, float m0, float m1) {
+  auto yflux = [&](int k, int r, int t, float m0, float m1) {
     const float m = 0.5f * (m0 + m1);
     // LDS row of v at padded row (pc + NG) - 2 is pc + 1 - ga = r
-    const float* L = lp + r * MPX + t + 3;
-    lfy[r][t] = point_flux(m, L[0], L[MPX], L[2 * MPX], L[3 * MPX], L[4 * MPX], L[5 * MPX]);
+    const float* L = lp2[k & 1] + r * MPX + t + 3;
+    lfy2[k & 1][r][t] = point_flux(m, L[0], L[MPX], L[2 * MPX], L[3 * MPX], L[4 * MPX], L[5 * MPX]);
   };
+  fetch_plane(kb);
   Lv nx = fetch(kb);
+  store_plane(kb);
+  fetch_plane(min(kb + 1, ke));
+  __syncthreads();
   for (int k = kb; k <= ke; ++k) {
+    const auto& lfx = lfx2[k & 1];
+    const auto& lfy = lfy2[k & 1];
     const Lv cu = nx;
-    if (k < ke) nx = fetch(k + 1);
-    const float vnext = cu.vnext;
     // this level's point words, requested before its fluxes are formed
     float e_dxn = 0.0f, e_dxs = 0.0f, e_sc0 = 0.0f, e_rs = 0.0f, e_rn = 0.0f, e_ten = 0.0f;
-    if (live) {
-      const int south = wc(g - 1, nj, ps, pn), north = wc(g, nj, ps, pn);
-      const int64_t lm = (int64_t)(k - 1) * mst;
-      const uint32_t on = (uint32_t)(north * ni + i) * 4u, os = (uint32_t)(south * ni + i) * 4u;
-      e_dxn = ldo(a.divx + lm, on);
-      e_dxs = ldo(a.divx + lm, os);
-      if (FLAT) {
-        e_sc0 = a.rr0[lm];
-      } else {
-        e_sc0 = a.gzv[(int64_t)g * ni + i];
-        e_rs = ldo(a.rho0 + lm, os);
-        e_rn = ldo(a.rho0 + lm, on);
-      }
-      e_ten = a.zero_held ? 0.0f : ldo((a.v1 ? a.v1 : a.vten) + (int64_t)k * vst, ocol);
+    const int64_t lm = (int64_t)(k - 1) * mst;
+    e_dxn = ldo(a.divx + lm, ohi);
+    e_dxs = ldo(a.divx + lm, olo);
+    if (FLAT) {
+      e_sc0 = a.rr0[lm];
+    } else {
+      e_sc0 = gzl;
+      e_rs = ldo(a.rho0 + lm, olo);
+      e_rn = ldo(a.rho0 + lm, ohi);
     }
-#pragma unroll
-    for (int q = 0; q < MPS; ++q) lp[threadIdx.x + q * MNT] = cu.plane[q];
-    __syncthreads();
+    e_ten = ldo((a.zero_held ? a.v : a.v1 ? a.v1 : a.vten) + (int64_t)k * vst, ocol);  // (unread when the held tendencies are zero)
+    nx = fetch(min(k + 1, ke));
     xflux(k, ty, tx, cu.m[0], cu.m[1]);
-    yflux(ty, tx, cu.m[2], cu.m[3]);
+    yflux(k, ty, tx, cu.m[2], cu.m[3]);
     if (xe) {
       if (tx < MTY) xflux(k, tx, MTX, cu.m[4], cu.m[5]);
     } else if (yn) {
-      yflux(MTY, tx, cu.m[4], cu.m[5]);
+      yflux(k, MTY, tx, cu.m[4], cu.m[5]);
     }
     float zhi = 0.0f;
-    if (live && k + 1 <= nk) zhi = zf(k + 1, win + 1);
+    if (live && k + 1 <= nk) zhi = zf(k + 1, win + 1, zwords(k + 1, cu.z0, cu.z1));
+    if (k < ke) store_plane(k + 1);  // (the buffer was last read before the barrier below of the level below)
+    fetch_plane(min(k + 2, ke));
     __syncthreads();
     if (live) {
       const int south = wc(g - 1, nj, ps, pn), north = wc(g, nj, ps, pn);
       float ax = (-(lfx[ty][tx + 1] - lfx[ty][tx])) * a.rdx;
       float ay = (-(lfy[ty + 1][tx] - lfy[ty][tx])) * a.rdy;
-      const float vc = lp[(ty + 3) * MPX + tx + 3];
+      const float vc = win[3];
       const float* Rs = a.rru + ix3(k, south + NG, 0, nyu, nxu);
       const float* Rn = a.rru + ix3(k, north + NG, 0, nyu, nxu);
       if (i == 0 && opn(a.obc, 0)) {
@@ -679,13 +735,12 @@ __global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6))) void k
       float tot = (ax + ay) + az;
       tot = tot + vc * (0.5f * (e_dxn + e_dxs));
       const float sc = FLAT ? e_sc0 : e_sc0 / (0.5f * (e_rs + e_rn));
-      sto(a.vten + (int64_t)k * vst, ocol, e_ten + tot * sc);
+      sto(a.vten + (int64_t)k * vst, ocol, (a.zero_held ? 0.0f : e_ten) + tot * sc);
     }
     zlo = zhi;
 #pragma unroll
     for (int q = 0; q < 6; ++q) win[q] = win[q + 1];
-    win[6] = vnext;
-    __syncthreads();
+    win[6] = (k + 4 <= nk + 1) ? cu.vnext : 0.0f;
   }
 }
 
@@ -693,7 +748,7 @@ template <bool FLAT>
 void launch_advu_tile(const MomArgs& a, int f0, int nf, hipStream_t s) {
   int kchunk = 1;
   const int tiles = ((nf + MTX - 1) / MTX) * ((a.nj + MTY - 1) / MTY);
-  const int chunks = mom_chunks(tiles, a.nk, &kchunk);
+  const int chunks = tile_chunks(tiles, a.nk, advu_waves(FLAT) / 2, &kchunk);
   GM1_TIMED(TK_MOM_ADVU, s, hipLaunchKernelGGL(k_mom_advu_tile<FLAT>, dim3(tiles * chunks), dim3(MNT), 0, s, a, f0,
                                                nf, kchunk, chunks));
 }
@@ -702,7 +757,7 @@ template <bool FLAT>
 void launch_advv_tile(const MomArgs& a, int g0, int nr, hipStream_t s) {
   int kchunk = 1;
   const int tiles = ((a.ni + MTX - 1) / MTX) * ((nr + MTY - 1) / MTY);
-  const int chunks = mom_chunks(tiles, a.nk, &kchunk);
+  const int chunks = tile_chunks(tiles, a.nk, 3, &kchunk);
   GM1_TIMED(TK_MOM_ADVV, s, hipLaunchKernelGGL(k_mom_advv_tile<FLAT>, dim3(tiles * chunks), dim3(MNT), 0, s, a, g0,
                                                nr, kchunk, chunks));
 }
@@ -716,7 +771,11 @@ GM1_DEV float wz_g(float m, int k, int nk, Get Q) {
   else if (k == 2) r = (m >= 0.0f) ? flx3(Q(1), Q(2), Q(3)) : flx5(Q(5), Q(4), Q(3), Q(2), Q(1));
   else if (k == nk - 1) r = (m >= 0.0f) ? flx5(Q(k - 2), Q(k - 1), Q(k), Q(k + 1), Q(k + 2)) : flx3(Q(k + 2), Q(k + 1), Q(k));
   else if (k == nk) r = (m >= 0.0f) ? flx3(Q(k - 1), Q(k), Q(k + 1)) : 0.5f * (Q(k) + Q(k + 1));
-  else r = (m >= 0.0f) ? flx5(Q(k - 2), Q(k - 1), Q(k), Q(k + 1), Q(k + 2)) : flx5(Q(k + 3), Q(k + 2), Q(k + 1), Q(k), Q(k - 1));
+  else {  // one value of the upwind words, whichever way the lanes' fluxes point
+    const bool up = m >= 0.0f;
+    const float q0 = Q(k - 2), q1 = Q(k - 1), q2 = Q(k), q3 = Q(k + 1), q4 = Q(k + 2), q5 = Q(k + 3);
+    r = flx5(up ? q0 : q5, up ? q1 : q4, up ? q2 : q3, up ? q3 : q2, up ? q4 : q1);
+  }
   return m * r;
 }
 
@@ -735,16 +794,16 @@ GM1_DEV float wz_g(float m, int k, int nk, Get Q) {
 constexpr int WLX = MTX + 6, WLY = MTY + 6, WCX = MTX + 2;
 constexpr int WPS = (WLY * WLX + MNT - 1) / MNT, WCS = ((MTY + 2) * WCX + MNT - 1) / MNT;
 template <bool FLAT>
-// (registers held to four waves per SIMD: two 512-lane workgroups per CU)
-__global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ __launch_bounds__(MNT) __attribute__((amdgpu_waves_per_eu(6)))
 void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
-  __shared__ float lw[WPS * MNT];           // w: row r = padded row ja + r, col c = padded x ia + c (pitch WLX)
-  __shared__ float lc[WCS * MNT];           // c2 of cells (clamp(ja-1+r), clamp(ia-1+c)) at level kf-1 (pitch WCX)
-  __shared__ float lfx[MTY][MTX + 1], lmx[MTY][MTX + 1];  // x flux and mass flux at face ia + t
-  __shared__ float lfy[MTY + 1][MTX], lmy[MTY + 1][MTX];  // y flux and mass flux at face ja + r
+  // (planes and fluxes each in two buffers, levels taking turns)
+  __shared__ float lw2[2][WPS * MNT];       // w: row r = padded row ja + r, col c = padded x ia + c (pitch WLX)
+  __shared__ float lc2[2][WCS * MNT];       // c2 of cells (clamp(ja-1+r), clamp(ia-1+c)) at level kf-1 (pitch WCX)
+  __shared__ float lfx2[2][MTY][MTX + 1], lmx2[2][MTY][MTX + 1];  // x flux and mass flux at face ia + t
+  __shared__ float lfy2[2][MTY + 1][MTX], lmy2[2][MTY + 1][MTX];  // y flux and mass flux at face ja + r
   __shared__ uint32_t lpo[WPS * MNT], lco[WCS * MNT];     // slot offsets (read back by their own lane)
   const int ni = a.ni, nj = a.nj, nk = a.nk;
-  const int tx = threadIdx.x % MTX, ty = threadIdx.x / MTX;
+  const int tx = threadIdx.x % MTX, ty = __builtin_amdgcn_readfirstlane(threadIdx.x / MTX);  // (a wavefront is one row)
   const int gx = (ni + MTX - 1) / MTX, gy = (nj + MTY - 1) / MTY;
   const int tile = xcd_tile((int)blockIdx.x, gx * gy * nchunks);
   const int ia = (tile % gx) * MTX, ja = ((tile / gx) % gy) * MTY;
@@ -758,10 +817,10 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
   const int64_t h = (int64_t)j * ni + i;
   const bool xe = (ty == MTY - 1), yn = (ty == MTY - 2);  // the wavefronts forming the extra faces
   // a level's words sit at 32-bit byte offsets from the level's base
-  const uint32_t oh = (uint32_t)(j * ni + i) * 4u, ow = (uint32_t)(y * nxs + x) * 4u;
+  const uint32_t oh = live ? (uint32_t)(j * ni + i) * 4u : 0u, ow = live ? (uint32_t)(y * nxs + x) * 4u : 0u;
   // the lane's faces: west x face (i, j), south y face (i, j), and the extra face
   const uint32_t orx = (j < nj && i <= ni) ? (uint32_t)(y * nxu + x) * 4u : 0u;
-  const uint32_t ory = (i < ni && j <= nj) ? ow : 0u;
+  const uint32_t ory = (i < ni && j <= nj) ? (uint32_t)(y * nxs + x) * 4u : 0u;
   uint32_t ore = 0u;
   if (xe && tx < MTY && ja + tx < nj && ia + MTX <= ni) ore = (uint32_t)((ja + tx + NG) * nxu + ia + MTX + NG) * 4u;
   if (yn && ja + MTY <= nj && i < ni) ore = (uint32_t)((ja + MTY + NG) * nxs + x) * 4u;
@@ -798,73 +857,88 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
     dxlo = ldo(a.divx + (int64_t)(kb - 2) * plane, oh);
     if (FLAT && a.dum8) d8lo = ldo(a.dum8 + (int64_t)(kb - 1) * wst, ow);
   }
+  const float uhx = live ? a.uh[x] : 0.0f, vhy = live ? a.vh[y] : 0.0f;
+  const float gzc = (!FLAT && live) ? a.gz[h] : 0.0f;
   struct Lv {
-    float plane[WPS], c2[WCS];
     float rx, ry, re;
-    float wnext, rrwn, divx, base, d8, c1;
+    float wnext, rrwn, divx, base, d8, c1, rrf0;
+  };
+  // one barrier a level, as in the u and v tiles: the planes above are stored while
+  // a level's fluxes are formed
+  float pln[WPS], pc2[WCS];  // planes in flight
+  auto fetch_plane = [&](int kf) {
+    const float* wp = a.w + (int64_t)kf * wst;
+#pragma unroll
+    for (int q = 0; q < WPS; ++q) pln[q] = ldo(wp, lpo[threadIdx.x + q * MNT]);
+    const float* c2k = a.c2 + (int64_t)(kf - 1) * plane;
+#pragma unroll
+    for (int q = 0; q < WCS; ++q) pc2[q] = ldo(c2k, lco[threadIdx.x + q * MNT]);
+  };
+  auto store_plane = [&](int kf) {
+#pragma unroll
+    for (int q = 0; q < WPS; ++q) lw2[kf & 1][threadIdx.x + q * MNT] = pln[q];
+#pragma unroll
+    for (int q = 0; q < WCS; ++q) lc2[kf & 1][threadIdx.x + q * MNT] = pc2[q];
   };
   auto fetch = [&](int kf) {
     Lv v;
-    const float* wp = a.w + (int64_t)kf * wst;
-#pragma unroll
-    for (int q = 0; q < WPS; ++q) v.plane[q] = ldo(wp, lpo[threadIdx.x + q * MNT]);
-    const float* c2k = a.c2 + (int64_t)(kf - 1) * plane;
-#pragma unroll
-    for (int q = 0; q < WCS; ++q) v.c2[q] = ldo(c2k, lco[threadIdx.x + q * MNT]);
     v.rx = rface(kf, orx, true);
     v.ry = rface(kf, ory, false);
-    v.re = (xe || yn) ? rface(kf, ore, xe) : 0.0f;
-    v.wnext = v.rrwn = v.divx = v.base = v.d8 = v.c1 = 0.0f;
-    if (live) {
-      const int lnext = kf + 4;
-      v.wnext = (lnext <= nk + 2) ? ldo(a.w + (int64_t)lnext * wst, ow) : 0.0f;
-      v.rrwn = ldo(a.rrw + (int64_t)(kf + 1) * wst, ow);
-      v.divx = ldo(a.divx + (int64_t)(kf - 1) * plane, oh);
-      v.base = a.zero_held ? 0.0f : ldo((a.w1 ? a.w1 : a.wten) + (int64_t)kf * wst, ow);
-      if (FLAT && a.dum8) {
-        v.d8 = ldo(a.dum8 + (int64_t)kf * wst, ow);
-        v.c1 = ldo(a.c1 + (int64_t)(kf - 1) * plane, oh);
-      }
+    v.re = ldo(xe ? a.rru + (int64_t)kf * ust : a.rrv + (int64_t)kf * vst, ore);
+    v.wnext = ldo(a.w + (int64_t)min(kf + 4, nk + 2) * wst, ow);
+    v.rrwn = ldo(a.rrw + (int64_t)(kf + 1) * wst, ow);
+    v.divx = ldo(a.divx + (int64_t)(kf - 1) * plane, oh);
+    v.base = ldo((a.zero_held ? a.w : a.w1 ? a.w1 : a.wten) + (int64_t)kf * wst, ow);  // (unread when the held tendencies are zero)
+    v.d8 = v.c1 = v.rrf0 = 0.0f;
+    if (!FLAT) v.rrf0 = ldo(a.rrf0 + (int64_t)(kf - 1) * plane, oh);
+    if (FLAT) {  // (dum8 and c1 unread without a dum8)
+      v.d8 = ldo((a.dum8 ? a.dum8 : a.rrw) + (int64_t)kf * wst, ow);
+      v.c1 = ldo((a.dum8 ? a.c1 : a.divx) + (int64_t)(kf - 1) * plane, oh);
     }
     return v;
   };
   // x face ia + t of row ja + r (wfx_base)
-  auto xface = [&](int r, int t, float mt, float mb) {
-    const float c2h = 0.5f * (lc[(r + 1) * WCX + t] + lc[(r + 1) * WCX + t + 1]);
+  auto xface = [&](int b, int r, int t, float mt, float mb) {
+    const float c2h = 0.5f * (lc2[b][(r + 1) * WCX + t] + lc2[b][(r + 1) * WCX + t + 1]);
     const float c1h = 1.0f - c2h;
     const float m = c2h * mt + c1h * mb;
-    const float* L = lw + (r + 3) * WLX + t;  // L[c] = w at padded x (ia + t + NG) - 3 + c
-    lfx[r][t] = point_flux(m, L[0], L[1], L[2], L[3], L[4], L[5]);
-    lmx[r][t] = m;
+    const float* L = lw2[b] + (r + 3) * WLX + t;  // L[c] = w at padded x (ia + t + NG) - 3 + c
+    lfx2[b][r][t] = point_flux(m, L[0], L[1], L[2], L[3], L[4], L[5]);
+    lmx2[b][r][t] = m;
   };
   // y face ja + r of column ia + t (wfy_base)
-  auto yface = [&](int r, int t, float mt, float mb) {
-    const float c2h = 0.5f * (lc[r * WCX + t + 1] + lc[(r + 1) * WCX + t + 1]);
+  auto yface = [&](int b, int r, int t, float mt, float mb) {
+    const float c2h = 0.5f * (lc2[b][r * WCX + t + 1] + lc2[b][(r + 1) * WCX + t + 1]);
     const float c1h = 1.0f - c2h;
     const float m = c2h * mt + c1h * mb;
-    const float* L = lw + r * WLX + t + 3;
-    lfy[r][t] = point_flux(m, L[0], L[WLX], L[2 * WLX], L[3 * WLX], L[4 * WLX], L[5 * WLX]);
-    lmy[r][t] = m;
+    const float* L = lw2[b] + r * WLX + t + 3;
+    lfy2[b][r][t] = point_flux(m, L[0], L[WLX], L[2 * WLX], L[3 * WLX], L[4 * WLX], L[5 * WLX]);
+    lmy2[b][r][t] = m;
   };
   const bool pw = opn(a.obc, 0), pe = opn(a.obc, 1), ps = opn(a.obc, 2), pn = opn(a.obc, 3);
+  fetch_plane(kb);
   Lv nx = fetch(kb);
+  store_plane(kb);
+  fetch_plane(min(kb + 1, ke));
+  __syncthreads();
   for (int kf = kb; kf <= ke; ++kf) {
+    const int b = kf & 1;
+    const auto &lfx = lfx2[b], &lmx = lmx2[b];
+    const auto &lfy = lfy2[b], &lmy = lmy2[b];
     const Lv cu = nx;
-    if (kf < ke) nx = fetch(kf + 1);
-#pragma unroll
-    for (int q = 0; q < WPS; ++q) lw[threadIdx.x + q * MNT] = cu.plane[q];
-#pragma unroll
-    for (int q = 0; q < WCS; ++q) lc[threadIdx.x + q * MNT] = cu.c2[q];
-    __syncthreads();
-    xface(ty, tx, cu.rx, rxp);
-    yface(ty, tx, cu.ry, ryp);
+    nx = fetch(min(kf + 1, ke));
+    xface(b, ty, tx, cu.rx, rxp);
+    yface(b, ty, tx, cu.ry, ryp);
     if (xe) {
-      if (tx < MTY) xface(tx, MTX, cu.re, rep);
+      if (tx < MTY) xface(b, tx, MTX, cu.re, rep);
     } else if (yn) {
-      yface(MTY, tx, cu.re, rep);
+      yface(b, MTY, tx, cu.re, rep);
     }
+    const float c2 = lc2[b][(ty + 1) * WCX + tx + 1];
     float zhi = 0.0f;
     if (live) zhi = wz_g(0.5f * (rrw_hi + cu.rrwn), kf, nk, [&](int lev) { return win[lev - (kf - 3)]; });
+    if (kf < ke) store_plane(kf + 1);
+    fetch_plane(min(kf + 2, ke));
     __syncthreads();
     if (live) {
       // the open sides take the neighbouring face's flux where the mass flux points inward
@@ -876,13 +950,12 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
       if (j == nj - 1 && pn && lmy[ty + 1][tx] <= 0.0f) fn = lfy[ty][tx];
       float ax, ay;
       if (FLAT) {
-        ax = ((-(fe - fw)) * a.rdx) * a.uh[x];
-        ay = ((-(fn - fs)) * a.rdy) * a.vh[y];
+        ax = ((-(fe - fw)) * a.rdx) * uhx;
+        ay = ((-(fn - fs)) * a.rdy) * vhy;
       } else {
-        ax = (-(fe - fw)) * (a.rdx * a.uh[x]);
-        ay = (-(fn - fs)) * (a.rdy * a.vh[y]);
+        ax = (-(fe - fw)) * (a.rdx * uhx);
+        ay = (-(fn - fs)) * (a.rdy * vhy);
       }
-      const float c2 = lc[(ty + 1) * WCX + tx + 1];
       const float c1 = 1.0f - c2;
       const float wc0 = win[3];
       if (i == 0 && pw) {
@@ -891,7 +964,7 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
         const float m = c2 * Rt[NG] + c1 * Rb[NG];
         if (m >= 0.0f) {
           const float c = c1 * (Rb[NG + 1] - Rb[NG]) + c2 * (Rt[NG + 1] - Rt[NG]);
-          ax = FLAT ? ax - ((wc0 * c) * a.rdx) * a.uh[x] : ax - wc0 * (c * (a.rdx * a.uh[x]));
+          ax = FLAT ? ax - ((wc0 * c) * a.rdx) * uhx : ax - wc0 * (c * (a.rdx * uhx));
         }
       } else if (i == ni - 1 && pe) {
         const float* Rt = a.rru + ix3(kf, y, 0, nyu, nxu);
@@ -899,7 +972,7 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
         const float m = c2 * Rt[NG + ni] + c1 * Rb[NG + ni];
         if (m <= 0.0f) {
           const float c = c1 * (Rb[x + 1] - Rb[x]) + c2 * (Rt[x + 1] - Rt[x]);
-          ax = FLAT ? ax - ((wc0 * c) * a.rdx) * a.uh[x] : ax - wc0 * (c * (a.rdx * a.uh[x]));
+          ax = FLAT ? ax - ((wc0 * c) * a.rdx) * uhx : ax - wc0 * (c * (a.rdx * uhx));
         }
       }
       if (j == 0 && ps) {
@@ -907,14 +980,14 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
         if (m >= 0.0f) {
           const float c = c1 * (a.rrv[ix3(kf - 1, NG + 1, x, nyv, nxs)] - a.rrv[ix3(kf - 1, NG, x, nyv, nxs)]) +
                           c2 * (a.rrv[ix3(kf, NG + 1, x, nyv, nxs)] - a.rrv[ix3(kf, NG, x, nyv, nxs)]);
-          ay = FLAT ? ay - ((wc0 * c) * a.rdy) * a.vh[y] : ay - wc0 * (c * (a.rdy * a.vh[y]));
+          ay = FLAT ? ay - ((wc0 * c) * a.rdy) * vhy : ay - wc0 * (c * (a.rdy * vhy));
         }
       } else if (j == nj - 1 && pn) {
         const float m = c2 * a.rrv[ix3(kf, NG + nj, x, nyv, nxs)] + c1 * a.rrv[ix3(kf - 1, NG + nj, x, nyv, nxs)];
         if (m <= 0.0f) {
           const float c = c1 * (a.rrv[ix3(kf - 1, y + 1, x, nyv, nxs)] - a.rrv[ix3(kf - 1, y, x, nyv, nxs)]) +
                           c2 * (a.rrv[ix3(kf, y + 1, x, nyv, nxs)] - a.rrv[ix3(kf, y, x, nyv, nxs)]);
-          ay = FLAT ? ay - ((wc0 * c) * a.rdy) * a.vh[y] : ay - wc0 * (c * (a.rdy * a.vh[y]));
+          ay = FLAT ? ay - ((wc0 * c) * a.rdy) * vhy : ay - wc0 * (c * (a.rdy * vhy));
         }
       }
       float az = (-(zhi - zlo)) * a.rdz;
@@ -922,9 +995,9 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
       float tot = (ax + ay) + az;
       tot = tot + wc0 * (c2 * cu.divx + c1 * dxlo);
       const float sc = FLAT ? a.rrf0[(int64_t)(kf - 1) * plane]
-                            : ldo(a.rrf0 + (int64_t)(kf - 1) * plane, oh) * a.gz[h];
+                            : cu.rrf0 * gzc;
       float* wt_k = a.wten + (int64_t)kf * wst;
-      const float wt = cu.base + tot * sc;
+      const float wt = (a.zero_held ? 0.0f : cu.base) + tot * sc;
       if (FLAT && a.dum8) sto(wt_k, ow, wt + (cu.c1 * d8lo + c2 * cu.d8));
       else sto(wt_k, ow, wt);
       d8lo = cu.d8;
@@ -937,8 +1010,7 @@ void k_mom_advw_tile(MomArgs a, int kchunk, int nchunks) {
     rep = cu.re;
 #pragma unroll
     for (int q = 0; q < 6; ++q) win[q] = win[q + 1];
-    win[6] = cu.wnext;
-    __syncthreads();
+    win[6] = (kf + 4 <= nk + 2) ? cu.wnext : 0.0f;
   }
 }
 
@@ -946,7 +1018,7 @@ template <bool FLAT>
 void launch_advw_tile(const MomArgs& a, hipStream_t s) {
   int kchunk = 1;
   const int tiles = ((a.ni + MTX - 1) / MTX) * ((a.nj + MTY - 1) / MTY);
-  const int chunks = mom_chunks(tiles, a.nk - 1, &kchunk);
+  const int chunks = tile_chunks(tiles, a.nk - 1, 3, &kchunk);
   GM1_TIMED(TK_MOM_ADVW, s, hipLaunchKernelGGL(k_mom_advw_tile<FLAT>, dim3(tiles * chunks), dim3(MNT), 0, s, a,
                                                kchunk, chunks));
 }
