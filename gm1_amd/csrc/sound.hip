@@ -937,54 +937,106 @@ GM1_DEV void average_uv_faces(const SoundArgs& a, const float* __restrict__ u3, 
 
 // sound.F's tridiagonal solve of one column for w(2..nk) over LDS planes of
 // C2W columns: forward elimination into ec (over mm) and ed (over dd), then
-// back substitution into dd.  The next level's LDS words are fetched while
-// the current level's division runs; s1/s2 of the level below are carried.
-template <int C2W>
+// back substitution into dd.  One lane a column, so its time is the chain of a
+// product, a sum, a division and a product a level: the rows aa, bb, -cc of the
+// next G levels are formed, and the words of the G after them read, between the
+// chain's operations, in straight code (no branch a level).  Against forming a
+// level's row inside its own step of the chain: a step of 203x149x57 2470 -> 2407 us,
+// of 320x320x80 (terrain) 9.10 -> 8.82 ms.  The flat pass's 80 registers hold
+// G = 1 (G = 4 spills there: 34.2 -> 35.7 ms a step at 640x768x80); G = 2 and 4
+// measured the same in the terrain pass.  Slower: a reciprocal by two fused Newton
+// steps (exact on every word of its range, but a branch guards the range), the rows
+// formed by all slots before the solve (a barrier and spills more), a raised
+// wave priority during it.
+template <int C2W, int G>
 GM1_DEV void thomas_column(const float* Ls1, const float* Ls2, float* Lmm, float* Ldd, int c, int nk, float asq) {
   auto at = [&](int k) { return k * C2W + c; };
-  float ec_prev = 0.0f, ed_prev = 0.0f, wtop = 0.0f;
+  struct Row {
+    float aa, bb, nc, dd;
+  };
+  struct Raw {
+    float mm, s1, s2, dd;
+  };
+  auto raw = [&](int k) {  // (levels past the top read the top's words, which no row takes)
+    const int q = at(min(k, nk));
+    return Raw{Lmm[q], Ls1[q], Ls2[q], Ldd[q]};
+  };
   float s1m = Ls1[at(1)], s2m = Ls2[at(1)];
-  float mmn = Lmm[at(2)], s1n = Ls1[at(2)], s2n = Ls2[at(2)], ddn = Ldd[at(2)];
-  for (int k = 2; k <= nk; ++k) {
-    const float mmk = mmn, s1k = s1n, s2k = s2n, dd = ddn;
-    if (k < nk) {
-      mmn = Lmm[at(k + 1)];
-      s1n = Ls1[at(k + 1)];
-      s2n = Ls2[at(k + 1)];
-      ddn = Ldd[at(k + 1)];
+  auto row = [&](const Raw& x, int k) {  // level k's row of the system (-cc in place of cc); levels in order
+    const float aa = (k >= 3) ? (-asq) * (x.mm * s1m) : 0.0f;
+    const float cc = (k < nk) ? (-asq) * ((-x.mm) * x.s2) : 0.0f;
+    const float diag = (-x.s1) + s2m;
+    s1m = x.s1;
+    s2m = x.s2;
+    return Row{aa, 1.0f - asq * (x.mm * diag), -cc, x.dd};
+  };
+  Row r[G];
+  Raw x[G];
+#pragma unroll
+  for (int u = 0; u < G; ++u) x[u] = raw(2 + u);
+#pragma unroll
+  for (int u = 0; u < G; ++u) r[u] = row(x[u], 2 + u);
+#pragma unroll
+  for (int u = 0; u < G; ++u) x[u] = raw(2 + G + u);
+  float ec = 0.0f, ed = 0.0f;  // (the first row's aa is 0, and 0*0 + bb = bb)
+  int k = 2;
+  for (; k + G - 1 <= nk; k += G) {
+    Raw y[G];
+    Row t[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) y[u] = raw(k + 2 * G + u);
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      const float inv = 1.0f / (r[u].aa * ec + r[u].bb);
+      ec = r[u].nc * inv;
+      ed = (r[u].dd - r[u].aa * ed) * inv;
+      Lmm[at(k + u)] = ec;
+      Ldd[at(k + u)] = ed;
+      t[u] = row(x[u], k + G + u);
     }
-    const float aa = (k >= 3) ? (-asq) * (mmk * s1m) : 0.0f;
-    const float cc = (k < nk) ? (-asq) * ((-mmk) * s2k) : 0.0f;
-    const float diag = (-s1k) + s2m;
-    const float bb = 1.0f - asq * (mmk * diag);
-    const float pivot = (k == 2) ? bb : aa * ec_prev + bb;
-    const float inv = 1.0f / pivot;
-    if (k < nk) {
-      const float eck = (-cc) * inv;
-      const float edk = ((k == 2) ? dd : dd - aa * ed_prev) * inv;
-      Lmm[at(k)] = eck;
-      Ldd[at(k)] = edk;
-      ec_prev = eck;
-      ed_prev = edk;
-    } else {
-      wtop = (dd - aa * ed_prev) * inv;
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      r[u] = t[u];
+      x[u] = y[u];
     }
-    s1m = s1k;
-    s2m = s2k;
   }
-  float wup = wtop;
-  Ldd[at(nk)] = wtop;
-  float ecn = Lmm[at(nk - 1)], edn = Ldd[at(nk - 1)];
-  for (int k = nk - 1; k >= 2; --k) {
-    const float eck = ecn, edk = edn;
-    if (k > 2) {
-      ecn = Lmm[at(k - 1)];
-      edn = Ldd[at(k - 1)];
+#pragma unroll
+  for (int u = 0; u < G - 1; ++u)
+    if (k + u <= nk) {
+      const float inv = 1.0f / (r[u].aa * ec + r[u].bb);
+      ec = r[u].nc * inv;
+      ed = (r[u].dd - r[u].aa * ed) * inv;
+      Lmm[at(k + u)] = ec;
+      Ldd[at(k + u)] = ed;
     }
-    const float wk = eck * wup + edk;
-    Ldd[at(k)] = wk;
-    wup = wk;
+  float w = ed;  // w(nk)
+  float e[G], d[G];
+#pragma unroll
+  for (int u = 0; u < G; ++u) {
+    e[u] = Lmm[at(max(nk - 1 - u, 2))];
+    d[u] = Ldd[at(max(nk - 1 - u, 2))];
   }
+  for (k = nk - 1; k - G + 1 >= 2; k -= G) {
+    float en[G], dn[G];
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      en[u] = Lmm[at(max(k - G - u, 2))];
+      dn[u] = Ldd[at(max(k - G - u, 2))];
+    }
+#pragma unroll
+    for (int u = 0; u < G; ++u) {
+      w = e[u] * w + d[u];
+      Ldd[at(k - u)] = w;
+      e[u] = en[u];
+      d[u] = dn[u];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < G - 1; ++u)
+    if (k - u >= 2) {
+      w = e[u] * w + d[u];
+      Ldd[at(k - u)] = w;
+    }
 }
 
 template <int C2W, int C2T, bool FLAT, bool PIPE, bool FUSE>
@@ -1523,7 +1575,7 @@ __device__ __forceinline__ void column2_body(const SoundArgs& a, int n, int tile
   }
   __syncthreads();
   // ---------------- phase B: Thomas recurrence, one lane per column
-  if (phys && slot == 0) thomas_column<C2W>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
+  if (phys && slot == 0) thomas_column<C2W, 1>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
   if constexpr (PIPE) {
     // while lane group 0 runs the recurrence, the level slots of the other
     // wavefronts add the u and v faces of every column of the tile into their
@@ -1634,7 +1686,10 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(4))) void k
 // read and one write of rru, rrv per two steps, where this pass moved them every
 // step), and this pass makes the open sides' next step: at 640x768x80 this pass
 // 816 -> 645 us and the pressure gradient 244 -> 302 us a small step, with no
-// open-side and ring-fill launches between small steps (9 + 6 us).
+// open-side and ring-fill launches between small steps (9 + 6 us).  Words a wait
+// needs are never younger than words it does not (piadv of the level above comes
+// with a level's own words, the rrw words behind the recurrence), and at 65..80
+// levels a slot holds five: 645 -> 600 us with the recurrence's straight code.
 constexpr int C3PLANES = 4;
 
 int column3_lds_bytes(int nk, int cw, int slots) {
@@ -1704,9 +1759,10 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
     const float* wi = a.w_in ? a.w_in : w;
     if (kb == 1) lw1[c] = wi[wst + wc];
     struct In {
-      float uw, ue, vs, vn, pc, pe, pw, pn, ps, wup, wt, ppten, ppterm, pp, th;
+      float uw, ue, vs, vn, pup, pe, pw, pn, ps, wup, wt, ppten, ppterm, pp, th;
     };
-    const uint32_t onp = (uint32_t)(ni + 2) * 4u, onx = (uint32_t)nxs * 4u, ows = (uint32_t)wst * 4u;
+    const uint32_t onp = (uint32_t)(ni + 2) * 4u, onx = (uint32_t)nxs * 4u, ows = (uint32_t)wst * 4u,
+                   ops = (uint32_t)((ni + 2) * (nj + 2)) * 4u;
     const float* pp_in = (first && a.nrk != 1) ? a.ppi : a.pp3d;  // the first small step reads ppi
     auto load = [&](int k) {
       const uint32_t op = (uint32_t)pix(k, pj, pi, ni, nj) * 4u;
@@ -1718,7 +1774,7 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
       v.ue = ldo(a.u3d, ou + 4u);
       v.vs = ldo(a.v3d, ov);
       v.vn = ldo(a.v3d, ov + onx);
-      v.pc = ldo(a.piadv, op);
+      v.pup = ldo(a.piadv, op + ops);
       v.pe = ldo(a.piadv, op + 4u);
       v.pw = ldo(a.piadv, op - 4u);
       v.pn = ldo(a.piadv, op + onp);
@@ -1733,23 +1789,24 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
     };
     float wraw = wi[(int64_t)kb * wst + wc];
     const int64_t pb = pix(kb - 1, pj, pi, ni, nj);
-    float pd = a.piadv[pb], thm = a.thv[pb];
+    float pd = a.piadv[pb], thm = a.thv[pb], pc = ldo(a.piadv, (uint32_t)pb * 4u + ops);
     In nx = load(kb);
 #pragma unroll
     for (int kk = 0; kk < CH; ++kk) {
       const int k = kb + kk;
       if (k <= ke) {
         const In cu = nx;
-        nx = load(k + 1);  // level nk+1 exists in every array read here
+        nx = load(min(k + 1, ke));  // (unguarded: a guarded load would make the wait for cu's words a wait for all)
         float div = (cu.ue - cu.uw) * a.rdx + (cu.vn - cu.vs) * a.rdy;
         if (fabsf(div) < smeps) div = 0.0f;
-        float hx = cu.uw * (cu.pc - cu.pw) + cu.ue * (cu.pe - cu.pc);
+        float hx = cu.uw * (pc - cu.pw) + cu.ue * (cu.pe - pc);
         hx = (-hx) * temx;
-        float hy = cu.vs * (cu.pc - cu.ps) + cu.vn * (cu.pn - cu.pc);
+        float hy = cu.vs * (pc - cu.ps) + cu.vn * (cu.pn - pc);
         hy = (-hy) * temy;
         const float hp = hx + hy;
-        const FlatTerms t = flat_terms(lcoef(k), k, nk, cu.ppterm, pd, cu.pc, nx.pc, cu.th, thm);
-        pd = cu.pc;
+        const FlatTerms t = flat_terms(lcoef(k), k, nk, cu.ppterm, pd, pc, cu.pup, cu.th, thm);
+        pd = pc;
+        pc = cu.pup;
         thm = cu.th;
         const float s1 = t.pk1 + t.qk, s2 = t.pk2 - t.qk;
         const float vert = wraw * s1 + cu.wup * s2;
@@ -1778,6 +1835,13 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
       }
     }
   }
+  // the words phase C adds to, requested here so that they arrive behind the recurrence
+  float rw[CH];
+  if (a.avg && phys && kb <= ke) {
+    const float* ra = n <= a.avg ? a.wa : a.rrw;
+#pragma unroll
+    for (int kk = 0; kk < CH; ++kk) rw[kk] = ldo(ra, (uint32_t)((int64_t)min(kb + kk, ke) * wst + wc) * 4u);
+  }
   __syncthreads();
   // ---------------- a slot's first level: its right-hand side from the previous slot's last level
   if (phys && kb <= ke && kb >= 2) {
@@ -1793,7 +1857,7 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
   // the slots outside wavefront 0 make the next small step's open-side step of
   // the tile's boundary faces (k_snd_ssopen_flat's statements): the column
   // beside a face is the only reader of it in this pass, and has read it
-  if (phys && slot == 0) thomas_column<C2W>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
+  if (phys && slot == 0) thomas_column<C2W, 1>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
   {
     constexpr int S0 = 64 / C2W;
     static_assert(C2S > S0, "the open sides need slots outside wavefront 0");
@@ -1823,11 +1887,6 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
   // ---------------- phase C: pressure update, filter, time averages
   if (phys && kb <= ke) {
     const float wlid = w[(int64_t)(nk + 1) * wst + wc];
-    float rw[CH];
-#pragma unroll
-    for (int kk = 0; kk < CH; ++kk)
-      if (a.avg && kb + kk <= ke)
-        rw[kk] = n <= a.avg ? a.wa[(int64_t)(kb + kk) * wst + wc] * a.beta : a.rrw[(int64_t)(kb + kk) * wst + wc];
 #pragma unroll
     for (int kk = 0; kk < CH; ++kk) {
       const int k = kb + kk;
@@ -1845,7 +1904,8 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
         a.ppd[p] = up + tend;
         if (a.nrk == 3 && last) a.ppx[p] = tend;
         if (a.avg) {
-          const float vw = (a.avg == AVG_PAIR ? rw[kk] + rwo[kk] : rw[kk]) + (last ? wk * a.alph : wk);
+          const float r0 = n <= a.avg ? rw[kk] * a.beta : rw[kk];
+          const float vw = (a.avg == AVG_PAIR ? r0 + rwo[kk] : r0) + (last ? wk * a.alph : wk);
           a.rrw[(int64_t)k * wst + wc] = last ? vw * tavg : vw;
         }
       }
@@ -1875,10 +1935,9 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
 // step), against 23 of the seven-plane pass.  Its 92 registers allow two
 // workgroups a CU; it is bound by the latency of the levels' words and of the
 // recurrence, not by HBM (2.7 TB/s algorithmic).  Measured a small step at
-// 320x320x80: 251 -> 208 us (and 155 -> 123 at 192x256x80).  Slower: held to 80
+// 320x320x80: 251 -> 196 us (and 155 -> 112 at 192x256x80).  Slower: held to 80
 // registers for three workgroups (20 spilled, 272 us), the column's metrics kept
-// in LDS (15 spilled), ten waves a workgroup (one workgroup a CU); words requested
-// two levels ahead measured the same.
+// in LDS (15 spilled), ten waves a workgroup (one workgroup a CU).
 int column4_lds_bytes(int nk, int cw, int slots) {
   return (C3PLANES * (nk + 1) * cw + (nk + 1) * 4 + 2 * slots * cw) * (int)sizeof(float);
 }
@@ -2018,7 +2077,7 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(4))) void k
       const int k = kb + kk;
       if (k <= ke) {
         const In cu = nx;
-        if (k < ke) nx = load(k + 1);
+        nx = load(min(k + 1, ke));  // (unguarded, as the flat pass's)
         const float4 lev = Ltab[k];
         ColumnFaces fhi = flo;
         float rho_hi = 0.0f, dum3_hi = 0.0f, hadvp_hi = 0.0f;
@@ -2075,6 +2134,13 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(4))) void k
       }
     }
   }
+  // the words phase C adds to, requested here so that they arrive behind the recurrence
+  float rw[CH];
+  if (a.avg && phys && kb <= ke) {
+    const float* ra = n <= a.avg ? a.wa : a.rrw;
+#pragma unroll
+    for (int kk = 0; kk < CH; ++kk) rw[kk] = ldo(ra, (uint32_t)((int64_t)min(kb + kk, ke) * wst + wc) * 4u);
+  }
   __syncthreads();
   // ---------------- a slot's first level: its right-hand side from the previous slot's last level
   if (phys && kb <= ke && kb >= 2) {
@@ -2087,15 +2153,10 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(4))) void k
   }
   __syncthreads();
   // ---------------- phase B: Thomas recurrence, one lane per column
-  if (phys && slot == 0) thomas_column<C2W>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
+  if (phys && slot == 0) thomas_column<C2W, 2>(Ls1, Ls2, Lmm, Ldd, c, nk, asq);
   __syncthreads();
   // ---------------- phase C: pressure update, filter, the w average
   if (phys && kb <= ke) {
-    float rw[CH];
-#pragma unroll
-    for (int kk = 0; kk < CH; ++kk)
-      if (a.avg && kb + kk <= ke)
-        rw[kk] = n <= a.avg ? a.wa[(int64_t)(kb + kk) * wst + wc] * a.beta : a.rrw[(int64_t)(kb + kk) * wst + wc];
 #pragma unroll
     for (int kk = 0; kk < CH; ++kk) {
       const int k = kb + kk;
@@ -2114,7 +2175,8 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(4))) void k
         a.ppd[p] = up + tend;
         if (a.nrk == 3 && last) a.ppx[p] = tend;
         if (a.avg) {
-          const float vw = (a.avg == AVG_PAIR ? rw[kk] + rwo[kk] : rw[kk]) + (last ? wk * a.alph : wk);
+          const float r0 = n <= a.avg ? rw[kk] * a.beta : rw[kk];
+          const float vw = (a.avg == AVG_PAIR ? r0 + rwo[kk] : r0) + (last ? wk * a.alph : wk);
           a.rrw[(int64_t)k * wst + wc] = last ? vw * tavg : vw;
         }
       }
@@ -2244,10 +2306,12 @@ static void launch_column3(bool narrow, const SoundArgs& a, int n, hipStream_t s
   const int chunk = (a.nk + slots - 1) / slots;
   if (narrow) {
     if (chunk <= 4) hipLaunchKernelGGL((k_snd_column3<16, 256, 4>), grid, dim3(256), lds, s, a, n);
+    else if (chunk <= 5) hipLaunchKernelGGL((k_snd_column3<16, 256, 5>), grid, dim3(256), lds, s, a, n);
     else if (chunk <= 6) hipLaunchKernelGGL((k_snd_column3<16, 256, 6>), grid, dim3(256), lds, s, a, n);
     else hipLaunchKernelGGL((k_snd_column3<16, 256, 8>), grid, dim3(256), lds, s, a, n);
   } else {
     if (chunk <= 4) hipLaunchKernelGGL((k_snd_column3<32, 512, 4>), grid, dim3(512), lds, s, a, n);
+    else if (chunk <= 5) hipLaunchKernelGGL((k_snd_column3<32, 512, 5>), grid, dim3(512), lds, s, a, n);
     else if (chunk <= 6) hipLaunchKernelGGL((k_snd_column3<32, 512, 6>), grid, dim3(512), lds, s, a, n);
     else hipLaunchKernelGGL((k_snd_column3<32, 512, 8>), grid, dim3(512), lds, s, a, n);
   }
