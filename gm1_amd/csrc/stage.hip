@@ -88,9 +88,11 @@ struct BuoyArgs {
 // interior u and v faces.  Each thread marches one column through a chunk of
 // BUOY_KC levels, carrying dum8 and the w-level buoyancy of its own cell and
 // of its west and south neighbours in registers: b at w level k+1 is formed
-// once and reused as level k's on the next iteration, so a cell's b is formed
-// once per chunk instead of six times.
-constexpr int BUOY_KC = 8;
+// once and reused as level k's on the next iteration.  Every word of the
+// chunk is requested before the first is used, by loads no lane skips (levels
+// clamped to the column, missing neighbours read the cell's own words): 102 -> 92 us at
+// 320x320x80 and 15 -> 4.4 at 64x64x40, against words loaded where they are used.
+constexpr int BUOY_KC = 4;
 
 __global__ __launch_bounds__(64) void k_buoyancy_col(BuoyArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -100,68 +102,74 @@ __global__ __launch_bounds__(64) void k_buoyancy_col(BuoyArgs a) {
   if (i >= ni || k0 > nk) return;
   const int k1 = min(k0 + BUOY_KC - 1, nk);
   const bool fu = i >= 1, fv = j >= 1;
-  const float* __restrict__ c1 = a.c1;
-  const float* __restrict__ c2 = a.c2;
-  const int64_t plane = (int64_t)nj * ni;
-  const int64_t cp = (int64_t)j * ni + i;       // c1/c2 column
-  const int64_t wp = fu ? cp - 1 : cp;          // west neighbour (unused when !fu)
-  const int64_t sp = fv ? cp - ni : cp;         // south neighbour (unused when !fv)
-  const int64_t sst = (int64_t)sy(nj) * sx(ni);
-  const float* __restrict__ dm = a.dum8;
-  const int64_t dc = ix3(0, j + NG, i + NG, sy(nj), sx(ni));
-  const int64_t dw = fu ? dc - 1 : dc;
-  const int64_t ds = fv ? dc - sx(ni) : dc;
-  // w level k0: zero at the surface (k0 == 1), else b(k0) from dum8(k0-1), dum8(k0).
-  float cur_c = dm[dc + k0 * sst], cur_w = dm[dw + k0 * sst], cur_s = dm[ds + k0 * sst];
-  float lo_c = 0.0f, lo_w = 0.0f, lo_s = 0.0f;
-  if (k0 > 1) {
-    const int64_t q = (int64_t)(k0 - 1) * plane;
-    const int64_t m = (int64_t)(k0 - 1) * sst;
-    lo_c = c1[q + cp] * dm[dc + m] + c2[q + cp] * cur_c;
-    lo_w = c1[q + wp] * dm[dw + m] + c2[q + wp] * cur_w;
-    lo_s = c1[q + sp] * dm[ds + m] + c2[q + sp] * cur_s;
+  const int nxs = sx(ni), nxu = ux(ni), nys = sy(nj), nyv = vy(nj);
+  const int64_t plane = (int64_t)nj * ni, sst = (int64_t)nys * nxs, ust = (int64_t)nys * nxu, vst = (int64_t)nyv * nxs;
+  const int64_t gxst = (int64_t)nj * (ni + 1), gyst = (int64_t)(nj + 1) * ni;
+  const uint32_t cp = (uint32_t)(j * ni + i) * 4u;  // c1/c2 column, and the west and south neighbours'
+  const uint32_t wp = fu ? cp - 4u : cp, sp = fv ? cp - (uint32_t)ni * 4u : cp;
+  const uint32_t dc = (uint32_t)((j + NG) * nxs + i + NG) * 4u;
+  const uint32_t dw = fu ? dc - 4u : dc, ds = fv ? dc - (uint32_t)nxs * 4u : dc;
+  const uint32_t du = (uint32_t)((j + NG) * nxu + i + NG) * 4u, gp = (uint32_t)(j * (ni + 1) + i) * 4u;
+  // dum8 at levels k0-1 .. k1+1, c1 and c2 at w levels k0 .. k1+1
+  float dmc[BUOY_KC + 2], dmw[BUOY_KC + 2], dms[BUOY_KC + 2];
+  float ac[BUOY_KC + 1], aw[BUOY_KC + 1], as[BUOY_KC + 1], bc[BUOY_KC + 1], bw[BUOY_KC + 1], bs[BUOY_KC + 1];
+  float gx[BUOY_KC + 1], gy[BUOY_KC + 1], tu[BUOY_KC], tv[BUOY_KC], tw[BUOY_KC];
+#pragma unroll
+  for (int q = 0; q < BUOY_KC + 2; ++q) {
+    const float* dm = a.dum8 + (int64_t)min(k0 - 1 + q, nk) * sst;
+    dmc[q] = ldo(dm, dc);
+    dmw[q] = ldo(dm, dw);
+    dms[q] = ldo(dm, ds);
   }
 #pragma unroll
-  for (int kk = 0; kk < BUOY_KC; ++kk) {
-    const int k = k0 + kk;
+  for (int q = 0; q < BUOY_KC + 1; ++q) {
+    const int64_t m = (int64_t)(min(k0 + q, nk) - 1) * plane;
+    ac[q] = ldo(a.c1 + m, cp);
+    aw[q] = ldo(a.c1 + m, wp);
+    as[q] = ldo(a.c1 + m, sp);
+    bc[q] = ldo(a.c2 + m, cp);
+    bw[q] = ldo(a.c2 + m, wp);
+    bs[q] = ldo(a.c2 + m, sp);
+    const int kg = min(k0 - 1 + q, nk);  // (gxu and gyv hold w levels 1..nk+1)
+    gx[q] = ldo(a.gxu + (int64_t)kg * gxst, gp);
+    gy[q] = ldo(a.gyv + (int64_t)kg * gyst, cp);
+  }
+#pragma unroll
+  for (int q = 0; q < BUOY_KC; ++q) {
+    const int k = min(k0 + q, k1);
+    tu[q] = ldo(a.uten + (int64_t)k * ust, du);
+    tv[q] = ldo(a.vten + (int64_t)k * vst, dc);
+    tw[q] = ldo(a.wten + (int64_t)k * sst, dc);
+  }
+  // b at w level k0 + q (zero at the surface and the lid)
+  auto buoy = [&](int q, const float* c1, const float* c2, const float* dm) {
+    const int kf = k0 + q;
+    return (kf >= 2 && kf <= nk) ? c1[q] * dm[q] + c2[q] * dm[q + 1] : 0.0f;
+  };
+  float lo_c = buoy(0, ac, bc, dmc), lo_w = buoy(0, aw, bw, dmw), lo_s = buoy(0, as, bs, dms);
+#pragma unroll
+  for (int q = 0; q < BUOY_KC; ++q) {
+    const int k = k0 + q;
     if (k > k1) break;
-    float hi_c = 0.0f, hi_w = 0.0f, hi_s = 0.0f, nxt_c = 0.0f, nxt_w = 0.0f, nxt_s = 0.0f;
-    if (k < nk) {  // w level k+1 is interior; level nk+1 (the lid) carries no buoyancy
-      const int64_t q = (int64_t)k * plane;
-      const int64_t m = (int64_t)(k + 1) * sst;
-      nxt_c = dm[dc + m];
-      nxt_w = dm[dw + m];
-      nxt_s = dm[ds + m];
-      hi_c = c1[q + cp] * cur_c + c2[q + cp] * nxt_c;
-      hi_w = c1[q + wp] * cur_w + c2[q + wp] * nxt_w;
-      hi_s = c1[q + sp] * cur_s + c2[q + sp] * nxt_s;
-    }
-    if (k >= 2) {
-      const int64_t d = ix3(k, j + NG, i + NG, sy(nj), sx(ni));
-      a.wten[d] = a.wten[d] + lo_c;
-    }
+    const float hi_c = buoy(q + 1, ac, bc, dmc), hi_w = buoy(q + 1, aw, bw, dmw), hi_s = buoy(q + 1, as, bs, dms);
+    if (k >= 2) sto(a.wten + (int64_t)k * sst, dc, tw[q] + lo_c);
     if (fu) {
       float t = (hi_c + hi_w) + (lo_c + lo_w);
       t = 0.125f * t;
-      t = t - 0.25f * (cur_c + cur_w);
-      t = t * (a.gxu[((int64_t)(k - 1) * nj + j) * (ni + 1) + i] + a.gxu[((int64_t)k * nj + j) * (ni + 1) + i]);
-      const int64_t d = ix3(k, j + NG, i + NG, sy(nj), ux(ni));
-      a.uten[d] = a.uten[d] + t;
+      t = t - 0.25f * (dmc[q + 1] + dmw[q + 1]);
+      t = t * (gx[q] + gx[q + 1]);
+      sto(a.uten + (int64_t)k * ust, du, tu[q] + t);
     }
     if (fv) {
       float t = (hi_c + hi_s) + (lo_c + lo_s);
       t = 0.125f * t;
-      t = t - 0.25f * (cur_c + cur_s);
-      t = t * (a.gyv[((int64_t)(k - 1) * (nj + 1) + j) * ni + i] + a.gyv[((int64_t)k * (nj + 1) + j) * ni + i]);
-      const int64_t d = ix3(k, j + NG, i + NG, vy(nj), sx(ni));
-      a.vten[d] = a.vten[d] + t;
+      t = t - 0.25f * (dmc[q + 1] + dms[q + 1]);
+      t = t * (gy[q] + gy[q + 1]);
+      sto(a.vten + (int64_t)k * vst, dc, tv[q] + t);
     }
     lo_c = hi_c;
     lo_w = hi_w;
     lo_s = hi_s;
-    cur_c = nxt_c;
-    cur_w = nxt_w;
-    cur_s = nxt_s;
   }
 }
 
@@ -293,11 +301,15 @@ __global__ __launch_bounds__(64) void k_getdivx_v(DivArgs a) {
   }
 }
 
-// k_getdivx_v with the column's levels split over GX_SLOTS level slots of one
-// workgroup: every slot first reads the raw averaged w of its levels and of
-// the level below them (which the slot below rewrites), then -- after the
-// barrier -- rewrites its own levels in place.  Columns up to
-// GX_SLOTS * GX_MAXL levels.
+// getdiv and getdivx's vertical pass of one column together, before k_getdivx_h
+// rescales the faces (their rescaled words are formed here by its own statements, so
+// rru and rrv are read once, as averaged).  The column's levels are split over
+// GX_SLOTS level slots of one workgroup: every slot first reads the raw averaged w of
+// its levels and of the level below them (which the slot below rewrites), then -- after
+// the barrier -- rewrites its own levels in place.  Words are requested a level ahead
+// by loads no lane skips.  Columns up to GX_SLOTS * GX_MAXL levels.  Against k_getdiv,
+// then the rescaling, then this pass on the rescaled words: 55 + 77 -> 94 us at
+// 320x320x80.
 constexpr int GX_SLOTS = 8;
 constexpr int GX_MAXL = 16;
 
@@ -307,56 +319,91 @@ bool slotted_columns(int ni, int nj, int nk) {
   return (int64_t)ni * nj < (int64_t)1 << 18 && nk <= GX_SLOTS * GX_MAXL;
 }
 
-__global__ __launch_bounds__(64 * GX_SLOTS) void k_getdivx_v_slots(DivArgs a) {
-  const int c = threadIdx.x % 64, slot = threadIdx.x / 64;
+__global__ __launch_bounds__(64 * GX_SLOTS) void k_post_acoustic(DivArgs a) {
+  const int c = threadIdx.x % 64, slot = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);  // (a wavefront is a slot)
   const int i = blockIdx.x * 64 + c;
   const int j = blockIdx.y;
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const bool live = i < ni;
+  const int ic = live ? i : ni - 1;
   const int L = (nk + GX_SLOTS - 1) / GX_SLOTS;
   const int kf0 = 2 + slot * L, kf1 = min(kf0 + L - 1, nk + 1);  // this slot's w levels (2..nk+1)
   const int nxu = ux(ni), nyu = sy(nj), nxs = sx(ni), nyv = vy(nj);
-  const int x = i + NG, y = j + NG;
-  const int64_t h = (int64_t)j * ni + i;
-  const int64_t wst = (int64_t)nyu * nxs, wc = (int64_t)y * nxs + x;
-  float raw[GX_MAXL + 1];  // raw[q]: averaged w at level kf0 - 1 + q
+  const int64_t ust = (int64_t)nyu * nxu, vst = (int64_t)nyv * nxs, wst = (int64_t)nyu * nxs, mst = (int64_t)nj * ni;
+  const uint32_t oc = (uint32_t)(j * ni + ic) * 4u, ol = (uint32_t)(j * ni + max(ic - 1, 0)) * 4u,
+                 oe = (uint32_t)(j * ni + min(ic + 1, ni - 1)) * 4u, os = (uint32_t)(max(j - 1, 0) * ni + ic) * 4u,
+                 on = (uint32_t)(min(j + 1, nj - 1) * ni + ic) * 4u;
+  const uint32_t ow = (uint32_t)((j + NG) * nxu + ic + NG) * 4u, ov = (uint32_t)((j + NG) * nxs + ic + NG) * 4u;
+  float raw[GX_MAXL + 1];  // raw[q]: averaged w at level kf0 - 1 + q (clamped to 1..nk, where it is not used)
 #pragma unroll
-  for (int q = 0; q <= GX_MAXL; ++q) {
-    const int kf = kf0 - 1 + q;
-    raw[q] = (live && kf <= kf1 && kf >= 2 && kf <= nk) ? a.rrw[(int64_t)kf * wst + wc] : 0.0f;
-  }
+  for (int q = 0; q <= GX_MAXL; ++q)
+    if (q <= L) raw[q] = ldo(a.rrw + (int64_t)min(kf0 - 1 + q, nk) * wst, ov);
   __syncthreads();
   if (!live || kf0 > kf1) return;
   const float dz = a.dz, rds = 1.0f / dz, rdsf = 1.0f / dz, zt = (float)nk * dz, rzt = 1.0f / zt;
-  const float ddx = a.dzdx[h], ddy = a.dzdy[h], g = a.gz[h];
-  auto val_at = [&](int kf, float w) {
-    if (kf <= 1 || kf > nk) return 0.0f;
+  const float ddx = ldo(a.dzdx, oc), ddy = ldo(a.dzdy, oc), g = ldo(a.gz, oc);
+  const float gw = a.rgzu[(int64_t)j * (ni + 1) + i], ge = a.rgzu[(int64_t)j * (ni + 1) + i + 1];
+  const float gs = ldo(a.rgzv, oc), gn = ldo(a.rgzv, oc + (uint32_t)ni * 4u);
+  struct In {
+    float uw, ue, vs, vn, rc, rl, re, rs, rn, rf, th;
+  };
+  auto load = [&](int k) {
+    const float *U = a.rru + (int64_t)k * ust, *V = a.rrv + (int64_t)k * vst, *R = a.rho0 + (int64_t)(k - 1) * mst;
+    return In{ldo(U, ow), ldo(U, ow + 4u), ldo(V, ov), ldo(V, ov + (uint32_t)nxs * 4u), ldo(R, oc), ldo(R, ol),
+              ldo(R, oe), ldo(R, os), ldo(R, on), ldo(a.rf0 + (int64_t)(k - 1) * mst, oc),
+              ldo(a.thterm + (int64_t)(k - 1) * mst, oc)};
+  };
+  struct Faces {
+    float w, e, s, n;
+  };
+  auto averaged = [&](const In& x) { return Faces{x.uw * gw, x.ue * ge, x.vs * gs, x.vn * gn}; };
+  auto rescaled = [&](const In& x) {  // k_getdivx_h's words
+    return Faces{((0.5f * (x.rl + x.rc)) * x.uw) * gw, ((0.5f * (x.rc + x.re)) * x.ue) * ge,
+                 ((0.5f * (x.rs + x.rc)) * x.vs) * gs, ((0.5f * (x.rc + x.rn)) * x.vn) * gn};
+  };
+  // the terrain term of w level kf between the faces of levels kf and kf - 1
+  auto terrain = [&](int kf, const Faces& hi, const Faces& lo) {
     const float sf = (float)(kf - 1) * dz, sm = ((float)(kf - 1) - 0.5f) * dz;
     float r2 = (sf - sm) * rds;
     const float r1 = 0.5f * (1.0f - r2);
     r2 = 0.5f * r2;
-    const float uxv = r2 * (a.rru[ix3(kf, y, x, nyu, nxu)] + a.rru[ix3(kf, y, x + 1, nyu, nxu)]) +
-                      r1 * (a.rru[ix3(kf - 1, y, x, nyu, nxu)] + a.rru[ix3(kf - 1, y, x + 1, nyu, nxu)]);
-    const float vyv = r2 * (a.rrv[ix3(kf, y, x, nyv, nxs)] + a.rrv[ix3(kf, y + 1, x, nyv, nxs)]) +
-                      r1 * (a.rrv[ix3(kf - 1, y, x, nyv, nxs)] + a.rrv[ix3(kf - 1, y + 1, x, nyv, nxs)]);
-    float t = uxv * ddx + vyv * ddy;
-    t = ((t * (sf - zt)) * g) * rzt;
-    return a.rf0[(int64_t)(kf - 1) * nj * ni + h] * w + t;
+    const float uxv = r2 * (hi.w + hi.e) + r1 * (lo.w + lo.e);
+    const float vyv = r2 * (hi.s + hi.n) + r1 * (lo.s + lo.n);
+    const float t = uxv * ddx + vyv * ddy;
+    return ((t * (sf - zt)) * g) * rzt;
   };
-  if (kf0 == 2) a.rrw[wst + wc] = 0.0f;
-  float below = val_at(kf0 - 1, raw[0]);
+  const bool bottom = kf0 == 2;
+  const In x0 = load(max(kf0 - 2, 1)), x1 = load(kf0 - 1);
+  In nx = load(min(kf0, nk));
+  Faces alo = averaged(x1), rlo = rescaled(x1);
+  float th = x1.th;
+  float wlo = bottom ? 0.0f : raw[0] + terrain(kf0 - 1, alo, averaged(x0));
+  float below = bottom ? 0.0f : x1.rf * raw[0] + terrain(kf0 - 1, rlo, rescaled(x0));
+  if (bottom) sto(a.rrw + wst, ov, 0.0f);
 #pragma unroll
   for (int q = 1; q <= GX_MAXL; ++q) {
     const int kf = kf0 - 1 + q;
     if (kf > kf1) break;
-    const float val = val_at(kf, raw[q]);
-    a.rrw[(int64_t)kf * wst + wc] = val;
-    const int k = kf - 1;
-    float d = (a.rru[ix3(k, y, x + 1, nyu, nxu)] - a.rru[ix3(k, y, x, nyu, nxu)]) * a.rdx +
-              (a.rrv[ix3(k, y + 1, x, nyv, nxs)] - a.rrv[ix3(k, y, x, nyv, nxs)]) * a.rdy;
-    d = d + (val - below) * rdsf;
-    a.divx[(int64_t)(k - 1) * nj * ni + h] = (fabsf(d) < 1.0e-20f) ? 0.0f : d;
+    const In cu = nx;  // level kf (the top level again above it, where both w words are 0)
+    nx = load(min(kf + 1, nk));
+    const Faces ahi = averaged(cu), rhi = rescaled(cu);
+    const float whi = (kf <= nk) ? raw[q] + terrain(kf, ahi, alo) : 0.0f;
+    const float val = (kf <= nk) ? cu.rf * raw[q] + terrain(kf, rhi, rlo) : 0.0f;
+    sto(a.rrw + (int64_t)kf * wst, ov, val);
+    const int64_t z = (int64_t)(kf - 2) * mst;  // the cell below
+    float d = (alo.e - alo.w) * a.rdx + (alo.n - alo.s) * a.rdy;
+    d = d + (whi - wlo) * rdsf;
+    if (fabsf(d) < 1.0e-20f) d = 0.0f;
+    sto(a.div + z, oc, d);
+    sto(a.theta_div + z, oc, d * th);
+    float dx = (rlo.e - rlo.w) * a.rdx + (rlo.n - rlo.s) * a.rdy;
+    dx = dx + (val - below) * rdsf;
+    sto(a.divx + z, oc, (fabsf(dx) < 1.0e-20f) ? 0.0f : dx);
+    wlo = whi;
     below = val;
+    alo = ahi;
+    rlo = rhi;
+    th = cu.th;
   }
 }
 
@@ -658,12 +705,15 @@ int gm1hip_post_acoustic(float* rru, float* rrv, float* rrw, const float* rho0_3
   hipStream_t s = (hipStream_t)stream;
   DivArgs a{rru, rrv, rrw, rho0_3d, rf0, rgzu, rgzv, dzdx, dzdy, gz, thterm, divergence, theta_div, divx,
             ni, nj, nk, 1.0f / dx, 1.0f / dy, dz};
-  hipLaunchKernelGGL(k_getdiv, dim3((ni + 63) / 64, nj, (nk + KB - 1) / KB), dim3(64), 0, s, a);
-  hipLaunchKernelGGL(k_getdivx_h, dim3((ni + 1 + 63) / 64, nj + 1, (nk + KB - 1) / KB), dim3(64), 0, s, a);
-  if (slotted_columns(ni, nj, nk))
-    hipLaunchKernelGGL(k_getdivx_v_slots, dim3((ni + 63) / 64, nj), dim3(64 * GX_SLOTS), 0, s, a);
-  else
+  const dim3 faces((ni + 1 + 63) / 64, nj + 1, (nk + KB - 1) / KB);
+  if (slotted_columns(ni, nj, nk)) {
+    hipLaunchKernelGGL(k_post_acoustic, dim3((ni + 63) / 64, nj), dim3(64 * GX_SLOTS), 0, s, a);
+    hipLaunchKernelGGL(k_getdivx_h, faces, dim3(64), 0, s, a);
+  } else {
+    hipLaunchKernelGGL(k_getdiv, dim3((ni + 63) / 64, nj, (nk + KB - 1) / KB), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(k_getdivx_h, faces, dim3(64), 0, s, a);
     hipLaunchKernelGGL(k_getdivx_v, dim3((ni + 63) / 64, nj), dim3(64), 0, s, a);
+  }
   GM1_LAUNCH_CHECK();
   return 0;
 }
