@@ -511,7 +511,7 @@ __device__ __forceinline__ void scalar_adv5_body_lanes(const ScalarAdvArgs& a) {
 // ahead and a level has one barrier.  Measured against guarded loads, the z face's words
 // loaded where they are used and three barriers a level: at 640x768x80 (flat) the WENO
 // compose 927 -> 675 us and the pdef tendencies 727 -> 605, at 320x320x80 (terrain)
-// 254 -> 154 and 182 -> 140.  Six waves per SIMD (three 512-lane workgroups a CU), except the
+// 254 -> 154 and 182 -> 140 (617, 515, 134 and 121 with weno5's short form).  Six waves per SIMD (three 512-lane workgroups a CU), except the
 // terrain WENO forms, which spill at six: four waves, 154 against 165 us at 320x320x80
 // (the flat form 720 against 675 at 640x768x80).
 constexpr int adv5_waves(bool weno, int mode, bool flat) { return weno && mode != MODE_PDEF && !flat ? 4 : 6; }

@@ -26,3 +26,53 @@ def test_gpu_scalar_tiles(device, nrk, sides, dims):
 def test_gpu_momentum_tiles(device, sides, dims):
     print("momentum tiles", dims, sides, flush=True)
     momentum_tests.test_gpu_momentum_advection_bit_exact(device, sides, dims)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("weps", [1.0e-17, 1.0e-20, 1.0e-30])
+@pytest.mark.parametrize("field", ["steps", "decades", "signed zeros", "huge"])
+def test_gpu_weno_words_over_the_whole_range(device, field, weps):
+    """The short evaluation and the statement it stands for: smooth and broken stencils, words over twenty
+    decades, exact cancellation, zeros of either sign, smoothness above and weps below the short form's range."""
+    import numpy as np
+    import torch
+
+    from gm1_amd.advection5 import launch_cuda_scalar_advection5
+    from helpers import F, assert_bits_equal, shapes, to_dev, to_host
+    from oracle import advection5 as oa
+
+    print("weno words", field, weps, flush=True)
+    ni, nj, nk = 70, 21, 16
+    rng = np.random.default_rng(len(field))
+    a, m, _ = scalar_tests._random_case(rng, ni, nj, nk)
+    sh = shapes(ni, nj, nk)
+    for k in ("rru", "rrv", "rrw"):
+        a[k] = rng.standard_normal(a[k].shape).astype(F)
+    x = rng.standard_normal(sh["s"])
+    if field == "steps":
+        s = 300.0 + np.round(2.0 * x) + 1e-6 * x
+    elif field == "decades":
+        s = x * 10.0 ** rng.uniform(-18.0, 4.0, x.shape)
+    elif field == "signed zeros":
+        s = np.where(rng.random(x.shape) < 0.8, np.copysign(0.0, x), 1e-3 * x)
+    else:
+        s = x * 10.0 ** rng.uniform(2.0, 12.0, x.shape)
+    s = s.astype(F)
+    divx = (rng.standard_normal((nk, nj, ni)) * 1e-3).astype(F)
+    want = np.zeros((nk, nj, ni), F)
+    fl = {"x": np.zeros(sh["u"], F), "y": np.zeros(sh["v"], F), "z": np.zeros(sh["w"], F)}
+    dfl = to_dev(fl, device)
+    kw = dict(ni=ni, nj=nj, nk=nk, nrk=3, dx=250.0, dy=200.0, dz=150.0, weps=weps, lateral_sides=(1, 1, 1, 1))
+    oa.cpu_scalar_advection5_inplace(s, a, m, divx, want, fl, **kw)
+    got = torch.zeros((nk, nj, ni), dtype=torch.float32, device=device)
+    launch_cuda_scalar_advection5(to_dev(s, device), to_dev(a, device), to_dev(m, device), to_dev(divx, device), got,
+                                  dfl, **kw)
+    torch.cuda.synchronize()
+    # the top and bottom faces' limiter takes max(0, x) of zeros of either sign, whose sign IEEE 754 leaves open:
+    # with signed zeros the words compared are those of the faces that WENO alone forms
+    zeros = field == "signed zeros"
+    faces = {"x": slice(None), "y": slice(None), "z": slice(4, nk - 1) if zeros else slice(None)}
+    for d in "xyz":
+        assert_bits_equal(to_host(dfl[d])[faces[d]], fl[d][faces[d]], f"flux {d}")
+    if not zeros:
+        assert_bits_equal(to_host(got), want, "tendency")
