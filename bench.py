@@ -42,24 +42,42 @@ WORD = 4
 # (each input read once, each output written once; halos, staggering and
 # 1-D/2-D metric columns are not counted).  Keyed by (kernel, flat column).
 KERNEL_WORDS = {
-    # reads u, v, w, wten, pp3d, ppten, ppterm, piadv, qk, pk1, pk2, mm, rr0,
-    # rrf0, rru, rrv, rrw; writes w, pp3d, ppd, rru, rrv, rrw
-    ("k_snd_column", False): 23,
+    # the resident column pass: reads u, v, w, wten, pp3d, ppten, ppterm, piadv, pk1, pk2, mm, rr0, rrf0;
+    # writes w, pp3d, ppd; rrw read and written every second small step
+    ("k_snd_column", False): 17,
     # flat column (1-D base state; qk, pk1, pk2, mm formed in registers from
     # ppterm, piadv, thv and per-level factors): reads u, v, w, wten, pp3d,
-    # ppten, ppterm, piadv, thv, rru, rrv, rrw; writes w, pp3d, ppd, rru, rrv, rrw
-    ("k_snd_column", True): 18,
-    # reads u, v, uten, vten, ppd, thv, gxu, gyv; writes u, v
-    ("k_snd_pgrad", False): 10,
-    # reads u, v, uten, vten, ppd, thv; writes u, v
-    ("k_snd_pgrad", True): 8,
+    # ppten, ppterm, piadv, thv; writes w, pp3d, ppd; rrw every second small step
+    ("k_snd_column", True): 13,
+    # reads u, v, uten, vten, ppd, thv, gxu, gyv; writes u, v; with the resident
+    # column pass rru, rrv read and written every second small step
+    ("k_snd_pgrad", False): 12,
+    # reads u, v, uten, vten, ppd, thv; writes u, v; rru, rrv every second small step
+    ("k_snd_pgrad", True): 10,
     # reads scalar, rru, rrv, rrw, divx, rr0; writes tendency
     ("k_scalar_adv5", False): 7,
     ("k_scalar_adv5", True): 7,
 }
 KERNELS = sorted({k for k, _ in KERNEL_WORDS})
+# the other column passes read and write rru, rrv and rrw every small step (and read qk on the
+# terrain family), in place of the pressure gradient
+AVERAGING_COLUMN_EXTRA_WORDS = {False: 6, True: 5}
+AVERAGING_PGRAD_WORDS = -2
 # the fused column passes also read uten, vten, ppd and write u, v (no pressure-gradient launch)
 FUSED_COLUMN_EXTRA_WORDS = 5
+
+
+def kernel_words(kernel: str, flat: bool, column_pass: str, nk: int) -> int:
+    """Words per cell of one launch of `kernel` beside the named column pass."""
+    words = KERNEL_WORDS[(kernel, flat)]
+    resident = nk <= 128 and column_pass.startswith("resident" if flat else "pipelined")
+    if kernel == "k_snd_column" and not resident:
+        words += AVERAGING_COLUMN_EXTRA_WORDS[flat]
+        if column_pass.startswith("fused"):
+            words += FUSED_COLUMN_EXTRA_WORDS
+    elif kernel == "k_snd_pgrad" and not resident:
+        words += AVERAGING_PGRAD_WORDS
+    return words
 
 
 def step_words(numq: int, small_steps: int) -> int:
@@ -523,9 +541,7 @@ def main(argv=None) -> int:
     ms_per_step = elapsed_ms / args.steps
     value = cfg.cells * args.steps / (elapsed_ms * 1e-3)
     avg_launch_s = kernel_ms * 1e-3 / max(launches, 1)
-    words = KERNEL_WORDS[(args.kernel, flat)]
-    if args.kernel == "k_snd_column" and st.column_pass.startswith("fused"):
-        words += FUSED_COLUMN_EXTRA_WORDS
+    words = kernel_words(args.kernel, flat, st.column_pass, cfg.nk)
     algo_bytes = words * WORD * cfg.cells
     achieved = algo_bytes / avg_launch_s / 1e9
     step_w = step_words(st.numq, small_steps)
