@@ -127,9 +127,11 @@ GM1_DEV float flx5(float s1, float s2, float s3, float s4, float s5) {
 // tau (5 u a weight, 8 u the sums, a quotient), the short form within 25 u P (7 u a
 // weight, 9 u each sum, the reciprocal of two Newton steps and a product), together
 // under 2^-47 P; where v - 2^-45 P and v + 2^-45 P round to one binary32 word it is the
-// statement's.  Elsewhere (about one lane in 2^20, NaN, zeros of either sign),
-// and where min(1e30, .) could act (tau > 1e9, weps < 1e-21; below them no product
-// leaves the binary64 range either), the statement itself.  WENO compose
+// statement's.  Elsewhere (about one lane in 2^20, zeros of either sign) and outside
+// b_i <= 1e9, 1e-21 <= weps <= 1e30, the statement itself: there a smoothness may be
+// NaN or infinite (the statement's min() drops it, so its word can be finite), min(1e30, .)
+// could act, or a product could leave the binary64 range (inside, every a_i lies in
+// 1e-21 .. 1.1e30, a weight over the common denominator in 1e-127 .. 1e181).  WENO compose
 // 677 -> 617 us and pdef tendencies 600 -> 515 at 640x768x80, 154 -> 134 and 141 -> 121
 // at 320x320x80 (terrain).
 GM1_DEV float weno5(float s1, float s2, float s3, float s4, float s5,
@@ -162,7 +164,10 @@ GM1_DEV float weno5(float s1, float s2, float s3, float s4, float s5,
     const double v = num * r;
     const double e = 0x1p-45 * (double)fmaxf(fmaxf(fabsf(p1), fabsf(p2)), fabsf(p3));
     const float lo = (float)(v - e), hi = (float)(v + e);
-    if (__float_as_uint(lo) == __float_as_uint(hi) && fmaxf(b1r, b3r) <= 1.0e9f && weps >= 1.0e-21) return lo;
+    // (as integers, which order the smoothnesses as floats do, with infinity and NaN above all)
+    const uint32_t above = (weps >= 1.0e-21 && weps <= 1.0e30) ? 0x4e6e6b29u /* the float after 1e9 */ : 0u;
+    const uint32_t smooth = max(max(__float_as_uint(b1r), __float_as_uint(b2r)), __float_as_uint(b3r));
+    if (__float_as_uint(lo) == __float_as_uint(hi) && smooth < above) return lo;
   }
   double tau = fabs(b1 - b3);
   double q1 = fmin(1.0e30, tau / a1);
