@@ -2395,14 +2395,15 @@ static int psolver3_stage(
     return (int)hipErrorInvalidValue;
   // flags & 128: the flat pass with its own levels' pressure words in registers
   // (16 level slots of at most 8 levels: nk <= 128)
-  // (the terrain column's pipelined request runs its resident pass where the column fits it)
-  const bool resident = flat ? (flags & 128) != 0
-                             : pipe && nk <= 128 && column4_lds_bytes(nk, cw, 16) <= lds_max &&
-                                   span < ((int64_t)1 << 32);
-  if ((flags & 128) && !flat) return (int)hipErrorInvalidValue;
-  if (resident && flat && (fuse || nk > 128 || column3_lds_bytes(nk, cw, 16) > lds_max ||
-                   span >= ((int64_t)1 << 32)))
+  if ((flags & 128) && (!flat || fuse || nk > 128 || column3_lds_bytes(nk, cw, 16) > lds_max ||
+                        span >= ((int64_t)1 << 32)))
     return (int)hipErrorInvalidValue;
+  // (the terrain column's pipelined request runs its resident pass where the column fits it.  The resident passes
+  // start rrw from wa in the second small step, when w3d holds the first one's: where w3d is wa itself, the pass
+  // that starts rrw before the first step runs in their place)
+  const bool resident = wa != w3d && (flat ? (flags & 128) != 0
+                                           : pipe && nk <= 128 && column4_lds_bytes(nk, cw, 16) <= lds_max &&
+                                                 span < ((int64_t)1 << 32));
   a.fresh_averages = resident ? 1 : 0;
   a.avg_on = resident ? 1 : 0;
   // (the fills after small steps 1..nloop-1 rewrite ppd's whole halo ring when every side is a family)

@@ -55,6 +55,41 @@ def test_gpu_flat_resident_stage_equals_the_staged_one(device, monkeypatch, nloo
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nloop", [1, 2, 3])
+def test_gpu_flat_resident_stage_with_w_held_in_place(device, monkeypatch, nloop):
+    """A caller whose w3d is its wa: rrw starts from the words before the first small step on every pass."""
+    from dataclasses import replace
+
+    import torch
+
+    from gm1_amd import stretched
+    from gm1_amd.fields import large_stretched_c3
+    from gm1_amd.large_step import create_gm1_large_step_state, host_initial_state, launch_cuda_gm1_large_step
+
+    cfg = replace(large_stretched_c3(33, 9, 18), stretched=(1800.0, 0.0, 1800.0, 60.0, 140.0))
+    print(f"w in place, nloop {nloop}", flush=True)
+    st = create_gm1_large_step_state(host_initial_state(cfg), device)
+    launch_cuda_gm1_large_step(st)
+    torch.cuda.synchronize()
+    schedule = stretched.sound3_stage_schedule_f32
+    monkeypatch.setattr(stretched, "sound3_stage_schedule_f32", lambda dt, ns, nrk: (nloop, schedule(dt, ns, nrk)[1]))
+    runs = {}
+    for column_pass in ("staged", "resident"):
+        for nrk in (1, 3):
+            a = {k: v.clone() for k, v in st.a.items()}
+            a["wa"] = a["w3d"]
+            stretched.launch_cuda_gm1_flat_acoustic_stage(a, st.metrics, ni=33, nj=9, nk=18, nrk=nrk, dt=cfg.dt,
+                                                          nsound=cfg.nsound, dx=cfg.dx, dy=cfg.dy, vertical=st.flat,
+                                                          lateral_sides=cfg.lateral_sides, column_pass=column_pass)
+            torch.cuda.synchronize()
+            runs[column_pass, nrk] = {n: to_host(a[n]) for n in OUT}
+    for nrk in (1, 3):
+        for n in OUT:
+            assert_bits_equal(runs["resident", nrk][n], runs["staged", nrk][n], f"stage {nrk} {n}")
+    assert np.abs(runs["staged", 1]["rrw"]).max() > 0.0
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nloop", [1, 2, 3, 6])
 @pytest.mark.parametrize("sides,ni,nj,nk,slopes", [((2, 2, 2, 2), 33, 9, 18, True), ((1, 1, 2, 2), 32, 11, 49, False),
                                                    ((2, 4, 1, 1), 31, 8, 65, True), ((4, 2, 2, 4), 64, 9, 81, False),
