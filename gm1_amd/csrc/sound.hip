@@ -1867,18 +1867,27 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
       for (int k = 1 + slot - S0; k <= nk; k += C2S - S0) {
         if (ow || oe) {
           const int64_t pu = (int64_t)k * ust + uc, rx = (int64_t)k * (nj + 2 * NG) + j + NG;
-          const float uw = a.u3d[pu], ue = a.u3d[pu + 1], d = ue - uw;
-          if (ow) a.u3d[pu] = uw + a.dts * (((((-a.radbcw[rx]) * d) * a.rdx) * a.uh[NG]) + a.uten[pu]);
+          float uw = a.u3d[pu];
+          const float ue = a.u3d[pu + 1];
+          if (ow) {  // (its new word is the east face's neighbour on a grid one cell wide)
+            uw = uw + a.dts * (((((-a.radbcw[rx]) * (ue - uw)) * a.rdx) * a.uh[NG]) + a.uten[pu]);
+            a.u3d[pu] = uw;
+          }
           if (oe)
-            a.u3d[pu + 1] = ue + a.dts * (((((-a.radbce[rx]) * d) * a.rdx) * a.uh[ni + NG - 1]) + a.uten[pu + 1]);
+            a.u3d[pu + 1] =
+                ue + a.dts * (((((-a.radbce[rx]) * (ue - uw)) * a.rdx) * a.uh[ni + NG - 1]) + a.uten[pu + 1]);
         }
         if (os || on) {
           const int64_t pv = (int64_t)k * vst + vc, ry = (int64_t)k * (ni + 2 * NG) + i + NG;
-          const float vs = a.v3d[pv], vn = a.v3d[pv + nxs], d = vn - vs;
-          if (os) a.v3d[pv] = vs + a.dts * (((((-a.radbcs[ry]) * d) * a.rdy) * a.vh[NG]) + a.vten[pv]);
+          float vs = a.v3d[pv];
+          const float vn = a.v3d[pv + nxs];
+          if (os) {
+            vs = vs + a.dts * (((((-a.radbcs[ry]) * (vn - vs)) * a.rdy) * a.vh[NG]) + a.vten[pv]);
+            a.v3d[pv] = vs;
+          }
           if (on)
             a.v3d[pv + nxs] =
-                vn + a.dts * (((((-a.radbcn[ry]) * d) * a.rdy) * a.vh[nj + NG - 1]) + a.vten[pv + nxs]);
+                vn + a.dts * (((((-a.radbcn[ry]) * (vn - vs)) * a.rdy) * a.vh[nj + NG - 1]) + a.vten[pv + nxs]);
         }
       }
     }

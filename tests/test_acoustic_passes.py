@@ -90,6 +90,36 @@ def test_gpu_flat_resident_stage_with_w_held_in_place(device, monkeypatch, nloop
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("sides,ni,nj", [((2, 2, 1, 1), 1, 9), ((1, 1, 2, 2), 9, 1), ((2, 2, 2, 2), 2, 2)])
+def test_gpu_flat_resident_stage_on_a_grid_one_cell_wide(device, monkeypatch, sides, ni, nj):
+    """Both faces of a cell open: the second face steps beside the first one's new word, as in the staged stage."""
+    import torch
+    from helpers import to_dev
+    from test_sound import _acoustic_case
+    from test_stretched import uniform_flat
+
+    from gm1_amd import stretched
+
+    nk = 18
+    print(f"resident stage {ni}x{nj}x{nk} sides {sides}", flush=True)
+    a0, m0 = _acoustic_case(np.random.default_rng(ni + 2 * nj), ni, nj, nk, terrain=False)
+    m = to_dev(m0, device)
+    column = stretched.flat_stretched_column(uniform_flat(nk, 100.0), device)
+    monkeypatch.setattr(stretched, "sound3_stage_schedule_f32", lambda dt, ns, nrk: (3, float(np.float32(dt / ns))))
+    runs = {}
+    for column_pass in ("staged", "resident"):
+        a = to_dev(a0, device)
+        stretched.launch_cuda_gm1_flat_acoustic_stage(a, m, ni=ni, nj=nj, nk=nk, nrk=1, dt=0.5, nsound=8, dx=250.0,
+                                                      dy=200.0, vertical=column, lateral_sides=sides,
+                                                      column_pass=column_pass)
+        torch.cuda.synchronize()
+        runs[column_pass] = {n: to_host(a[n]) for n in OUT}
+    for n in OUT:
+        assert_bits_equal(runs["resident"][n], runs["staged"][n], n)
+    assert np.isfinite(runs["staged"]["u3d"]).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("nloop", [1, 2, 3, 6])
 @pytest.mark.parametrize("sides,ni,nj,nk,slopes", [((2, 2, 2, 2), 33, 9, 18, True), ((1, 1, 2, 2), 32, 11, 49, False),
                                                    ((2, 4, 1, 1), 31, 8, 65, True), ((4, 2, 2, 4), 64, 9, 81, False),
