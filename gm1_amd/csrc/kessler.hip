@@ -172,11 +172,8 @@ struct KesArgs {
 // ------------------------------------------------------------------ column phase
 // Column loops load KB levels at a time (independent loads in flight) and
 // then run the level arithmetic in k order, so every binary64 sum and every
-// carried value is the sequential one.  (KB = 4 runs two waves a SIMD, 8 one:
-// 141 against 192 us at 320x320x80 and 680 against 766 at 640x768x80, but 56
-// against 51 at 97x61x50; 2 takes 167, 746 and 68.)
-constexpr int KB = 4;
-
+// carried value is the sequential one.
+template <int KB>
 __global__ __launch_bounds__(64) void k_kes_column(KesArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const int j = blockIdx.y;
@@ -365,6 +362,14 @@ __global__ __launch_bounds__(64) void k_kes_column(KesArgs a) {
   }
   a.colbud[3 * plane + h] = bud;
 }
+
+// Levels a batch.  Up to one wave a SIMD (1024 of them) eight levels hide more latency
+// in a wave of their own; beyond, four levels run two waves a SIMD (189 registers) where
+// eight run one (256).  Eight and four measured 50 and 56 us at 97x61x50 (122 waves), 65
+// and 74 at 128x192x64 (384), 66 and 75 at 203x149x57 (596), 98 and 116 at 256x256x80
+// (1024); 178 and 126 at 256x300x80 (1200), 193 and 143 at 320x320x80 (1600), 303 and
+// 283 at 400x400x80 (2800), 785 and 681 at 640x768x80 (7680).
+int column_batch(int64_t waves) { return waves <= 1024 ? 8 : 4; }
 
 // ------------------------------------------------------------------ cell phase
 GM1_DEV double wave_sum(double v) {
@@ -964,7 +969,9 @@ int kessler_driver(const float* ruh, const float* rvh, const float* rmh, const f
   double* rows = (double*)base;
   base += (5LL * nj + 5LL * nk) * 8;
   a.wavestat = (int*)base;
-  hipLaunchKernelGGL(k_kes_column, dim3((ni + 63) / 64, nj), dim3(64), 0, s, a);
+  const dim3 columns((ni + 63) / 64, nj);
+  if (column_batch((int64_t)columns.x * columns.y) == 8) hipLaunchKernelGGL(k_kes_column<8>, columns, dim3(64), 0, s, a);
+  else hipLaunchKernelGGL(k_kes_column<4>, columns, dim3(64), 0, s, a);
   hipLaunchKernelGGL(k_kes_cell, dim3(a.nseg, nj, nk), dim3(64), 0, s, a);
   int* statscr = a.wavestat + 2LL * nk * nj * a.nseg;
   const int row_blocks = (5 * nj + ROW_WAVES - 1) / ROW_WAVES;

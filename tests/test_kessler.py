@@ -331,3 +331,24 @@ def test_gpu_branch_decisions_on_c2_like_fields(device):
     dn, _ = _decisions(k, "numpy", dz=cfg.dz, dt=cfg.dt, eqt=2)
     np.testing.assert_array_equal(got & BRANCH_MASK, dn & BRANCH_MASK)
     assert (((got >> ITER_SHIFT) & 0xFF) != ((dn >> ITER_SHIFT) & 0xFF)).mean() < 5e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ni,nj,nk", [(70, 512, 8), (70, 512, 13), (70, 513, 9), (70, 513, 14), (9, 8, 17)])
+def test_gpu_column_pass_of_either_batch(device, ni, nj, nk):
+    """1024 waves of columns (eight levels a batch) and 1026 (four), with whole and ragged batches, word for word."""
+    import torch
+
+    from gm1_amd.kessler import Gm1KesslerDriverSelection, launch_cuda_gm1_kessler_driver
+
+    print(f"kessler columns {ni}x{nj}x{nk}", flush=True)
+    _, a = c2_like_kessler_fields(ni, nj, nk, seed=nk)
+    da = _device_arrays(a, device)
+    launch_cuda_gm1_kessler_driver(da, ni=ni, nj=nj, nk=nk, dx=250.0, dy=250.0, dz=250.0, dt=6.0,
+                                   selection=Gm1KesslerDriverSelection(equation_set=2))
+    torch.cuda.synchronize()
+    with ok.transcendentals("rounded"):
+        ok.kessler_driver(a, dx=250.0, dy=250.0, dz=250.0, dt=6.0, equation_set=2)
+    for name in FIELDS:
+        assert_bits_equal(da[name].cpu().numpy(), a[name], name)
+    np.testing.assert_allclose(da["qbudget"].cpu().numpy(), a["qbudget"], rtol=1e-12, atol=1e-30)
