@@ -10,6 +10,7 @@ carriers instead of ``cupy.ndarray``.  The work runs in
 
 from __future__ import annotations
 
+import ctypes
 import math
 from collections.abc import Mapping, MutableMapping
 from dataclasses import dataclass
@@ -27,6 +28,7 @@ CM1_NRKMAX = 3
 CM1_WENO_SIFORM = 2
 SCALAR_TILE_LOCAL_OBC = 0
 
+signature("gm1hip_tile_chunk_levels", I, I, I, restype=ctypes.c_int64)
 signature("gm1hip_terrain_mass_flux5", P, P, P, P, P, P, P, P, P, P, P, P, P, P, I, I, I, Fl, Fl, Fl, P)
 signature("gm1hip_scalar_advection5", P, P, P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, D, Fl, Fl, Fl, U, P)
 

@@ -1093,6 +1093,12 @@ int launch_scalar_tile(ScalarAdvArgs& a, int use_weno, int mode, hipStream_t s) 
 
 extern "C" {
 
+int64_t gm1hip_tile_chunk_levels(int tiles, int nk, int per_cu) {
+  int kchunk = 0;
+  if (tiles >= 1 && nk >= 1 && per_cu >= 1) tile_chunks(tiles, nk, per_cu, &kchunk);
+  return kchunk;
+}
+
 int gm1hip_terrain_mass_flux5(const float* u3d, const float* v3d, const float* w3d,
                               float* rru, float* rrv, float* rrw, const float* rho0_3d,
                               const float* rf0, const float* rgzu, const float* rgzv,

@@ -36,6 +36,11 @@ int gm1hip_terrain_mass_flux5(const float* u3d, const float* v3d, const float* w
                               const float* rgzv, const float* dzdx, const float* dzdy, const float* gz, float* divx,
                               int ni, int nj, int nk, float dx, float dy, float dz, void* stream);
 
+// Levels a workgroup marches in one chunk when a marching tile kernel (scalar advection, momentum, the batched
+// compose, the pdef repair) runs `tiles` 64x8 tiles over nk levels with per_cu workgroups on a CU.  A query:
+// nothing is launched.
+int64_t gm1hip_tile_chunk_levels(int tiles, int nk, int per_cu);
+
 // Replaces launch_cuda_scalar_advection5 (cuda_advection5.py:948-1049):
 // 5th-order (use_weno=0) or WENO5 (use_weno=1) face fluxes and the scalar
 // tendency in one LDS-tiled pass.  flux_x/y/z may be NULL (fluxes then stay
