@@ -47,3 +47,31 @@ def test_gpu_staged_columns_forward_words_and_adjoint(device, ni, nj, nk):
             assert np.linalg.norm(g - want[n]) <= 1e-3 * np.linalg.norm(want[n])
         else:
             assert _rel(g, want[n]) <= 1e-4, n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ni,nj,nk", [(33, 6, 6), (32, 7, 16), (8, 9, 33), (9, 8, 64), (35, 6, 65), (6, 6, 128), (9, 7, 130)])
+def test_gpu_staged_columns_adjoint_at_every_cell(device, ni, nj, nk):
+    """With the WENO weights held at their forward values nothing amplifies a rounding, and every field, theta' too
+    (where the column's coefficient adjoints of thv and ppterm end), meets the stage test's 1e-4 at each cell: a
+    level taken wrong where two slots meet would not."""
+    import torch
+
+    from gm1_amd.adjoint_step import DryPeriodicStep
+
+    print(f"adjoint columns, weights held {ni}x{nj}x{nk}", flush=True)
+    cfg, host, a, prof, c = state32(seed=nk, ni=ni, nj=nj, nk=nk)
+    S32 = unpad_np(a, ni, nj, nk)
+    step = DryPeriodicStep(cfg, host["metrics"], host["base"], device, weno="frozen")
+    dev = lambda x: torch.from_numpy(np.ascontiguousarray(x, dtype=np.float32)).to(device)  # noqa: E731
+    _, als, p = _oracle64_trajectory(a, host, cfg, prof, c)
+    end, T = als.Step(p).forward({n: v.astype(np.float64) for n, v in S32.items()}, als.Tape(exact=False))
+    rng = np.random.default_rng(nk)
+    Sb = {n: rng.standard_normal(end[n].shape) for n in FIELDS}
+    want = als.Step(p).adjoint(T, Sb)
+    got = step.adjoint({n: dev(v) for n, v in S32.items()}, {n: dev(v) for n, v in Sb.items()})
+    torch.cuda.synchronize()
+    errs = {n: _rel(got[n].cpu().numpy(), want[n]) for n in FIELDS}
+    print({n: f"{e:.1e}" for n, e in errs.items()}, flush=True)
+    for n, e in errs.items():
+        assert e <= 1e-4, (n, e)
