@@ -52,10 +52,11 @@ GM1_DEV int xcd_tile(int linear, int n) {
 // least (of counts within a hundredth, the largest).  A chunk takes a level more than
 // it has (its window and first plane), full rounds of resident workgroups take a
 // chunk's time each, and a last round takes 0.5 + 0.5 f of it where its fullest CU
-// holds a fraction f of per_cu (fewer waves on a CU each run faster).  The rule follows
-// the measured minima: 200 tiles of 80 levels at two per CU, 5 chunks 154 us, 10 160,
-// 16 173, 4 179; 200 of 80 at three, 5 140, 10 142, 3 152, 4 167; 48 of 64 at three,
-// 16 36 us, 10 40, 5 44; 960 of 80 at three, 4 604 us, 5 612, 10 640, 2 625.
+// holds a fraction f of per_cu (fewer waves on a CU each run faster).  The rule lands
+// within 2 % of the measured minima (its own count first): 200 tiles of 80 levels at two
+// per CU, 5 chunks 154 us, 10 160, 16 173, 4 179; 200 of 80 at three, 10 142, 5 140,
+// 3 152, 4 167; 48 of 64 at three, 16 36 us, 10 40, 5 44; 960 of 80 at three, 4 604 us,
+// 5 612, 10 640, 2 625.
 inline int tile_chunks(int tiles, int nk, int per_cu, int* kchunk) {
   auto cost = [&](int kc) {
     const int64_t groups = (int64_t)tiles * ((nk + kc - 1) / kc), slots = 256 * per_cu;

@@ -322,8 +322,8 @@ GM1_DEV float point_flux(float m, float q0, float q1, float q2, float q3, float 
 // requested a level ahead, and a level has one barrier.  Measured against guarded
 // loads, the z fluxes' words loaded where they are used and three barriers a level:
 // u 442 -> 333, v 401 -> 340, w 420 -> 410 us at 640x768x80 (flat), 124 -> 78, 120 -> 78
-// and 111 -> 77 at 320x320x80 (terrain).  Six waves per SIMD (three workgroups a CU), where only the u
-// tile spills a few registers; on the terrain family, whose u tile needs more, four
+// and 111 -> 77 at 320x320x80 (terrain).  Six waves per SIMD (three workgroups a CU), where the flat u
+// and w tiles spill four and two registers; on the terrain family, whose u tile needs more, four
 // waves are faster (82 -> 78 us at 320x320x80; flat, 364 against 333 at 640x768x80).
 constexpr int advu_waves(bool flat) { return flat ? 6 : 4; }
 template <bool FLAT>

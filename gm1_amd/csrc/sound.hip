@@ -2,17 +2,28 @@
 //
 // Replaces the kernel family of cuda_psolver3_terrain_open.py (prepare,
 // pgrad, two column passes, average) plus its open-boundary, radiation and
-// fill companions.  Per small step this build issues:
-//   [ssopen]  open-side normal velocity step (one thread per edge column)
+// fill companions.  A small step of the resident passes (the default of both
+// families up to 128 levels, k_snd_column3 flat and k_snd_column4 terrain) is:
+//   [ssopen]  open-side normal velocity step: every small step on the terrain
+//             family, the first one only on the flat column (whose column pass
+//             makes the next one's)
 //   pgrad     u/v forward step on every face the family advances, including
-//             periodic boundary faces (one launch instead of two)
-//   column    ONE pass per column: divergence, fpk, bcwsfc, pressure
-//             advection, the Thomas solve for w (upward elimination,
-//             downward substitution fused with the pressure update) and the
-//             rru/rrv/rrw time averages.  The reference needs two column
-//             passes, a bcwsfc launch and an average launch for this.
-//   [fill]    one-cell ppd halo between small steps
-// The column thread walks k with every access i-fastest across the wavefront.
+//             periodic boundary faces (one launch instead of two), reading
+//             ppd's halo words from the cells the fill would copy; at every
+//             second small step also the rru/rrv time averages, two steps'
+//             words at once
+//   column    ONE pass per column: divergence, fpk, bcwsfc (terrain), pressure
+//             advection, the Thomas solve for w and the pressure update, the
+//             columns' levels spread over the threads of a workgroup; at every
+//             second small step the rrw average; on the flat column the next
+//             small step's open faces
+// and the one-cell ppd halo is filled once, after the last small step but one
+// (where every side is a lateral family; ppd's ring holds older words until
+// then).  The other column passes (staged, pipelined, fused, register) fill it
+// between all small steps and form all three averages in every column pass;
+// the fused one makes the pressure gradient's step too.  The reference needs
+// two column passes, a bcwsfc launch and an average launch for a small step's
+// column work.
 #include "boundary.h"
 #include "timing.h"
 
@@ -1941,10 +1952,10 @@ __global__ __launch_bounds__(C2T) __attribute__((amdgpu_waves_per_eu(6))) void k
 // the prepare pass's own statement) and the u and v averages are the pressure
 // gradient's: 17 words a cell and step (u, v, w, wten, pp3d, ppten, ppterm,
 // piadv, rr0, rrf0, pk1, pk2, mm read; w, pp3d, ppd written; rrw at every second
-// step), against 23 of the seven-plane pass.  Its 92 registers allow two
-// workgroups a CU; it is bound by the latency of the levels' words and of the
-// recurrence, not by HBM (2.7 TB/s algorithmic).  Measured a small step at
-// 320x320x80: 251 -> 196 us (and 155 -> 112 at 192x256x80).  Slower: held to 80
+// step), against 23 of the seven-plane pass.  Its 87 to 104 registers (96 at five
+// levels a slot) allow two workgroups a CU; it is bound by the latency of the levels' words and of the
+// recurrence, not by HBM (3.1 TB/s algorithmic).  Measured a small step at
+// 320x320x80: 251 -> 182 us (and 155 -> 110 at 192x256x80).  Slower: held to 80
 // registers for three workgroups (20 spilled, 272 us), the column's metrics kept
 // in LDS (15 spilled), ten waves a workgroup (one workgroup a CU).
 int column4_lds_bytes(int nk, int cw, int slots) {
@@ -2380,7 +2391,8 @@ static int psolver3_stage(
   const bool narrow = (flags & 8) != 0;
   // flags & 16: the staged pass with its loads issued a level (phase A) or a
   // batch of levels (phase C) ahead, wten staged through LDS with the other
-  // phase-A words, and the u/v time averages run beside the recurrence
+  // phase-A words, and the u/v time averages run beside the recurrence; on the
+  // terrain family up to 128 levels the resident pass instead (below)
   const int cw = narrow ? 16 : 32;
   const int lds_max = lds_limit() - (int)(cw * sizeof(float));  // less the static w(1) row
   // (a column too tall for the seventh plane runs the six-plane staged pass)
